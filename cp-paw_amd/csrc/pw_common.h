@@ -63,6 +63,25 @@ __host__ __device__ inline T2 cconj(T2 a) { a.y = -a.y; return a; }
 template <typename T2, typename S>
 __host__ __device__ inline T2 cscale(T2 a, S s) { a.x *= s; a.y *= s; return a; }
 
+// Destination of the column products: psi[b][G] = (src or psi)[b][G] + C,
+// then times num / m(G) when mpsi is set (OPSI: the copy of PSI0, ADDPRO and
+// the mass scaling of WAVES_OPSI in one pass, the same operations in order)
+struct ColOut {
+  double2 *psi;
+  const double2 *src;
+  const double *mpsi;
+  double num;
+  __device__ void store(size_t i, int ig, double cr, double ci) const {
+    const double2 s = src ? src[i] : psi[i];
+    double2 v = make_double2(s.x + cr, s.y + ci);
+    if (mpsi) {
+      const double f = num / mpsi[ig];
+      v = make_double2(f * v.x, f * v.y);
+    }
+    psi[i] = v;
+  }
+};
+
 // ---------------------------------------------------------------------------
 // 1-D FFT factorisation
 // ---------------------------------------------------------------------------
@@ -108,6 +127,10 @@ struct pw_plan {
   std::vector<int> z2iz;       // nr3, -1 if empty
   std::vector<int> zlist;      // nzp: z of each used plane
   int nmax[3] = {0, 0, 0};     // max |IGVEC(k)|
+  // one G of each pair (G, -G), in the order of the sphere: (G, -G) indices;
+  // G = 0 is its own partner
+  std::vector<int2> hg;
+  int nh = 0;
   Fft1D f[3];
   Fft1D fyz[2];                // y and z factors of the in-place yz pass (no radix 16)
   // device copies
@@ -117,6 +140,7 @@ struct pw_plan {
   int *d_yz2stripe = nullptr, *d_z2iz = nullptr, *d_zlist = nullptr;
   int *d_stripe_pos = nullptr, *d_zpos = nullptr, *d_ypen = nullptr;
   double *d_g2 = nullptr, *d_gvec = nullptr;
+  int2 *d_hg = nullptr;
   double2 *d_tw[3] = {nullptr, nullptr, nullptr};
   float2 *d_twf[3] = {nullptr, nullptr, nullptr};
   hipStream_t stream = 0;
@@ -272,6 +296,15 @@ struct pw_waveset {
   size_t pfac_bytes = 0;
   std::vector<double> pfac_pos;
   bool pfac_valid = false;
+  // FP64 form: the same factors on the half list, F [NSP*LMNXX][NHP] doubles,
+  // then E [NAT][NHP] double2, for the positions hfac_pos; used while the PRO
+  // table has PRO(G) = PRO(-G) (pro_sym), which makes P(-G) = conj(P(G))
+  void *d_hfac = nullptr;
+  size_t hfac_bytes = 0;
+  std::vector<double> hfac_pos;
+  bool hfac_valid = false;
+  bool pro_sym = true;
+  int4 *d_ipro4 = nullptr;     // per projector: F row, atom, l, 0
   double2 *d_phase = nullptr;  // nat*3*(2*nmaxx+1)
   int nphase = 0;              // 2*nmaxx+1
   std::vector<double> phase_pos;   // positions of the tables in d_phase
@@ -363,6 +396,16 @@ int k_denmat(pw_waveset *ws, const double2 *proj, double *dst);
 int k_dot_vrho(pw_waveset *ws, double *dst);
 int ws_part(pw_waveset *ws, size_t bytes);
 int ws_small(pw_waveset *ws, size_t bytes);
+
+// FP64 products on the half list of G pairs (pw_gamma.hip)
+inline int half_pad(const pw_plan *p) { return (p->nh + 31) / 32 * 32; }
+int half_factors_room(pw_waveset *ws);
+int half_factors(pw_waveset *ws);
+int half_projections(pw_waveset *ws, const double2 *psi, double2 *proj);
+int half_overlap(pw_waveset *ws, const double2 *psi1, const double2 *psi2, const double4 *p1c, int nz, double *mat);
+int half_addpro(pw_waveset *ws, const ColOut &out, const double2 *x);
+int half_addopsi(pw_waveset *ws, double2 *psibar, const double2 *chi, const double *lam);
+int half_force(pw_waveset *ws, const double2 *psi, const double2 *ded, double *dst);
 
 // orthogonalisation (pw_ortho.hip)
 void ortho_graph_release(pw_waveset *ws);

@@ -5,79 +5,11 @@
 //   P(atom,lmn,G) = YLM(G,lm) PRO(G,ln) (-i)^l exp(-iG.R)
 // (WAVES_EXPANDPRO, src/paw_waves1.f90:6070-6109) from per-axis phase tables,
 // so the NPRO x NGL projector matrix costs no HBM traffic.
-#include "pw_common.h"
+#include "pw_device.h"
 
 namespace {
 
 constexpr int kB = 256;
-
-struct ProjGeo {
-  int ngl, nbh, nat, lmnxx, nphase, nmaxx;
-  const int *igvec;        // 3*ngl
-  const double *pro;       // [nbarepro][ngl]
-  const double *ylm;       // [lmx][ngl]
-  const double2 *phase;    // [nat][3][nphase]
-  const int *atom_isp, *ipro0, *ibpro, *lmnx;
-  const int *lmn_ln, *lmn_lm, *lmn_l;   // [nsp][lmnxx]
-};
-
-__device__ inline double2 czero() { return make_double2(0.0, 0.0); }
-
-// XCD-aware tile order.  Workgroups are dealt to the eight XCDs in turn
-// (linear id mod 8), and each XCD has its own L2.  The tiles that read the
-// same operand block (one G range) get linear ids of one residue mod 8 that
-// follow each other in that XCD's order, so the block is fetched from HBM once
-// instead of once per tile.  Grid: xcd_blocks(ninner, nshared) in x.
-constexpr int kXcd = 8;
-struct XcdTile {
-  int inner, shared;
-  bool valid;
-};
-__device__ inline XcdTile xcd_tile(int ninner, int nshared) {
-  const int L = blockIdx.x, x = L % kXcd, slot = L / kXcd;
-  XcdTile t;
-  t.inner = slot % ninner;
-  t.shared = (slot / ninner) * kXcd + x;
-  t.valid = t.shared < nshared;
-  return t;
-}
-inline unsigned xcd_blocks(int ninner, int nshared) {
-  return (unsigned)((nshared + kXcd - 1) / kXcd) * kXcd * ninner;
-}
-
-__device__ inline double2 eigr_of(const ProjGeo &q, int atom, int ig) {
-  const int *iv = q.igvec + 3 * ig;
-  const double2 *ph = q.phase + (size_t)atom * 3 * q.nphase;
-  double2 e = cmul(ph[iv[0] + q.nmaxx], ph[q.nphase + iv[1] + q.nmaxx]);
-  return cmul(e, ph[2 * q.nphase + iv[2] + q.nmaxx]);
-}
-
-// sum of v over the 16 lanes of a DPP row (lanes 16k .. 16k+15), in every lane
-// of the row: four rotate-and-add steps on the cross-lane (DPP) path of the
-// VALU (row_ror 8, 4, 2, 1), no LDS traffic
-template <int CTRL>
-__device__ inline double dpp_ror(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
-__device__ inline double row16_sum(double v) {
-  v += dpp_ror<0x128>(v);
-  v += dpp_ror<0x124>(v);
-  v += dpp_ror<0x122>(v);
-  v += dpp_ror<0x121>(v);
-  return v;
-}
-
-// z * (-i)^l
-__device__ inline double2 rot_mil(double2 z, int l) {
-  switch (l & 3) {
-    case 0: return z;
-    case 1: return make_double2(z.y, -z.x);
-    case 2: return make_double2(-z.x, -z.y);
-    default: return make_double2(-z.y, z.x);
-  }
-}
 
 // P(atom, lmn, G) given eigr; returns zero for an empty slot
 __device__ inline double2 pro_val(const ProjGeo &q, int atom, int lmn, int ig, double2 eigr) {
@@ -116,15 +48,9 @@ __global__ void k_phase(int nat, int nphase, int nmaxx, PhaseArgs a, double2 *ph
 // padded to 16 (mod 32) doubles so that the 16 x 4 operand reads of a wave
 // are free of bank conflicts.
 // ---------------------------------------------------------------------------
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-
 constexpr int KC = 16;   // K depth staged in LDS per step (four MFMA K slices)
 
 constexpr int padw(int w) { return w + ((16 - w % 32) + 32) % 32; }
-
-__device__ inline dbl4 mfma4(double a, double b, dbl4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
 
 // (cr + i ci) += (ar + i ai)(br + i bi)
 __device__ inline void cmfma(dbl4 &cr, dbl4 &ci, double ar, double ai, double br, double bi) {
@@ -141,19 +67,6 @@ struct GenProj {
   __device__ double2 operator()(int r, int ig) const {
     const int2 al = iptab[r];
     return cconj(pro_val(q, al.x, al.y, ig, eigr_of(q, al.x, ig)));
-  }
-};
-
-// stacked rows [conj(psi1_i(G)) ; psi1_i(-G)] for the band overlaps; rows
-// [0,nbhp) give T, rows [nbhp, 2 nbhp) give TM (nbhp = nbh rounded up to 16)
-struct GenOvl {
-  const double2 *psi1;
-  const int *minusg;
-  int ngl, nbh, nbhp;
-  __device__ double2 operator()(int r, int ig) const {
-    if (r < nbhp) return r < nbh ? cconj(psi1[(size_t)r * ngl + ig]) : czero();
-    r -= nbhp;
-    return r < nbh ? psi1[(size_t)r * ngl + minusg[ig]] : czero();
   }
 };
 
@@ -214,51 +127,6 @@ __global__ void __launch_bounds__(64 * NW) k_rowgemm(Gen gen, int nrow, int ngl,
   }
 }
 
-// sum of split partials: out[i] = scale * sum_s part[s][i] in a fixed order.
-// A block takes 32 outputs; its 8 lanes per output stride over the splits
-// with four accumulators each and are combined through LDS.
-constexpr int kRedC = 32, kRedS = 8;
-
-__device__ inline double rz(double) { return 0.0; }
-__device__ inline double2 rz(double2) { return make_double2(0.0, 0.0); }
-__device__ inline double radd(double a, double b) { return a + b; }
-__device__ inline double2 radd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
-__device__ inline double rscale(double a, double s) { return a * s; }
-__device__ inline double2 rscale(double2 a, double s) { return make_double2(a.x * s, a.y * s); }
-
-// out[i] = scale * sum_k part[k][i]: kRedS lanes per column take the splits
-// k = sl, sl + kRedS, ...; each lane issues its loads 16 at a time and adds
-// them in k order, then the lanes are added in order (deterministic)
-template <typename T>
-__global__ void __launch_bounds__(kRedC * kRedS) k_reduce_split(const T *__restrict__ part, int ns, int n,
-                                                                double scale, T *__restrict__ out) {
-  __shared__ T red[kRedS][kRedC];
-  const int c = threadIdx.x % kRedC, sl = threadIdx.x / kRedC;
-  const int i = blockIdx.x * kRedC + c;
-  T acc = rz(T());
-  if (i < n) {
-    constexpr int V = 16;
-    for (int k0 = sl; k0 < ns; k0 += V * kRedS) {
-      T v[V];
-#pragma unroll
-      for (int u = 0; u < V; ++u) {
-        const int k = k0 + u * kRedS;
-        v[u] = k < ns ? part[(size_t)k * n + i] : rz(T());
-      }
-#pragma unroll
-      for (int u = 0; u < V; ++u) acc = radd(acc, v[u]);
-    }
-  }
-  red[sl][c] = acc;
-  __syncthreads();
-  if (sl != 0 || i >= n) return;
-  T r = red[0][c];
-#pragma unroll
-  for (int q = 1; q < kRedS; ++q) r = radd(r, red[q][c]);
-  out[i] = rscale(r, scale);
-}
-
-
 // ---------------------------------------------------------------------------
 // psi[b][G] += sum_k A(b,k) B(k,G): the band-major output is C^T, so a lane's
 // MFMA results are 16 consecutive G of one band (coalesced read-modify-write).
@@ -277,25 +145,6 @@ struct AddproB {
   __device__ double2 operator()(int k, int ig) const {
     const int2 al = iptab[k];
     return pro_val(q, al.x, al.y, ig, eigr_of(q, al.x, ig));
-  }
-};
-
-// Destination of the column products: psi[b][G] = (src or psi)[b][G] + C,
-// then times num / m(G) when mpsi is set (OPSI: the copy of PSI0, ADDPRO and
-// the mass scaling of WAVES_OPSI in one pass, the same operations in order)
-struct ColOut {
-  double2 *psi;
-  const double2 *src;
-  const double *mpsi;
-  double num;
-  __device__ void store(size_t i, int ig, double cr, double ci) const {
-    const double2 s = src ? src[i] : psi[i];
-    double2 v = make_double2(s.x + cr, s.y + ci);
-    if (mpsi) {
-      const double f = num / mpsi[ig];
-      v = make_double2(f * v.x, f * v.y);
-    }
-    psi[i] = v;
   }
 };
 
@@ -585,26 +434,6 @@ __device__ inline void fold_lambda(const double *lam, int nb, int i, int j, doub
   l1 = make_double2(0.5 * (a11 + a22), 0.5 * (a12 - a21));
   l2 = make_double2(0.5 * (a11 - a22), 0.5 * (a12 + a21));
 }
-
-// ADDOPSI: psibar[j][G] += sum_i L1[i][j] chi[i][G] + L2[i][j] conj(chi[i][-G])
-// as one column GEMM over the stacked K = 2 NBH
-struct AddopsiA {
-  const double *lam;
-  int nb, nbh;
-  __device__ double2 operator()(int k, int j) const {
-    double2 l1, l2;
-    fold_lambda(lam, nb, k < nbh ? k : k - nbh, j, l1, l2);
-    return k < nbh ? l1 : l2;
-  }
-};
-struct AddopsiB {
-  const double2 *chi;
-  const int *minusg;
-  int ngl, nbh;
-  __device__ double2 operator()(int k, int ig) const {
-    return k < nbh ? chi[(size_t)k * ngl + ig] : cconj(chi[(size_t)(k - nbh) * ngl + minusg[ig]]);
-  }
-};
 
 // ---------------------------------------------------------------------------
 // Split-BF16x3 MFMA building blocks (mixed form).  A value x is carried as
@@ -1669,17 +1498,6 @@ __global__ void k_propagate_g(int ngl, int nbh, double a1, double a2, double a3n
   psim[idx] = make_double2(a1 * p0.x + a2 * pm.x + a3 * h.x, a1 * p0.y + a2 * pm.y + a3 * h.y);
 }
 
-ProjGeo make_pgeo(pw_waveset *ws) {
-  ProjGeo q;
-  pw_plan *p = ws->plan;
-  q.ngl = p->ngl; q.nbh = ws->nbh; q.nat = ws->nat; q.lmnxx = ws->lmnxx;
-  q.nphase = ws->nphase; q.nmaxx = (ws->nphase - 1) / 2;
-  q.igvec = p->d_igvec; q.pro = ws->d_pro; q.ylm = ws->d_ylm; q.phase = ws->d_phase;
-  q.atom_isp = ws->d_atom_isp; q.ipro0 = ws->d_ipro0; q.ibpro = ws->d_ibpro; q.lmnx = ws->d_lmnx;
-  q.lmn_ln = ws->d_lmn_ln; q.lmn_lm = ws->d_lmn_lm; q.lmn_l = ws->d_lmn_l;
-  return q;
-}
-
 // blocks of 16 bands per workgroup (at most 8) and the number of band tiles
 void band_tiles(int nbh, int *nblk, int *ntiles) {
   const int total = (nbh + 15) / 16;
@@ -1782,7 +1600,7 @@ struct RowPart {
 
 template <int NW, class Gen>
 int run_rowgemm(pw_waveset *ws, const Gen &gen, int nrow, const double2 *psi, double scale,
-                double2 *out, double2 **res, const char *name, RowPart *defer = nullptr) {
+                double2 *out, double2 **res, const char *name) {
   const int ngl = ws->plan->ngl, nbh = ws->nbh;
   int nblk, tb;
   band_tiles(nbh, &nblk, &tb);
@@ -1803,10 +1621,6 @@ int run_rowgemm(pw_waveset *ws, const Gen &gen, int nrow, const double2 *psi, do
     PW_NB_SWITCH(nblk, PW_LAUNCH)
 #undef PW_LAUNCH
     PW_HIP(hipGetLastError());
-  }
-  if (defer) {
-    *defer = RowPart{part, ns, n, scale};
-    return PW_OK;
   }
   {
     ScopeTimer tm(ws, "reduce");
@@ -1989,6 +1803,7 @@ int k_projections(pw_waveset *ws, const double2 *psi, const double2 *phase, doub
     RowPf gen{pfac_of(ws)};
     return run_rowgemm_bf<4>(ws, gen, ws->npro, gb, ws->plan->vol, proj, nullptr, "projections");
   }
+  if (ws->pro_sym) return half_projections(ws, psi, proj);
   ProjGeo q = make_pgeo(ws);
   q.phase = phase;
   GenProj gen{q, ws->d_ipro_tab};
@@ -2008,6 +1823,7 @@ static int addpro_to(pw_waveset *ws, const ColOut &out, const double2 *phase, co
     if (ws->tune_col_waves == 2) return run_colgemm_bf<2>(ws, ga, gb, ws->npro, out, "addpro");
     return run_colgemm_bf<4>(ws, ga, gb, ws->npro, out, "addpro");
   }
+  if (ws->pro_sym) return half_addpro(ws, out, x);
   ProjGeo q = make_pgeo(ws);
   q.phase = phase;
   AddproA ga{x, ws->nbh};
@@ -2056,6 +1872,7 @@ int k_force(pw_waveset *ws, const double2 *psi, const double2 *phase, const doub
     PW_HIP(hipGetLastError());
     return PW_OK;
   }
+  if (ws->pro_sym) return half_force(ws, psi, ded, dst);
   const int ngt = (q.ngl + 16 * NGB - 1) / (16 * NGB);
   PW_TRY(ws_part(ws, (size_t)ngt * n * sizeof(double)));
   {
@@ -2077,8 +1894,9 @@ int k_force(pw_waveset *ws, const double2 *psi, const double2 *phase, const doub
 int k_overlap(pw_waveset *ws, const double2 *psi1, const double2 *psi2, double *mat, bool, bool) {
   pw_plan *p = ws->plan;
   const int nbh = ws->nbh, nbhp = (nbh + 15) / 16 * 16;
+  if (ws->prec == PW_PREC_FP64) return half_overlap(ws, psi1, psi2, nullptr, 0, mat);
   double2 *red = nullptr;
-  if (ws->prec == PW_PREC_MIXED) {
+  {
     const size_t bytes = runs_bytes(nbh, p->ngl);
     PW_TRY(ws_split(ws, 3 * bytes));   // outside a runs scope all three go to the scratch
     OvlRuns gen;
@@ -2089,9 +1907,6 @@ int k_overlap(pw_waveset *ws, const double2 *psi1, const double2 *psi2, double *
     if (psi2 == psi1) gb.s = gen.rows;
     else PW_TRY(wave_runs(ws, psi2, false, 2 * bytes, &gb.s));
     PW_TRY(run_rowgemm_bf<2>(ws, gen, 2 * nbhp, gb, p->vol, nullptr, &red, "overlap"));
-  } else {
-    GenOvl gen{psi1, p->d_minusg, p->ngl, nbh, nbhp};
-    PW_TRY(run_rowgemm<2>(ws, gen, 2 * nbhp, psi2, p->vol, nullptr, &red, "overlap"));
   }
   k_unravel_pw<<<(nbh * nbh + 255) / 256, 256, 0, ws->stream>>>(nbh, ws->nb, red, red + (size_t)nbhp * nbh,
                                                                   mat);
@@ -2118,8 +1933,9 @@ int k_overlap_full(pw_waveset *ws, const double2 *psi1, const double2 *psi2, con
     k_overlap1c<<<grid, 256, 0, ws->stream>>>(ws->npro, nbh, proj1, ws->d_xproj, p1c);
     PW_HIP(hipGetLastError());
   }
+  if (ws->prec == PW_PREC_FP64) return half_overlap(ws, psi1, psi2, p1c, nz, mat);
   RowPart rp;
-  if (ws->prec == PW_PREC_MIXED) {
+  {
     const size_t bytes = runs_bytes(nbh, p->ngl);
     PW_TRY(ws_split(ws, 3 * bytes));   // outside a runs scope all three go to the scratch
     OvlRuns gen;
@@ -2130,9 +1946,6 @@ int k_overlap_full(pw_waveset *ws, const double2 *psi1, const double2 *psi2, con
     if (psi2 == psi1) gb.s = gen.rows;
     else PW_TRY(wave_runs(ws, psi2, false, 2 * bytes, &gb.s));
     PW_TRY(run_rowgemm_bf<2>(ws, gen, 2 * nbhp, gb, p->vol, nullptr, nullptr, "overlap", &rp));
-  } else {
-    GenOvl gen{psi1, p->d_minusg, p->ngl, nbh, nbhp};
-    PW_TRY(run_rowgemm<2>(ws, gen, 2 * nbhp, psi2, p->vol, nullptr, nullptr, "overlap", &rp));
   }
   {
     ScopeTimer tm(ws, "reduce");
@@ -2167,9 +1980,7 @@ int k_addopsi(pw_waveset *ws, double2 *psibar, const double2 *chi, const double 
     if (ws->tune_col_waves == 2) return run_colgemm_bf<2>(ws, ga, gb, nk, ColOut{psibar}, "addopsi");
     return run_colgemm_bf<4>(ws, ga, gb, nk, ColOut{psibar}, "addopsi");
   }
-  AddopsiA ga{lam, ws->nb, ws->nbh};
-  AddopsiB gb{chi, p->d_minusg, p->ngl, ws->nbh};
-  return run_colgemm<2>(ws, ga, gb, 2 * ws->nbh, ColOut{psibar}, "addopsi");
+  return half_addopsi(ws, psibar, chi, lam);
 }
 
 int k_addoproj(pw_waveset *ws, double2 *proj, const double2 *oproj, const double *lam) {

@@ -253,6 +253,9 @@ static int build_plan(pw_plan *p, const double *rbas, double epw_psi, double epw
     p->minusg[n] = it->second;
     if (it->second == n) p->ngamma = n;
   }
+  for (int n = 0; n < ng; ++n)
+    if (p->minusg[n] >= n) p->hg.push_back(make_int2(n, p->minusg[n]));
+  p->nh = (int)p->hg.size();
   // G vectors and |G|^2 (PLANEWAVE_GVECTORS, GETR8A('G2'))
   p->gvec.resize(3 * ng);
   p->g2.resize(ng);
@@ -363,6 +366,7 @@ static int upload_plan(pw_plan *p) {
   PW_TRY(upload(&p->d_z2iz, p->z2iz));
   PW_TRY(upload(&p->d_g2, p->g2));
   PW_TRY(upload(&p->d_gvec, p->gvec));
+  PW_TRY(upload(&p->d_hg, p->hg));
   for (int k = 0; k < 3; ++k) {
     int n = p->f[k].n;
     std::vector<double2> tw(n);
@@ -435,7 +439,7 @@ extern "C" int pw_plan_destroy(pw_plan *p) {
   if (!p) return PW_OK;
   void *ptrs[] = {p->d_minusg, p->d_igvec, p->d_stripe_off, p->d_stripe_g, p->d_stripe_x,
                   p->d_stripe_s, p->d_zlist, p->d_yz2stripe, p->d_z2iz, p->d_g2, p->d_gvec, p->d_stripe_buf,
-                  p->d_plane_buf, p->d_dens_part, p->d_vt, p->d_stripe_pos, p->d_zpos, p->d_ypen, p->d_tw[0], p->d_tw[1], p->d_tw[2], p->d_twf[0],
+                  p->d_plane_buf, p->d_dens_part, p->d_vt, p->d_stripe_pos, p->d_zpos, p->d_ypen, p->d_hg, p->d_tw[0], p->d_tw[1], p->d_tw[2], p->d_twf[0],
                   p->d_twf[1], p->d_twf[2], p->d_pot_tabs, p->d_pot};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);

@@ -242,6 +242,11 @@ static int phase_at(pw_waveset *ws, const std::vector<double> &r) {
     ws->pfac_pos = r;
     ws->pfac_valid = true;
   }
+  if (ws->prec == PW_PREC_FP64 && ws->pro_sym && (!ws->hfac_valid || ws->hfac_pos != r)) {
+    PW_TRY(half_factors(ws));
+    ws->hfac_pos = r;
+    ws->hfac_valid = true;
+  }
   return PW_OK;
 }
 
@@ -452,15 +457,18 @@ extern "C" int pw_waves_create(pw_plan *plan, int nb, int nat, int nsp, const in
   up(&ws->d_lmn_lm, ws->lmn_lm);
   up(&ws->d_lmn_l, ws->lmn_l);
   {
-    std::vector<int> tab;
+    std::vector<int> tab, tab4;
     for (int a = 0; a < nat; ++a)
       for (int l = 0; l < ws->lmnx[ws->isp[a]]; ++l) {
-        tab.push_back(a);
-        tab.push_back(l);
+        const int k = ws->isp[a] * ws->lmnxx + l;
+        tab.insert(tab.end(), {a, l});
+        tab4.insert(tab4.end(), {k, a, ws->lmn_l[k], 0});
       }
     up((int **)&ws->d_ipro_tab, tab);
+    up((int **)&ws->d_ipro4, tab4);
   }
   if (rc == PW_OK) rc = ylm_table(ws);
+  if (rc == PW_OK && prec == PW_PREC_FP64) rc = half_factors_room(ws);
   if (rc != PW_OK) return fail(rc);
   if (hipStreamCreateWithFlags(&ws->stream, hipStreamNonBlocking) != hipSuccess) return fail(pw_fail(PW_ERR_HIP, "hipStreamCreate failed"));
   ws->own_stream = true;
@@ -513,9 +521,11 @@ int ws_reset_run(pw_waveset *ws) {
   f.d_fpm = ws->d_fpm; f.d_fab = ws->d_fab; f.d_domat = ws->d_domat; f.d_dhmat = ws->d_dhmat;
   f.d_atom_isp = ws->d_atom_isp; f.d_ipro0 = ws->d_ipro0; f.d_ibpro = ws->d_ibpro; f.d_lmnx = ws->d_lmnx;
   f.d_lmn_ln = ws->d_lmn_ln; f.d_lmn_lm = ws->d_lmn_lm; f.d_lmn_l = ws->d_lmn_l; f.d_ipro_tab = ws->d_ipro_tab;
+  f.d_ipro4 = ws->d_ipro4;
   f.d_phase = ws->d_phase; f.d_small_mats = ws->d_small_mats;
   f.d_res = ws->d_res; f.h_res = ws->h_res;
   f.d_pfac = ws->d_pfac; f.pfac_bytes = ws->pfac_bytes;
+  f.d_hfac = ws->d_hfac; f.hfac_bytes = ws->hfac_bytes;
   f.d_part = ws->d_part; f.part_bytes = ws->part_bytes;
   f.d_split = ws->d_split; f.split_bytes = ws->split_bytes;
   f.d_wruns = ws->d_wruns; f.wruns_bytes = ws->wruns_bytes;
@@ -541,7 +551,7 @@ extern "C" int pw_waves_destroy(pw_waveset *ws) {
                   ws->d_occ, ws->d_rlam0, ws->d_rlamm,
                   ws->d_fpm, ws->d_fab, ws->d_domat, ws->d_dhmat, ws->d_atom_isp, ws->d_ipro0,
                   ws->d_ibpro, ws->d_lmnx, ws->d_lmn_ln, ws->d_lmn_lm, ws->d_lmn_l, ws->d_phase,
-                  ws->d_part, ws->d_small, ws->d_ortho, ws->d_small_mats, ws->d_ipro_tab, ws->d_pfac,
+                  ws->d_part, ws->d_small, ws->d_ortho, ws->d_small_mats, ws->d_ipro_tab, ws->d_ipro4, ws->d_pfac, ws->d_hfac,
                   ws->d_split, ws->d_wruns};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
@@ -597,6 +607,19 @@ extern "C" int pw_waves_setr8a(pw_waveset *ws, const char *id, int len, const do
     // caller layout PRO(NGL,NBAREPRO) column-major == [ibare][ngl]
     PW_HIP(hipMemcpy(ws->d_pro, val, (size_t)len * sizeof(double), hipMemcpyHostToDevice));
     ws->pfac_valid = false;
+    ws->hfac_valid = false;
+    // radial tables have PRO(G) = PRO(-G) (to the rounding of |G|)
+    ws->pro_sym = true;
+    for (int k = 0; k < ws->nbarepro && ws->pro_sym; ++k) {
+      const double *row = val + (size_t)k * p->ngl;
+      for (const int2 &h : p->hg) {
+        const double a = row[h.x], b = row[h.y];
+        if (!(std::fabs(a - b) <= 1.0e-15 * std::max(std::fabs(a), std::fabs(b)))) {
+          ws->pro_sym = false;
+          break;
+        }
+      }
+    }
   } else if (s == "OCC") {
     PW_TRY(chk(ws->nb));
     ws->occ.assign(val, val + ws->nb);
@@ -1027,6 +1050,7 @@ extern "C" int pw_waves_etot(pw_waveset *ws) {
   // the phase tables and projector factors are redone at least once per step
   ws->phase_valid = false;
   ws->pfac_valid = false;
+  ws->hfac_valid = false;
   ScopeTimer whole(ws, "WAVES$ETOT");
   if (ws->first) {
     PW_TRY(pw_waves_gramschmidt(ws));

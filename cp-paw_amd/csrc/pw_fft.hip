@@ -17,218 +17,13 @@
 // Work buffers: stripes [band][x][stripe], planes [band][iz][y][x].
 #include <type_traits>
 
-#include "pw_common.h"
+#include "pw_dft.h"
+#include "pw_pencil.h"
 
 namespace {
 
 constexpr int kBlock = 256;
 constexpr int kTX = 16;       // x columns per y/z tile
-
-template <typename T2> struct Prec;
-template <> struct Prec<double2> {
-  typedef double T;
-  static __device__ inline double2 from(double2 v) { return v; }
-};
-template <> struct Prec<float2> {
-  typedef float T;
-  static __device__ inline float2 from(double2 v) { return make_float2((float)v.x, (float)v.y); }
-};
-
-template <typename T2>
-__device__ inline T2 czero() { T2 r; r.x = 0; r.y = 0; return r; }
-
-// a * (sign * i)
-template <typename T2>
-__device__ inline T2 mul_si(T2 a, int sign) {
-  T2 r;
-  r.x = sign > 0 ? -a.y : a.y;
-  r.y = sign > 0 ? a.x : -a.x;
-  return r;
-}
-
-// cos/sin(2 pi m / R)
-template <int R> struct Roots;
-template <> struct Roots<3> {
-  static constexpr double c[3] = {1.0, -0.5, -0.5};
-  static constexpr double s[3] = {0.0, 0.86602540378443864676, -0.86602540378443864676};
-};
-template <> struct Roots<5> {
-  static constexpr double c[5] = {1.0, 0.30901699437494742410, -0.80901699437494742410,
-                                  -0.80901699437494742410, 0.30901699437494742410};
-  static constexpr double s[5] = {0.0, 0.95105651629515357212, 0.58778525229247312917,
-                                  -0.58778525229247312917, -0.95105651629515357212};
-};
-template <> struct Roots<7> {
-  static constexpr double c[7] = {1.0, 0.62348980185873353053, -0.22252093395631440429,
-                                  -0.90096886790241912624, -0.90096886790241912624,
-                                  -0.22252093395631440429, 0.62348980185873353053};
-  static constexpr double s[7] = {0.0, 0.78183148246802980871, 0.97492791218182360702,
-                                  0.43388373911755812048, -0.43388373911755812048,
-                                  -0.97492791218182360702, -0.78183148246802980871};
-};
-template <> struct Roots<11> {
-  static constexpr double c[11] = {1.0, 0.84125353283118116886, 0.41541501300188642553,
-                                   -0.14231483827328514044, -0.65486073394528506406,
-                                   -0.95949297361449738989, -0.95949297361449738989,
-                                   -0.65486073394528506406, -0.14231483827328514044,
-                                   0.41541501300188642553, 0.84125353283118116886};
-  static constexpr double s[11] = {0.0, 0.54064081745559758211, 0.90963199535451837141,
-                                   0.98982144188093273238, 0.75574957435425828377,
-                                   0.28173255684142969771, -0.28173255684142969771,
-                                   -0.75574957435425828377, -0.98982144188093273238,
-                                   -0.90963199535451837141, -0.54064081745559758211};
-};
-
-template <> struct Roots<9> {
-  static constexpr double c[9] = {1.0, 0.766044443118978035202, 0.173648177666930348852, -0.5,
-                                  -0.939692620785908384054, -0.939692620785908384054, -0.5,
-                                  0.173648177666930348852, 0.766044443118978035202};
-  static constexpr double s[9] = {0.0, 0.642787609686539326323, 0.984807753012208059367,
-                                  0.866025403784438646764, 0.342020143325668733044,
-                                  -0.342020143325668733044, -0.866025403784438646764,
-                                  -0.984807753012208059367, -0.642787609686539326323};
-};
-template <> struct Roots<16> {
-  static constexpr double c[16] = {1.0, 0.923879532511286756128, 0.707106781186547524401,
-                                   0.382683432365089771728, 0.0, -0.382683432365089771728,
-                                   -0.707106781186547524401, -0.923879532511286756128, -1.0,
-                                   -0.923879532511286756128, -0.707106781186547524401,
-                                   -0.382683432365089771728, 0.0, 0.382683432365089771728,
-                                   0.707106781186547524401, 0.923879532511286756128};
-  static constexpr double s[16] = {0.0, 0.382683432365089771728, 0.707106781186547524401,
-                                   0.923879532511286756128, 1.0, 0.923879532511286756128,
-                                   0.707106781186547524401, 0.382683432365089771728, 0.0,
-                                   -0.382683432365089771728, -0.707106781186547524401,
-                                   -0.923879532511286756128, -1.0, -0.923879532511286756128,
-                                   -0.707106781186547524401, -0.382683432365089771728};
-};
-
-template <typename T2, int R>
-__device__ inline void dft(T2 *v, int sign);
-
-// DFT of size R = P Q from P-point and Q-point DFTs: input r = Q a + b,
-// output q = q1 + P q2; Y_b = DFT_P over a, times exp(sign 2 pi i b q1 / R),
-// then DFT_Q over b.
-template <typename T2, int P, int Q>
-__device__ inline void dft_pq(T2 *v, int sign) {
-  typedef typename Prec<T2>::T T;
-  constexpr int R = P * Q;
-  T2 y[Q][P];
-#pragma unroll
-  for (int b = 0; b < Q; ++b) {
-    T2 t[P];
-#pragma unroll
-    for (int a = 0; a < P; ++a) t[a] = v[Q * a + b];
-    dft<T2, P>(t, sign);
-#pragma unroll
-    for (int q1 = 0; q1 < P; ++q1) y[b][q1] = t[q1];
-  }
-#pragma unroll
-  for (int b = 1; b < Q; ++b)
-#pragma unroll
-    for (int q1 = 1; q1 < P; ++q1) {
-      const int m = (b * q1) % R;
-      T2 w;
-      w.x = (T)Roots<R>::c[m];
-      w.y = sign > 0 ? (T)Roots<R>::s[m] : -(T)Roots<R>::s[m];
-      y[b][q1] = cmul(y[b][q1], w);
-    }
-#pragma unroll
-  for (int q1 = 0; q1 < P; ++q1) {
-    T2 t[Q];
-#pragma unroll
-    for (int b = 0; b < Q; ++b) t[b] = y[b][q1];
-    dft<T2, Q>(t, sign);
-#pragma unroll
-    for (int q2 = 0; q2 < Q; ++q2) v[q1 + P * q2] = t[q2];
-  }
-}
-
-// in-register DFT of size R: v[q] <- sum_r v[r] exp(sign 2 pi i r q / R)
-template <typename T2, int R>
-__device__ inline void dft(T2 *v, int sign) {
-  typedef typename Prec<T2>::T T;
-  if constexpr (R == 2) {
-    T2 a = v[0], b = v[1];
-    v[0] = cadd(a, b); v[1] = csub(a, b);
-  } else if constexpr (R == 3) {
-    // m = v0 - t/2, out(1,2) = m +- sign sin(2 pi/3) i d: 12 operations
-    const T c = (T)-0.5, s = (T)0.86602540378443864676;
-    const T2 t = cadd(v[1], v[2]), d = csub(v[1], v[2]);
-    T2 m;
-    m.x = v[0].x + c * t.x;
-    m.y = v[0].y + c * t.y;
-    v[0] = cadd(v[0], t);
-    const T sx = sign > 0 ? s : -s;
-    T2 o1, o2;
-    o1.x = m.x - sx * d.y;
-    o1.y = m.y + sx * d.x;
-    o2.x = m.x + sx * d.y;
-    o2.y = m.y - sx * d.x;
-    v[1] = o1;
-    v[2] = o2;
-  } else if constexpr (R == 4) {
-    T2 t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]);
-    T2 t2 = cadd(v[1], v[3]), t3 = mul_si(csub(v[1], v[3]), sign);
-    v[0] = cadd(t0, t2); v[2] = csub(t0, t2);
-    v[1] = cadd(t1, t3); v[3] = csub(t1, t3);
-  } else if constexpr (R == 9) {
-    dft_pq<T2, 3, 3>(v, sign);
-  } else if constexpr (R == 16) {
-    dft_pq<T2, 4, 4>(v, sign);
-  } else if constexpr (R == 8) {
-    T2 e[4] = {v[0], v[2], v[4], v[6]};
-    T2 o[4] = {v[1], v[3], v[5], v[7]};
-    dft<T2, 4>(e, sign);
-    dft<T2, 4>(o, sign);
-    const T r2 = (T)0.70710678118654752440;
-    // w^q, w = exp(sign 2 pi i/8)
-    T2 w1; w1.x = r2; w1.y = sign > 0 ? r2 : -r2;
-    T2 w3; w3.x = -r2; w3.y = sign > 0 ? r2 : -r2;
-    T2 o1 = cmul(o[1], w1), o2 = mul_si(o[2], sign), o3 = cmul(o[3], w3);
-    v[0] = cadd(e[0], o[0]); v[4] = csub(e[0], o[0]);
-    v[1] = cadd(e[1], o1);   v[5] = csub(e[1], o1);
-    v[2] = cadd(e[2], o2);   v[6] = csub(e[2], o2);
-    v[3] = cadd(e[3], o3);   v[7] = csub(e[3], o3);
-  } else {
-    constexpr int H = (R - 1) / 2;
-    T2 sp[H], sm[H];
-#pragma unroll
-    for (int r = 1; r <= H; ++r) {
-      sp[r - 1] = cadd(v[r], v[R - r]);
-      sm[r - 1] = mul_si(csub(v[r], v[R - r]), sign);
-    }
-    // out[q], out[R-q] = a_q +- b_q with a_q = v0 + sum_r cos(2 pi r q/R) sp_r
-    // and b_q = sum_r sin(2 pi r q/R) sm_r (cos even, sin odd in q)
-    T2 out[R];
-    out[0] = v[0];
-#pragma unroll
-    for (int r = 0; r < H; ++r) out[0] = cadd(out[0], sp[r]);
-#pragma unroll
-    for (int q = 1; q <= H; ++q) {
-      T2 a = v[0], b;
-#pragma unroll
-      for (int r = 1; r <= H; ++r) {
-        const int m = (r * q) % R;
-        const T c = (T)Roots<R>::c[m];
-        a.x += sp[r - 1].x * c;
-        a.y += sp[r - 1].y * c;
-      }
-      b.x = sm[0].x * (T)Roots<R>::s[q % R];
-      b.y = sm[0].y * (T)Roots<R>::s[q % R];
-#pragma unroll
-      for (int r = 2; r <= H; ++r) {
-        const T s = (T)Roots<R>::s[(r * q) % R];
-        b.x += sm[r - 1].x * s;
-        b.y += sm[r - 1].y * s;
-      }
-      out[q] = cadd(a, b);
-      out[R - q] = csub(a, b);
-    }
-#pragma unroll
-    for (int q = 0; q < R; ++q) v[q] = out[q];
-  }
-}
 
 // One Stockham stage over npen pencils of length n in LDS.
 // Element e of pencil p lives at base[p*ps + e*es].
@@ -291,21 +86,8 @@ __device__ T2 *lds_fft(T2 *b0, T2 *b1, const Fft1D &f, int npen, int es, int ps,
   return in;
 }
 
-// The Stockham chain of a length N fixed at compile time (fft_factor's rule
-// for these passes: odd radices, then 16, 8, 4, 2); STAGE ST of NST with the
+// The Stockham chain of a length N fixed at compile time; stage ST with the
 // span NS = product of the earlier radices.  Returns the result buffer.
-__host__ __device__ constexpr Fft1D fft_stockham_ct(int n) {
-  Fft1D f{};
-  f.n = n;
-  int m = n;
-  const int order[9] = {9, 3, 5, 7, 11, 16, 8, 4, 2};
-  for (int io = 0; io < 9; ++io)
-    while (m % order[io] == 0 && f.nstage < 12) {
-      f.radix[f.nstage++] = order[io];
-      m /= order[io];
-    }
-  return f;
-}
 template <typename T2, int N, int ST, int NS>
 __device__ inline T2 *lds_fft_ct(T2 *in, T2 *out, int npen, int es, int ps, const T2 *tw, int sign, bool pen_fast) {
   constexpr Fft1D f = fft_stockham_ct(N);
@@ -352,8 +134,10 @@ inline dim3 x_grid(int ngroups, int nb) { return dim3((unsigned)(8 * ((nb + 7) /
 // distinct banks
 __host__ __device__ inline int x_pitch(int nr1) { return nr1 | 1; }
 
-// ---- x pass, forward: sphere -> stripes [band][x][stripe] --------------------
-template <typename T2, int NX = 0>
+// ---- x pass, forward: sphere -> stripes --------------------------------------
+// [band][x][stripe] for the yz passes (one x column is a plane's input), ROW:
+// [band][stripe][x] for the pencil passes of the full-grid transforms
+template <typename T2, int NX = 0, bool ROW = false>
 __global__ void __launch_bounds__(kBlock) k_xfwd(Geo g, Fft1D f, const T2 *tw, const double2 *psi,
                                                  T2 *stripes, int nb) {
   constexpr int PX = XTile<T2>::n;
@@ -376,6 +160,11 @@ __global__ void __launch_bounds__(kBlock) k_xfwd(Geo g, Fft1D f, const T2 *tw, c
   T2 *r;
   if constexpr (NX > 0) r = lds_fft_ct<T2, NX, 0, 1>(b0, b1, PX, 1, xp, tw, +1, false);
   else r = lds_fft<T2>(b0, b1, f, PX, 1, xp, tw, +1, false);
+  if constexpr (ROW) {
+    T2 *dst = stripes + ((size_t)band * g.nstripe + s0) * g.nr1;
+    for (int i = threadIdx.x; i < ns * g.nr1; i += blockDim.x) dst[i] = r[i / g.nr1 * xp + i % g.nr1];
+    return;
+  }
   T2 *dst = stripes + (size_t)band * g.nr1 * g.nstripe + s0;
   for (int i = threadIdx.x; i < ns * g.nr1; i += blockDim.x) {
     const int x = i / ns, sl = i % ns;
@@ -384,7 +173,7 @@ __global__ void __launch_bounds__(kBlock) k_xfwd(Geo g, Fft1D f, const T2 *tw, c
 }
 
 // ---- x pass, inverse: stripes -> sphere (gather, scale, optional G^2/2 psi) ---
-template <typename T2, int NX = 0>
+template <typename T2, int NX = 0, bool ROW = false>
 __global__ void __launch_bounds__(kBlock) k_xinv(Geo g, Fft1D f, const T2 *tw, const T2 *stripes,
                                                  double2 *out, const double2 *psi, double scale,
                                                  int add_kin, int nb) {
@@ -398,10 +187,16 @@ __global__ void __launch_bounds__(kBlock) k_xinv(Geo g, Fft1D f, const T2 *tw, c
   T2 *b1 = b0 + PX * xp;
   const int s0 = grp * PX;
   const int ns = min(PX, g.nstripe - s0);
-  const T2 *src = stripes + (size_t)band * g.nr1 * g.nstripe + s0;
-  for (int i = threadIdx.x; i < PX * g.nr1; i += blockDim.x) {
-    const int x = i / PX, sl = i % PX;
-    b0[sl * xp + x] = sl < ns ? src[(size_t)x * g.nstripe + sl] : czero<T2>();
+  if constexpr (ROW) {
+    const T2 *src = stripes + ((size_t)band * g.nstripe + s0) * g.nr1;
+    for (int i = threadIdx.x; i < PX * g.nr1; i += blockDim.x)
+      b0[i / g.nr1 * xp + i % g.nr1] = i < ns * g.nr1 ? src[i] : czero<T2>();
+  } else {
+    const T2 *src = stripes + (size_t)band * g.nr1 * g.nstripe + s0;
+    for (int i = threadIdx.x; i < PX * g.nr1; i += blockDim.x) {
+      const int x = i / PX, sl = i % PX;
+      b0[sl * xp + x] = sl < ns ? src[(size_t)x * g.nstripe + sl] : czero<T2>();
+    }
   }
   __syncthreads();
   T2 *r;
@@ -424,78 +219,20 @@ __global__ void __launch_bounds__(kBlock) k_xinv(Geo g, Fft1D f, const T2 *tw, c
   }
 }
 
-// ---- y pass forward: stripes -> planes -----------------------------------------
-template <typename T2>
-__global__ void __launch_bounds__(kBlock) k_yfwd(Geo g, Fft1D f, const T2 *tw, const T2 *stripes,
-                                                 T2 *planes) {
+// ---- y and z passes of the full-grid transforms, any length --------------------
+// The pass of pw_pencil.h with the length and the stages from the plan, for
+// lengths that have no instantiation there: kTX pencils in LDS.
+template <typename T2, int SIGN>
+__global__ void __launch_bounds__(kBlock) k_pencil_any(PencilArgs a, Fft1D f, const T2 *tw) {
   extern __shared__ unsigned char smem_raw[];
   T2 *b0 = reinterpret_cast<T2 *>(smem_raw);
-  T2 *b1 = b0 + kTX * g.nr2;
-  const int ntx = (g.nr1 + kTX - 1) / kTX;
-  const int iz = blockIdx.x / ntx;
-  const int x0 = (blockIdx.x % ntx) * kTX;
-  const int band = blockIdx.y;
-  const int z = g.zlist[iz];
-  const T2 *src = stripes + (size_t)band * g.nstripe * g.nr1;
-  for (int w = threadIdx.x; w < g.nr2 * kTX; w += blockDim.x) {
-    const int y = w / kTX, x = w % kTX, gx = x0 + x;
-    const int s = g.yz2stripe[y + g.nr2 * z];
-    b0[w] = (s >= 0 && gx < g.nr1) ? src[(size_t)gx * g.nstripe + s] : czero<T2>();
-  }
+  T2 *b1 = b0 + kTX * f.n;
+  const int ntile = (a.npen + kTX - 1) / kTX, grp = blockIdx.x / ntile, q0 = (blockIdx.x % ntile) * kTX;
+  const PencilIo<T2> io(a, grp, blockIdx.y, SIGN > 0);
+  for (int w = threadIdx.x; w < f.n * kTX; w += blockDim.x) b0[w] = io.load(w / kTX, q0 + w % kTX);
   __syncthreads();
-  T2 *r = lds_fft<T2>(b0, b1, f, kTX, kTX, 1, tw, +1, true);
-  T2 *dst = planes + (((size_t)band * g.nzp + iz) * g.nr2) * g.nr1;
-  for (int w = threadIdx.x; w < g.nr2 * kTX; w += blockDim.x) {
-    const int y = w / kTX, x = w % kTX, gx = x0 + x;
-    if (gx < g.nr1) dst[(size_t)y * g.nr1 + gx] = r[w];
-  }
-}
-
-// ---- y pass inverse: planes -> stripes ------------------------------------------
-template <typename T2>
-__global__ void __launch_bounds__(kBlock) k_yinv(Geo g, Fft1D f, const T2 *tw, const T2 *planes,
-                                                 T2 *stripes) {
-  extern __shared__ unsigned char smem_raw[];
-  T2 *b0 = reinterpret_cast<T2 *>(smem_raw);
-  T2 *b1 = b0 + kTX * g.nr2;
-  const int ntx = (g.nr1 + kTX - 1) / kTX;
-  const int iz = blockIdx.x / ntx;
-  const int x0 = (blockIdx.x % ntx) * kTX;
-  const int band = blockIdx.y;
-  const int z = g.zlist[iz];
-  const T2 *src = planes + (((size_t)band * g.nzp + iz) * g.nr2) * g.nr1;
-  for (int w = threadIdx.x; w < g.nr2 * kTX; w += blockDim.x) {
-    const int y = w / kTX, x = w % kTX, gx = x0 + x;
-    b0[w] = gx < g.nr1 ? src[(size_t)y * g.nr1 + gx] : czero<T2>();
-  }
-  __syncthreads();
-  T2 *r = lds_fft<T2>(b0, b1, f, kTX, kTX, 1, tw, -1, true);
-  T2 *dst = stripes + (size_t)band * g.nstripe * g.nr1;
-  for (int w = threadIdx.x; w < g.nr2 * kTX; w += blockDim.x) {
-    const int y = w / kTX, x = w % kTX, gx = x0 + x;
-    const int s = g.yz2stripe[y + g.nr2 * z];
-    if (s >= 0 && gx < g.nr1) dst[(size_t)gx * g.nstripe + s] = r[w];
-  }
-}
-
-// z pencils of one (y, x tile) from the plane buffer (zero on empty planes)
-template <typename T2>
-__device__ inline void load_zpencils(const Geo &g, const T2 *planes_band, int y, int x0, T2 *b0) {
-  for (int w = threadIdx.x; w < g.nr3 * kTX; w += blockDim.x) {
-    const int z = w / kTX, x = w % kTX, gx = x0 + x;
-    const int iz = g.z2iz[z];
-    b0[w] = (iz >= 0 && gx < g.nr1) ? planes_band[((size_t)iz * g.nr2 + y) * g.nr1 + gx]
-                                    : czero<T2>();
-  }
-}
-
-template <typename T2>
-__device__ inline void store_zpencils(const Geo &g, T2 *planes_band, int y, int x0, const T2 *r) {
-  for (int w = threadIdx.x; w < g.nr3 * kTX; w += blockDim.x) {
-    const int z = w / kTX, x = w % kTX, gx = x0 + x;
-    const int iz = g.z2iz[z];
-    if (iz >= 0 && gx < g.nr1) planes_band[((size_t)iz * g.nr2 + y) * g.nr1 + gx] = r[w];
-  }
+  const T2 *r = lds_fft<T2>(b0, b1, f, kTX, kTX, 1, tw, SIGN, true);
+  for (int w = threadIdx.x; w < f.n * kTX; w += blockDim.x) io.store(w / kTX, q0 + w % kTX, r[w]);
 }
 
 // ---- in-place LDS transforms for the resident yz plane -----------------------
@@ -1132,48 +869,6 @@ __global__ void k_transpose_sum(int A, int B, int nsum, const TI *in, TO *out) {
   }
 }
 
-// ---- z pass with full-grid output (PLANEWAVE$FFT 'GTOR') ----------------------------
-template <typename T2>
-__global__ void __launch_bounds__(kBlock) k_zout(Geo g, Fft1D f, const T2 *tw, const T2 *planes,
-                                                 T2 *fofr) {
-  extern __shared__ unsigned char smem_raw[];
-  T2 *b0 = reinterpret_cast<T2 *>(smem_raw);
-  T2 *b1 = b0 + kTX * g.nr3;
-  const int ntx = (g.nr1 + kTX - 1) / kTX;
-  const int y = blockIdx.x / ntx;
-  const int x0 = (blockIdx.x % ntx) * kTX;
-  const int band = blockIdx.y;
-  load_zpencils<T2>(g, planes + (size_t)band * g.nzp * g.nr2 * g.nr1, y, x0, b0);
-  __syncthreads();
-  T2 *r = lds_fft<T2>(b0, b1, f, kTX, kTX, 1, tw, +1, true);
-  T2 *dst = fofr + (size_t)band * g.nr1 * g.nr2 * g.nr3;
-  for (int w = threadIdx.x; w < g.nr3 * kTX; w += blockDim.x) {
-    const int z = w / kTX, x = w % kTX, gx = x0 + x;
-    if (gx < g.nr1) dst[((size_t)z * g.nr2 + y) * g.nr1 + gx] = r[w];
-  }
-}
-
-// ---- z pass with full-grid input (PLANEWAVE$FFT 'RTOG') -----------------------------
-template <typename T2>
-__global__ void __launch_bounds__(kBlock) k_zin(Geo g, Fft1D f, const T2 *tw, const T2 *fofr,
-                                                T2 *planes) {
-  extern __shared__ unsigned char smem_raw[];
-  T2 *b0 = reinterpret_cast<T2 *>(smem_raw);
-  T2 *b1 = b0 + kTX * g.nr3;
-  const int ntx = (g.nr1 + kTX - 1) / kTX;
-  const int y = blockIdx.x / ntx;
-  const int x0 = (blockIdx.x % ntx) * kTX;
-  const int band = blockIdx.y;
-  const T2 *src = fofr + (size_t)band * g.nr1 * g.nr2 * g.nr3;
-  for (int w = threadIdx.x; w < g.nr3 * kTX; w += blockDim.x) {
-    const int z = w / kTX, x = w % kTX, gx = x0 + x;
-    b0[w] = gx < g.nr1 ? src[((size_t)z * g.nr2 + y) * g.nr1 + gx] : czero<T2>();
-  }
-  __syncthreads();
-  T2 *r = lds_fft<T2>(b0, b1, f, kTX, kTX, 1, tw, -1, true);
-  store_zpencils<T2>(g, planes + (size_t)band * g.nzp * g.nr2 * g.nr1, y, x0, r);
-}
-
 Geo make_geo(const pw_plan *p) {
   Geo g;
   g.nr1 = p->nr1; g.nr2 = p->nr2; g.nr3 = p->nr3; g.ngl = p->ngl;
@@ -1210,64 +905,82 @@ int with_x(const pw_plan *p, F &&f) {
   return f(ICX<0>{});
 }
 
-template <typename T2>
-int run_forward_x(pw_plan *p, const Geo &g, int nb, const double2 *psi, hipStream_t s) {
-  T2 *stripes = (T2 *)p->d_stripe_buf;
+template <typename T2, bool ROW = false>
+int run_forward_x(pw_plan *p, const Geo &g, int nb, const double2 *psi, T2 *stripes, hipStream_t s) {
   constexpr int PX = XTile<T2>::n;
   const dim3 gx = x_grid((p->nstripe + PX - 1) / PX, nb);
   const size_t lds = 2 * PX * x_pitch(p->nr1) * sizeof(T2);
   PW_TRY(with_x(p, [&](auto nx) -> int {
-    k_xfwd<T2, decltype(nx)::value><<<gx, kBlock, lds, s>>>(g, p->f[0], twid<T2>(p, 0), psi, stripes, nb);
+    k_xfwd<T2, decltype(nx)::value, ROW><<<gx, kBlock, lds, s>>>(g, p->f[0], twid<T2>(p, 0), psi, stripes, nb);
     return PW_OK;
   }));
   PW_HIP(hipGetLastError());
   return PW_OK;
 }
 
-template <typename T2>
+template <typename T2, bool ROW = false>
 int run_inverse_x(pw_plan *p, const Geo &g, int nb, double2 *out, const double2 *psi, double scale,
-                  int add_kin, hipStream_t s) {
-  T2 *stripes = (T2 *)p->d_stripe_buf;
+                  int add_kin, const T2 *stripes, hipStream_t s) {
   constexpr int PX = XTile<T2>::n;
   const dim3 gx = x_grid((p->nstripe + PX - 1) / PX, nb);
   const size_t lds = 2 * PX * x_pitch(p->nr1) * sizeof(T2);
   PW_TRY(with_x(p, [&](auto nx) -> int {
-    k_xinv<T2, decltype(nx)::value><<<gx, kBlock, lds, s>>>(g, p->f[0], twid<T2>(p, 0), stripes, out, psi, scale,
-                                                            add_kin, nb);
+    k_xinv<T2, decltype(nx)::value, ROW><<<gx, kBlock, lds, s>>>(g, p->f[0], twid<T2>(p, 0), stripes, out, psi,
+                                                                 scale, add_kin, nb);
     return PW_OK;
   }));
   PW_HIP(hipGetLastError());
   return PW_OK;
 }
 
+// a y (axis 1) or z (axis 2) pass over the pencils of nb bands
 template <typename T2>
-int run_forward_xy(pw_plan *p, const Geo &g, int nb, const double2 *psi, T2 *stripes, T2 *planes,
-                   hipStream_t s) {
-  const int ntx = (p->nr1 + kTX - 1) / kTX;
-  constexpr int PX = XTile<T2>::n;
-  const dim3 gx = x_grid((p->nstripe + PX - 1) / PX, nb);
-  k_xfwd<T2><<<gx, kBlock, 2 * PX * x_pitch(p->nr1) * sizeof(T2), s>>>(g, p->f[0], twid<T2>(p, 0), psi,
-                                                              stripes, nb);
-  dim3 gy(p->nzp * ntx, nb);
-  k_yfwd<T2><<<gy, kBlock, 2 * kTX * p->nr2 * sizeof(T2), s>>>(g, p->f[1], twid<T2>(p, 1),
-                                                               stripes, planes);
+int run_pencils(const pw_plan *p, int axis, int sign, int nb, const PencilArgs &a, hipStream_t s) {
+  const Fft1D &f = p->f[axis];
+  if (pencil_pass(f, sizeof(T2) == sizeof(double2), sign, nb, a, twid<T2>(p, axis), s)) {
+    PW_HIP(hipGetLastError());
+    return PW_OK;
+  }
+  const dim3 grid((unsigned)((a.npen + kTX - 1) / kTX * a.ngrp), nb);
+  const size_t lds = 2 * kTX * (size_t)f.n * sizeof(T2);
+  if (sign > 0) k_pencil_any<T2, +1><<<grid, kBlock, lds, s>>>(a, f, twid<T2>(p, axis));
+  else k_pencil_any<T2, -1><<<grid, kBlock, lds, s>>>(a, f, twid<T2>(p, axis));
   PW_HIP(hipGetLastError());
   return PW_OK;
 }
 
-template <typename T2>
-int run_inverse_yx(pw_plan *p, const Geo &g, int nb, double2 *out, T2 *stripes, T2 *planes,
-                   hipStream_t s) {
-  const int ntx = (p->nr1 + kTX - 1) / kTX;
-  dim3 gy(p->nzp * ntx, nb);
-  k_yinv<T2><<<gy, kBlock, 2 * kTX * p->nr2 * sizeof(T2), s>>>(g, p->f[1], twid<T2>(p, 1),
-                                                               planes, stripes);
-  constexpr int PX = XTile<T2>::n;
-  const dim3 gx = x_grid((p->nstripe + PX - 1) / PX, nb);
-  k_xinv<T2><<<gx, kBlock, 2 * PX * x_pitch(p->nr1) * sizeof(T2), s>>>(g, p->f[0], twid<T2>(p, 0),
-                                                              stripes, out, nullptr, 1.0 / (double)p->nrl, 0, nb);
-  PW_HIP(hipGetLastError());
-  return PW_OK;
+// stripes [stripe][x] <-> planes [iz][y][x]: pencils x of each z plane that holds stripes
+PencilArgs y_pencils(const pw_plan *p, const void *src, void *dst, bool forward) {
+  PencilArgs a{};
+  a.src = src;
+  a.dst = dst;
+  a.npen = p->nr1;
+  a.ngrp = p->nzp;
+  a.grow = p->d_zlist;
+  a.nmap = p->nr2;
+  const size_t nst = (size_t)p->nstripe * p->nr1, npl = (size_t)p->nr2 * p->nr1;
+  a.map = p->d_yz2stripe;
+  a.sstride = a.dstride = p->nr1;
+  a.sband = forward ? nst : npl * p->nzp;
+  a.sgrp = forward ? 0 : npl;
+  a.dband = forward ? npl * p->nzp : nst;
+  a.dgrp = forward ? npl : 0;
+  return a;
+}
+
+// planes [iz][y][x] <-> grid [z][y][x]: pencils (y, x), contiguous in both
+PencilArgs z_pencils(const pw_plan *p, const void *src, void *dst, bool forward) {
+  PencilArgs a{};
+  a.src = src;
+  a.dst = dst;
+  a.npen = p->nr2 * p->nr1;
+  a.ngrp = 1;
+  a.map = p->d_z2iz;
+  a.sstride = a.dstride = a.npen;
+  const size_t npl = (size_t)p->nzp * a.npen;
+  a.sband = forward ? npl : (size_t)p->nrl;
+  a.dband = forward ? (size_t)p->nrl : npl;
+  return a;
 }
 
 // dynamic LDS of a yz workgroup; beyond 64 KiB the kernel's limit is raised
@@ -1344,7 +1057,7 @@ int vpsi_t(pw_plan *p, int nb, const double2 *psi, const double *v, double2 *hps
   PW_TRY(yz_fits(p, lds));
   Geo g = make_geo(p);
   PW_TRY(vt_of<T2>(p, v, s));
-  PW_TRY(run_forward_x<T2>(p, g, nb, psi, s));
+  PW_TRY(run_forward_x<T2>(p, g, nb, psi, (T2 *)p->d_stripe_buf, s));
   if (yz_big(p)) {
     PW_TRY(yz_lds(k_yz_vpsi<T2, true>, lds));
     k_yz_vpsi<T2, true><<<dim3(p->nr1, nb), kYZ, lds, s>>>(g, p->fyz[0], p->fyz[1], twid<T2>(p, 1), twid<T2>(p, 2),
@@ -1359,7 +1072,7 @@ int vpsi_t(pw_plan *p, int nb, const double2 *psi, const double *v, double2 *hps
     }));
   }
   PW_HIP(hipGetLastError());
-  return run_inverse_x<T2>(p, g, nb, hpsi, psi, 1.0 / (double)p->nrl, add_kin, s);
+  return run_inverse_x<T2>(p, g, nb, hpsi, psi, 1.0 / (double)p->nrl, add_kin, (const T2 *)p->d_stripe_buf, s);
 }
 
 template <typename T2>
@@ -1375,7 +1088,7 @@ int density_t(pw_plan *p, int nb, const double2 *psi, const double *occ2, double
                      ((size_t)p->yzpitch * p->nr3 + p->nr2 + p->nr3) * sizeof(T2) + (size_t)p->nzp * sizeof(int);
   PW_TRY(yz_fits(p, lds));
   Geo g = make_geo(p);
-  PW_TRY(run_forward_x<T2>(p, g, nb, psi, s));
+  PW_TRY(run_forward_x<T2>(p, g, nb, psi, (T2 *)p->d_stripe_buf, s));
   // band groups so that the grid holds about target_blocks workgroups
   int ngrp = std::max(1, std::min(nb, (target_blocks + p->nr1 - 1) / p->nr1));
   const int bpg = (nb + ngrp - 1) / ngrp;
@@ -1417,23 +1130,18 @@ int density_t(pw_plan *p, int nb, const double2 *psi, const double *occ2, double
 // both is written before it is read, so neither needs clearing
 template <typename T2>
 int gtor_t(pw_plan *p, int nb, const double2 *fofg, T2 *fofr, T2 *stripes, T2 *planes, hipStream_t s) {
-  Geo g = make_geo(p);
-  PW_TRY(run_forward_xy<T2>(p, g, nb, fofg, stripes, planes, s));
-  const int ntx = (p->nr1 + kTX - 1) / kTX;
-  dim3 gz(p->nr2 * ntx, nb);
-  k_zout<T2><<<gz, kBlock, 2 * kTX * p->nr3 * sizeof(T2), s>>>(g, p->f[2], twid<T2>(p, 2), planes, fofr);
-  PW_HIP(hipGetLastError());
-  return PW_OK;
+  const Geo g = make_geo(p);
+  PW_TRY((run_forward_x<T2, true>(p, g, nb, fofg, stripes, s)));
+  PW_TRY(run_pencils<T2>(p, 1, +1, nb, y_pencils(p, stripes, planes, true), s));
+  return run_pencils<T2>(p, 2, +1, nb, z_pencils(p, planes, fofr, true), s);
 }
 
 template <typename T2>
 int rtog_t(pw_plan *p, int nb, double2 *fofg, const T2 *fofr, T2 *stripes, T2 *planes, hipStream_t s) {
-  Geo g = make_geo(p);
-  const int ntx = (p->nr1 + kTX - 1) / kTX;
-  dim3 gz(p->nr2 * ntx, nb);
-  k_zin<T2><<<gz, kBlock, 2 * kTX * p->nr3 * sizeof(T2), s>>>(g, p->f[2], twid<T2>(p, 2), fofr, planes);
-  PW_HIP(hipGetLastError());
-  return run_inverse_yx<T2>(p, g, nb, fofg, stripes, planes, s);
+  const Geo g = make_geo(p);
+  PW_TRY(run_pencils<T2>(p, 2, -1, nb, z_pencils(p, fofr, planes, false), s));
+  PW_TRY(run_pencils<T2>(p, 1, -1, nb, y_pencils(p, planes, stripes, false), s));
+  return run_inverse_x<T2, true>(p, g, nb, fofg, nullptr, 1.0 / (double)p->nrl, 0, stripes, s);
 }
 
 // full-grid transforms in batches of at most c bands through the given buffers

@@ -152,6 +152,7 @@ struct pw_plan {
   void *d_vt = nullptr; size_t vt_bytes = 0;   // V(r) as [x][z][y] in the work precision
   // POTENTIAL$VOFRHO on this (density) plane-wave object: setup tables and work
   double *d_pot_tabs = nullptr; int pot_nsp = 0;
+  bool pot_sym = true;         // the tables have T(G) = T(-G): one G of each pair suffices
   std::vector<int> pot_lmrx;   // LMRX per species (POTENTIAL_HARTREE's LMRX(NSP))
   void *d_pot = nullptr; size_t pot_bytes = 0;
   double *h_pot = nullptr; size_t h_pot_bytes = 0; int pot_nat = 0;   // pinned: results and staged atom data
@@ -176,8 +177,11 @@ int plan_device(pw_plan *p);   // uploads maps and twiddles on first use
 // FFT pipelines (pw_fft.hip).  T selects the arithmetic (FP64 / FP32).
 // psi/fofg are complex128 sphere arrays (NGL per band).
 struct FftCtx;
-int fft_gtor_full(pw_plan *p, int nfft, const double2 *fofg, void *fofr, int prec, hipStream_t s);
-int fft_rtog_full(pw_plan *p, int nfft, double2 *fofg, const void *fofr, int prec, hipStream_t s);
+// real (FP64): fofr is a real array of NRL per transform (the imaginary part
+// dropped or zero); add: sphere coefficients added to the result
+int fft_gtor_full(pw_plan *p, int nfft, const double2 *fofg, void *fofr, int prec, hipStream_t s, bool real = false);
+int fft_rtog_full(pw_plan *p, int nfft, double2 *fofg, const void *fofr, int prec, hipStream_t s, bool real = false,
+                  const double2 *add = nullptr);
 // hpsi = FFT^-1[v FFT psi] + (add_kin ? G^2/2 psi : 0)
 int fft_vpsi(pw_plan *p, int nb, const double2 *psi, const double *v, double2 *hpsi,
              int add_kin, int prec, hipStream_t s);

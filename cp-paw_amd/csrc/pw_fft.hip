@@ -117,18 +117,26 @@ template <typename T2> struct XTile;
 template <> struct XTile<double2> { static constexpr int n = 16; };
 template <> struct XTile<float2> { static constexpr int n = 32; };
 
-// Workgroup -> (stripe group, band) of the x passes, a 1D grid of
-// 8 ceil(nb/8) ngroups workgroups: consecutive workgroups go to the eight XCDs
-// in turn, and each XCD takes every stripe group of its bands (band = xcd +
+// Workgroup -> (stripe group, band) of the x passes, a 1D grid of nb ngroups
+// workgroups: consecutive workgroups go to the eight XCDs in turn.  In whole
+// octets of bands each XCD takes every stripe group of its bands (band = xcd +
 // 8 k), so the coefficients of a band, gathered and scattered in G order by
-// all its stripe groups, pass through one XCD's L2 instead of eight.
-__device__ inline bool x_block(int ngroups, int nb, int &group, int &band) {
-  const int id = blockIdx.x, x = id % 8, j = id / 8;
-  band = x + 8 * (j / ngroups);
+// all its stripe groups, pass through one XCD's L2 instead of eight.  The
+// groups of the last nb mod 8 bands are dealt to all XCDs: with one band
+// (VOFRHO's transforms) they had all run on one XCD, 21 and 17 us for the
+// passes of the Si64 density sphere against 9 and 8.
+__device__ inline void x_block(int ngroups, int nb, int &group, int &band) {
+  const int id = blockIdx.x, whole = nb / 8 * 8, r = id - whole * ngroups;
+  if (r >= 0) {
+    band = whole + r / ngroups;
+    group = r % ngroups;
+    return;
+  }
+  const int j = id / 8;
+  band = id % 8 + 8 * (j / ngroups);
   group = j % ngroups;
-  return band < nb;
 }
-inline dim3 x_grid(int ngroups, int nb) { return dim3((unsigned)(8 * ((nb + 7) / 8) * ngroups)); }
+inline dim3 x_grid(int ngroups, int nb) { return dim3((unsigned)(nb * ngroups)); }
 // LDS pitch of the x passes' stripe tiles: odd, so that the tile's transposes
 // (neighbouring lanes on neighbouring stripes, one pitch apart) fall into
 // distinct banks
@@ -143,7 +151,7 @@ __global__ void __launch_bounds__(kBlock) k_xfwd(Geo g, Fft1D f, const T2 *tw, c
   constexpr int PX = XTile<T2>::n;
   if constexpr (NX > 0) g.nr1 = NX;
   int grp, band;
-  if (!x_block((g.nstripe + PX - 1) / PX, nb, grp, band)) return;
+  x_block((g.nstripe + PX - 1) / PX, nb, grp, band);
   extern __shared__ unsigned char smem_raw[];
   const int xp = x_pitch(g.nr1);
   T2 *b0 = reinterpret_cast<T2 *>(smem_raw);
@@ -173,6 +181,8 @@ __global__ void __launch_bounds__(kBlock) k_xfwd(Geo g, Fft1D f, const T2 *tw, c
 }
 
 // ---- x pass, inverse: stripes -> sphere (gather, scale, optional G^2/2 psi) ---
+// add_kin: 0 nothing, 1 + G^2/2 psi, kAddPlain + psi
+constexpr int kAddPlain = 2;
 template <typename T2, int NX = 0, bool ROW = false>
 __global__ void __launch_bounds__(kBlock) k_xinv(Geo g, Fft1D f, const T2 *tw, const T2 *stripes,
                                                  double2 *out, const double2 *psi, double scale,
@@ -180,7 +190,7 @@ __global__ void __launch_bounds__(kBlock) k_xinv(Geo g, Fft1D f, const T2 *tw, c
   constexpr int PX = XTile<T2>::n;
   if constexpr (NX > 0) g.nr1 = NX;
   int grp, band;
-  if (!x_block((g.nstripe + PX - 1) / PX, nb, grp, band)) return;
+  x_block((g.nstripe + PX - 1) / PX, nb, grp, band);
   extern __shared__ unsigned char smem_raw[];
   const int xp = x_pitch(g.nr1);
   T2 *b0 = reinterpret_cast<T2 *>(smem_raw);
@@ -210,7 +220,7 @@ __global__ void __launch_bounds__(kBlock) k_xinv(Geo g, Fft1D f, const T2 *tw, c
     T2 v = r[(g.stripe_s[e] - s0) * xp + g.stripe_x[e]];
     double2 o = make_double2((double)v.x * scale, (double)v.y * scale);
     if (add_kin) {
-      const double h = 0.5 * g.g2[ig];
+      const double h = add_kin == kAddPlain ? 1.0 : 0.5 * g.g2[ig];
       const double2 p = ps[ig];
       o.x += h * p.x;
       o.y += h * p.y;
@@ -222,13 +232,13 @@ __global__ void __launch_bounds__(kBlock) k_xinv(Geo g, Fft1D f, const T2 *tw, c
 // ---- y and z passes of the full-grid transforms, any length --------------------
 // The pass of pw_pencil.h with the length and the stages from the plan, for
 // lengths that have no instantiation there: kTX pencils in LDS.
-template <typename T2, int SIGN>
+template <typename T2, int SIGN, bool REAL>
 __global__ void __launch_bounds__(kBlock) k_pencil_any(PencilArgs a, Fft1D f, const T2 *tw) {
   extern __shared__ unsigned char smem_raw[];
   T2 *b0 = reinterpret_cast<T2 *>(smem_raw);
   T2 *b1 = b0 + kTX * f.n;
   const int ntile = (a.npen + kTX - 1) / kTX, grp = blockIdx.x / ntile, q0 = (blockIdx.x % ntile) * kTX;
-  const PencilIo<T2> io(a, grp, blockIdx.y, SIGN > 0);
+  const PencilIo<T2> io(a, grp, blockIdx.y, SIGN > 0, REAL);
   for (int w = threadIdx.x; w < f.n * kTX; w += blockDim.x) b0[w] = io.load(w / kTX, q0 + w % kTX);
   __syncthreads();
   const T2 *r = lds_fft<T2>(b0, b1, f, kTX, kTX, 1, tw, SIGN, true);
@@ -943,8 +953,17 @@ int run_pencils(const pw_plan *p, int axis, int sign, int nb, const PencilArgs &
   }
   const dim3 grid((unsigned)((a.npen + kTX - 1) / kTX * a.ngrp), nb);
   const size_t lds = 2 * kTX * (size_t)f.n * sizeof(T2);
-  if (sign > 0) k_pencil_any<T2, +1><<<grid, kBlock, lds, s>>>(a, f, twid<T2>(p, axis));
-  else k_pencil_any<T2, -1><<<grid, kBlock, lds, s>>>(a, f, twid<T2>(p, axis));
+  const auto tw = twid<T2>(p, axis);
+  if constexpr (sizeof(T2) == sizeof(double2)) {
+    if (a.real) {
+      if (sign > 0) k_pencil_any<T2, +1, true><<<grid, kBlock, lds, s>>>(a, f, tw);
+      else k_pencil_any<T2, -1, true><<<grid, kBlock, lds, s>>>(a, f, tw);
+      PW_HIP(hipGetLastError());
+      return PW_OK;
+    }
+  }
+  if (sign > 0) k_pencil_any<T2, +1, false><<<grid, kBlock, lds, s>>>(a, f, tw);
+  else k_pencil_any<T2, -1, false><<<grid, kBlock, lds, s>>>(a, f, tw);
   PW_HIP(hipGetLastError());
   return PW_OK;
 }
@@ -969,8 +988,9 @@ PencilArgs y_pencils(const pw_plan *p, const void *src, void *dst, bool forward)
 }
 
 // planes [iz][y][x] <-> grid [z][y][x]: pencils (y, x), contiguous in both
-PencilArgs z_pencils(const pw_plan *p, const void *src, void *dst, bool forward) {
+PencilArgs z_pencils(const pw_plan *p, const void *src, void *dst, bool forward, bool real) {
   PencilArgs a{};
+  a.real = real;
   a.src = src;
   a.dst = dst;
   a.npen = p->nr2 * p->nr1;
@@ -1129,35 +1149,38 @@ int density_t(pw_plan *p, int nb, const double2 *psi, const double *occ2, double
 // (nb x NSTRIPE x NR1) and planes (nb x NZPLANE x NR2 x NR1); every element of
 // both is written before it is read, so neither needs clearing
 template <typename T2>
-int gtor_t(pw_plan *p, int nb, const double2 *fofg, T2 *fofr, T2 *stripes, T2 *planes, hipStream_t s) {
+int gtor_t(pw_plan *p, int nb, const double2 *fofg, void *fofr, T2 *stripes, T2 *planes, bool real, hipStream_t s) {
   const Geo g = make_geo(p);
   PW_TRY((run_forward_x<T2, true>(p, g, nb, fofg, stripes, s)));
   PW_TRY(run_pencils<T2>(p, 1, +1, nb, y_pencils(p, stripes, planes, true), s));
-  return run_pencils<T2>(p, 2, +1, nb, z_pencils(p, planes, fofr, true), s);
+  return run_pencils<T2>(p, 2, +1, nb, z_pencils(p, planes, fofr, true, real), s);
 }
 
 template <typename T2>
-int rtog_t(pw_plan *p, int nb, double2 *fofg, const T2 *fofr, T2 *stripes, T2 *planes, hipStream_t s) {
+int rtog_t(pw_plan *p, int nb, double2 *fofg, const void *fofr, T2 *stripes, T2 *planes, bool real, const double2 *add,
+           hipStream_t s) {
   const Geo g = make_geo(p);
-  PW_TRY(run_pencils<T2>(p, 2, -1, nb, z_pencils(p, fofr, planes, false), s));
+  PW_TRY(run_pencils<T2>(p, 2, -1, nb, z_pencils(p, fofr, planes, false, real), s));
   PW_TRY(run_pencils<T2>(p, 1, -1, nb, y_pencils(p, planes, stripes, false), s));
-  return run_inverse_x<T2, true>(p, g, nb, fofg, nullptr, 1.0 / (double)p->nrl, 0, stripes, s);
+  return run_inverse_x<T2, true>(p, g, nb, fofg, add, 1.0 / (double)p->nrl, add ? kAddPlain : 0, stripes, s);
 }
 
-// full-grid transforms in batches of at most c bands through the given buffers
+// full-grid transforms in batches of at most c bands through the given
+// buffers; real (FP64): fofr is a real array; add: added to the coefficients (RTOG)
 int full_fft(pw_plan *p, bool gtor, int nfft, int c, double2 *fofg, void *fofr, int prec, void *stripes,
-             void *planes, hipStream_t s) {
+             void *planes, hipStream_t s, bool real = false, const double2 *add = nullptr) {
+  const size_t es = prec != PW_PREC_FP64 ? sizeof(float2) : (real ? sizeof(double) : sizeof(double2));
   for (int b0 = 0; b0 < nfft; b0 += c) {
     const int n = std::min(c, nfft - b0);
     double2 *fg = fofg + (size_t)b0 * p->ngl;
+    void *fr = (char *)fofr + (size_t)b0 * p->nrl * es;
+    const double2 *ad = add ? add + (size_t)b0 * p->ngl : nullptr;
     if (prec == PW_PREC_FP64) {
-      double2 *fr = (double2 *)fofr + (size_t)b0 * p->nrl;
-      if (gtor) PW_TRY(gtor_t<double2>(p, n, fg, fr, (double2 *)stripes, (double2 *)planes, s));
-      else PW_TRY(rtog_t<double2>(p, n, fg, fr, (double2 *)stripes, (double2 *)planes, s));
+      if (gtor) PW_TRY(gtor_t<double2>(p, n, fg, fr, (double2 *)stripes, (double2 *)planes, real, s));
+      else PW_TRY(rtog_t<double2>(p, n, fg, fr, (double2 *)stripes, (double2 *)planes, real, ad, s));
     } else {
-      float2 *fr = (float2 *)fofr + (size_t)b0 * p->nrl;
-      if (gtor) PW_TRY(gtor_t<float2>(p, n, fg, fr, (float2 *)stripes, (float2 *)planes, s));
-      else PW_TRY(rtog_t<float2>(p, n, fg, fr, (float2 *)stripes, (float2 *)planes, s));
+      if (gtor) PW_TRY(gtor_t<float2>(p, n, fg, fr, (float2 *)stripes, (float2 *)planes, false, s));
+      else PW_TRY(rtog_t<float2>(p, n, fg, fr, (float2 *)stripes, (float2 *)planes, false, ad, s));
     }
   }
   return PW_OK;
@@ -1197,16 +1220,18 @@ int fft_density(pw_plan *p, int nb, const double2 *psi, const double *occ2, doub
   return density_t<float2>(p, nb, psi, occ2, rho, target_blocks, s);
 }
 
-int fft_gtor_full(pw_plan *p, int nfft, const double2 *fofg, void *fofr, int prec, hipStream_t s) {
+int fft_gtor_full(pw_plan *p, int nfft, const double2 *fofg, void *fofr, int prec, hipStream_t s, bool real) {
   const int c = chunk_of(p, prec);
   PW_TRY(plan_work(p, std::min(nfft, c), prec, true));
-  return full_fft(p, true, nfft, c, const_cast<double2 *>(fofg), fofr, prec, p->d_stripe_buf, p->d_plane_buf, s);
+  return full_fft(p, true, nfft, c, const_cast<double2 *>(fofg), fofr, prec, p->d_stripe_buf, p->d_plane_buf, s, real);
 }
 
-int fft_rtog_full(pw_plan *p, int nfft, double2 *fofg, const void *fofr, int prec, hipStream_t s) {
+int fft_rtog_full(pw_plan *p, int nfft, double2 *fofg, const void *fofr, int prec, hipStream_t s, bool real,
+                  const double2 *add) {
   const int c = chunk_of(p, prec);
   PW_TRY(plan_work(p, std::min(nfft, c), prec, true));
-  return full_fft(p, false, nfft, c, fofg, const_cast<void *>(fofr), prec, p->d_stripe_buf, p->d_plane_buf, s);
+  return full_fft(p, false, nfft, c, fofg, const_cast<void *>(fofr), prec, p->d_stripe_buf, p->d_plane_buf, s, real,
+                  add);
 }
 
 // ---------------------------------------------------------------------------

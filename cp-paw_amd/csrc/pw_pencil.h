@@ -14,6 +14,7 @@ struct PencilArgs {
   int npen, ngrp;              // pencils of a group, groups
   const int *map, *grow;
   int nmap, sstride, dstride;
+  bool real;                   // FP64: the grid side is a real array (imaginary parts zero / dropped)
   size_t sband, sgrp, dband, dgrp;
 };
 
@@ -27,14 +28,25 @@ template <typename T2> struct PencilIo {
   const int *map;
   unsigned ss, ds;
   int npen;
-  bool forward;   // a constant in every kernel
-  __device__ PencilIo(const PencilArgs &a, int grp, int band, bool forward)
+  bool forward, real;   // constants in every kernel
+  __device__ PencilIo(const PencilArgs &a, int grp, int band, bool forward, bool real)
       : src((const T2 *)a.src + band * a.sband + grp * a.sgrp), dst((T2 *)a.dst + band * a.dband + grp * a.dgrp),
         map(a.map + (a.grow ? a.nmap * a.grow[grp] : 0)), ss(a.sstride), ds(a.dstride), npen(a.npen),
-        forward(forward) {}
+        forward(forward), real(real) {
+    // the real side counts elements of half the size (one group)
+    if (real && forward) dst = (T2 *)((decltype(T2::x) *)a.dst + band * a.dband);
+    if (real && !forward) src = (const T2 *)((const decltype(T2::x) *)a.src + band * a.sband);
+  }
   __device__ T2 load(int e, int q) const {
     const int m = forward ? map[e] : e;
-    const T2 v = src[(unsigned)max(m, 0) * ss + (unsigned)min(q, npen - 1)];
+    const unsigned o = (unsigned)max(m, 0) * ss + (unsigned)min(q, npen - 1);
+    T2 v;
+    if (real && !forward) {
+      v.x = reinterpret_cast<const decltype(v.x) *>(src)[o];
+      v.y = 0;
+    } else {
+      v = src[o];
+    }
     const bool ok = m >= 0 && q < npen;
     T2 z;
     z.x = ok ? v.x : 0;
@@ -46,8 +58,13 @@ template <typename T2> struct PencilIo {
     typedef decltype(v.x) V2 __attribute__((ext_vector_type(2)));
     const int m = forward ? e : map[e];
     if (m < 0 || q >= npen) return;
-    const V2 o = {v.x, v.y};
-    __builtin_nontemporal_store(o, reinterpret_cast<V2 *>(dst + ((unsigned)m * ds + (unsigned)q)));
+    const unsigned i = (unsigned)m * ds + (unsigned)q;
+    if (real && forward) {
+      reinterpret_cast<decltype(v.x) *>(dst)[i] = v.x;
+    } else {
+      const V2 o = {v.x, v.y};
+      __builtin_nontemporal_store(o, reinterpret_cast<V2 *>(dst + i));
+    }
   }
 };
 

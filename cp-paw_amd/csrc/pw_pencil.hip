@@ -82,13 +82,13 @@ __device__ inline void pencil_stage(const PencilIo<T2> &io, int q0, T2 *in, T2 *
   }
 }
 
-template <typename T2, int N, int SIGN>
+template <typename T2, int N, int SIGN, bool REAL>
 __global__ void __launch_bounds__(kPB) k_pencil(PencilArgs a, const T2 *__restrict__ tw) {
   constexpr int NST = pencil_stages<T2>(N).nstage, TP = pencil_tile<T2, N>();
   // stage 0 writes b1; a third stage writes b0
   __shared__ T2 b1[NST > 1 ? N * TP : 1], b0[NST > 2 ? N * TP : 1];
   const int ntile = (a.npen + TP - 1) / TP, grp = blockIdx.x / ntile, q0 = (blockIdx.x - grp * ntile) * TP;
-  const PencilIo<T2> io(a, grp, blockIdx.y, SIGN > 0);
+  const PencilIo<T2> io(a, grp, blockIdx.y, SIGN > 0, REAL);
   pencil_stage<T2, N, 0, 1>(io, q0, b0, b1, tw, SIGN);
 }
 
@@ -96,8 +96,15 @@ template <typename T2, int N>
 void launch(int sign, int nb, const PencilArgs &a, const void *tw, hipStream_t s) {
   constexpr int TP = pencil_tile<T2, N>();
   const dim3 grid((unsigned)((a.npen + TP - 1) / TP * a.ngrp), nb);
-  if (sign > 0) k_pencil<T2, N, +1><<<grid, kPB, 0, s>>>(a, (const T2 *)tw);
-  else k_pencil<T2, N, -1><<<grid, kPB, 0, s>>>(a, (const T2 *)tw);
+  if constexpr (sizeof(T2) == sizeof(double2)) {
+    if (a.real) {
+      if (sign > 0) k_pencil<T2, N, +1, true><<<grid, kPB, 0, s>>>(a, (const T2 *)tw);
+      else k_pencil<T2, N, -1, true><<<grid, kPB, 0, s>>>(a, (const T2 *)tw);
+      return;
+    }
+  }
+  if (sign > 0) k_pencil<T2, N, +1, false><<<grid, kPB, 0, s>>>(a, (const T2 *)tw);
+  else k_pencil<T2, N, -1, false><<<grid, kPB, 0, s>>>(a, (const T2 *)tw);
 }
 
 }  // namespace

@@ -24,8 +24,9 @@
 // so results do not depend on scheduling.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
-#include "pw_common.h"
+#include "pw_device.h"
 
 namespace {
 
@@ -41,12 +42,15 @@ constexpr double kAU = 31.10e-3, kBU = -48.0e-3, kCU = 2.0e-3, kDU = -11.6e-3;
 struct PotGeo {
   int ngl, nrl, nat, nsp, ngamma, lmrxx;
   const int *lmrx;       // nsp: LMRX of each species
+  const int2 *hg;        // (G, -G) of each pair of the half list, nh of them
+  int nh, full;          // full: every G on its own (tables without T(G) = T(-G))
+  const double2 *phase;  // nat x 3 x nph: exp(-i n b_k . R_a), n = -nmax .. nmax
+  int nph;
   const int *igvec;      // 3 x ngl
   const double *gvec;    // 3 x ngl
   const double *g2;      // ngl
   const double *tabs;    // [4][nsp][ngl]: PSCORG, VBARG, G0, V0
   const int *isp;        // nat, 0-based
-  const double *gr;      // nat x 3: b_k . R_a
   const double *qlm;     // nat x lmrxx (QLM(LMRXX,NAT))
   double vol;
 };
@@ -122,24 +126,35 @@ __device__ inline double2 cfac_l(int l) {
 
 __device__ inline int l_of(int lm) { return lm < 1 ? 0 : (lm < 4 ? 1 : (lm < 9 ? 2 : (lm < 16 ? 3 : 4))); }
 
-// sum_{LM < LMRX} CFAC(LM) QLM(LM) YLMOFG(LM) (complex)
-__device__ inline double2 comp_factor(const PotGeo &g, int a, int n, const double *y) {
+// sum_{LM < n} CFAC(LM) QLM(LM) YLMOFG(LM) (complex), n <= LM
+template <int LM>
+__device__ inline double2 comp_factor(const double *q, int n, const double *y) {
   double re = 0.0, im = 0.0;
-  const double *q = g.qlm + (size_t)a * g.lmrxx;
-  for (int lm = 0; lm < n; ++lm) {
+#pragma unroll
+  for (int lm = 0; lm < LM; ++lm) {
     const double2 c = cfac_l(l_of(lm));
-    re += c.x * q[lm] * y[lm];
-    im += c.y * q[lm] * y[lm];
+    const double v = lm < n ? q[lm] * y[lm] : 0.0;
+    re += c.x * v;
+    im += c.y * v;
   }
   return make_double2(re, im);
 }
 
-__device__ inline double2 eigr(const PotGeo &g, int a, int ig) {
-  const double ph = (double)g.igvec[3 * ig] * g.gr[3 * a] + (double)g.igvec[3 * ig + 1] * g.gr[3 * a + 1] +
-                    (double)g.igvec[3 * ig + 2] * g.gr[3 * a + 2];
+// the G pair of index h: (G, -G), the second equal to the first for a G on its own
+__device__ inline int2 pot_pair(const PotGeo &g, int h) { return g.full ? make_int2(h, h) : g.hg[h]; }
+
+// phase tables of all atoms, exp(-i n b_k . R_a)
+__global__ void k_pot_phase(int nat, int nph, const double *gr, double2 *phase) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nat * 3 * nph) return;
   double s, c;
-  sincos(ph, &s, &c);
-  return make_double2(c, -s);
+  sincos((double)(i % nph - nph / 2) * gr[i / nph], &s, &c);
+  phase[i] = make_double2(c, -s);
+}
+
+// exp(-i G.R) from one atom's tables in LDS
+__device__ inline double2 pot_eigr(const double2 *ph, int nph, int3 n) {
+  return cmul(cmul(ph[n.x], ph[nph + n.y]), ph[2 * nph + n.z]);
 }
 
 __device__ inline double tab(const PotGeo &g, int which, int s, int ig) {
@@ -160,72 +175,127 @@ __device__ inline double block_sum(double v, double *sh) {
   return r;
 }
 
-__global__ void k_real_to_c(int n, const double *__restrict__ r, double2 *__restrict__ c) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) c[i] = make_double2(r[i], 0.0);
-}
-
-__global__ void k_c_to_real(int n, const double2 *__restrict__ c, double *__restrict__ r) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) r[i] = c[i].x;
-}
-
-// Per G: core, compensation, VBAR and V0 sums over atoms; the background and
-// the Hartree potential; EHARTREE partial sums (src/paw_potential.f90:
-// 1038-1066, 1145-1205).  rhog gains the core; vg = VG; vh = POT + VG.
-// scal[0] = RHOB (written by the thread of G = 0).
-__global__ void __launch_bounds__(kPotThreads) k_pot_g(PotGeo g, double2 *__restrict__ rhog,
+// Per G pair: core, compensation, VBAR and V0 sums over atoms; the background
+// and the Hartree potential; EHARTREE partial sums (src/paw_potential.f90:
+// 1038-1066, 1145-1205).  rhog gains the core; vg = VG; vh = POT + VG; the
+// values at -G are the conjugates (real density, radial tables).  scal[0] =
+// RHOB (written by the thread of G = 0).
+//
+// Bound by the NAT x NG phase factors: each is a product of three table
+// entries in LDS instead of a sincos, formed once for G and -G, and enters
+// the sums of its species (the tables are applied once per run of atoms of
+// one species).  A workgroup takes 256 pairs with four groups of waves that
+// share the atoms of a chunk (the tables of a chunk are read once per 256
+// pairs and 16 waves keep a CU busy).  72 -> 31 us at Si64 (191 711 G, 64
+// atoms); 64 pairs per workgroup, which reads the tables four times as often,
+// took 59 us.
+constexpr int kPotG = 256, kPotS = 4;      // G pairs and atom groups of a k_pot_g workgroup
+struct PotSums {
+  double2 core, comp, pot;
+};
+template <int LM>
+__global__ void __launch_bounds__(kPotG *kPotS) k_pot_g(PotGeo g, int ac, double2 *__restrict__ rhog,
                                                        double2 *__restrict__ vg_out, double2 *__restrict__ vh,
                                                        double *__restrict__ epart, double *__restrict__ scal) {
-  __shared__ double sh[kPotThreads / 64];
-  const int ig = blockIdx.x * kPotThreads + threadIdx.x;
-  double e = 0.0;
-  if (ig < g.ngl) {
-    double2 core = {0.0, 0.0}, comp = {0.0, 0.0}, pot = {0.0, 0.0};
-    double vb = 0.0;
-    double y[kLmrxxMax];
-    solid_ylm(g.lmrxx, g.gvec[3 * ig], g.gvec[3 * ig + 1], g.gvec[3 * ig + 2], y);
-    for (int a = 0; a < g.nat; ++a) {
-      const int s = g.isp[a];
-      const double2 ea = eigr(g, a, ig);
+  extern __shared__ double2 sph[];         // ac atoms x 3 x nph
+  __shared__ PotSums red[kPotS - 1][kPotG];
+  __shared__ double she[kPotG / 64];
+  const int hl = threadIdx.x % kPotG, grp = threadIdx.x / kPotG;
+  const int h = blockIdx.x * kPotG + hl, nh = g.full ? g.ngl : g.nh;
+  const bool in = h < nh;
+  const int2 gp = pot_pair(g, in ? h : 0);
+  const int ig = gp.x;
+  const int nm = g.nph / 2;
+  const int3 n = make_int3(g.igvec[3 * ig] + nm, g.igvec[3 * ig + 1] + nm, g.igvec[3 * ig + 2] + nm);
+  double y[LM];
+  solid_ylm(LM, g.gvec[3 * ig], g.gvec[3 * ig + 1], g.gvec[3 * ig + 2], y);
+  PotSums a = {czero(), czero(), czero()};
+  double2 se = czero(), sq = czero();      // sums of exp(-iG.R) and of the compensation factors of one species
+  int sp = -1;
+  auto flush = [&]() {
+    if (sp < 0) return;
+    const double fc = tab(g, 0, sp, ig) * kY0, vbar = tab(g, 1, sp, ig) * kY0;
+    const double g0 = tab(g, 2, sp, ig), v0 = tab(g, 3, sp, ig);
+    a.core.x += fc * se.x;
+    a.core.y += fc * se.y;
+    a.comp.x += g0 * sq.x;
+    a.comp.y += g0 * sq.y;
+    a.pot.x += v0 * sq.x + vbar * se.x;
+    a.pot.y += v0 * sq.y + vbar * se.y;
+    se = sq = czero();
+  };
+  for (int a0 = 0; a0 < g.nat; a0 += ac) {
+    const int na = min(ac, g.nat - a0);
+    __syncthreads();
+    for (int i = threadIdx.x; i < na * 3 * g.nph; i += kPotG * kPotS) sph[i] = g.phase[(size_t)a0 * 3 * g.nph + i];
+    __syncthreads();
+    for (int k = grp; k < na; k += kPotS) {
+      const int at = a0 + k, s = g.isp[at];
+      if (s != sp) {
+        flush();
+        sp = s;
+      }
+      const double2 e = pot_eigr(sph + (size_t)k * 3 * g.nph, g.nph, n);
       // CSVAR = sum_LM CFAC(LM) QLM(LM) YLMOFG(LM,G) EIGR(G)
-      const double2 cs = cmul(comp_factor(g, a, g.lmrx[s], y), ea);
-      const double fc = tab(g, 0, s, ig) * kY0;
-      const double g0 = tab(g, 2, s, ig), v0 = tab(g, 3, s, ig), vbar = tab(g, 1, s, ig) * kY0;
-      core.x += fc * ea.x;
-      core.y += fc * ea.y;
-      comp.x += cs.x * g0;
-      comp.y += cs.y * g0;
-      pot.x += cs.x * v0 + vbar * ea.x;
-      pot.y += cs.y * v0 + vbar * ea.y;
-      if (ig == g.ngamma) vb += g.qlm[(size_t)a * g.lmrxx] * kY0 * v0;
+      const double2 c = comp_factor<LM>(g.qlm + (size_t)at * g.lmrxx, g.lmrx[s], y);
+      se = cadd(se, e);
+      sq = cadd(sq, cmul(c, e));
+    }
+  }
+  flush();
+  if (grp > 0) red[grp - 1][hl] = a;
+  __syncthreads();
+  double e = 0.0;
+  if (grp == 0 && in) {
+#pragma unroll
+    for (int w = 0; w < kPotS - 1; ++w) {
+      a.core = cadd(a.core, red[w][hl].core);
+      a.comp = cadd(a.comp, red[w][hl].comp);
+      a.pot = cadd(a.pot, red[w][hl].pot);
     }
     double2 rg = rhog[ig];
-    rg.x += core.x;
-    rg.y += core.y;
-    rhog[ig] = rg;
-    double2 r2 = {rg.x + comp.x, rg.y + comp.y};
+    rg.x += a.core.x;
+    rg.y += a.core.y;
+    const double2 r2 = cadd(rg, a.comp);
     double2 v;
     if (ig == g.ngamma) {
+      double vb = 0.0;
+      for (int at = 0; at < g.nat; ++at) vb += g.qlm[(size_t)at * g.lmrxx] * kY0 * tab(g, 3, g.isp[at], ig);
       const double rhob = -r2.x;
       v = make_double2(-vb, 0.0);
-      e = (rg.x * pot.x + rg.y * pot.y) + rhob * vb;
+      e = (rg.x * a.pot.x + rg.y * a.pot.y) + rhob * vb;
       scal[0] = rhob;
     } else {
       const double f = 4.0 * kPi / g.g2[ig];
       v = make_double2(r2.x * f, r2.y * f);
-      e = 0.5 * (r2.x * v.x + r2.y * v.y) + (rg.x * pot.x + rg.y * pot.y);
+      e = 0.5 * (r2.x * v.x + r2.y * v.y) + (rg.x * a.pot.x + rg.y * a.pot.y);
     }
+    const double2 o = cadd(a.pot, v);
+    rhog[ig] = rg;
     vg_out[ig] = v;
-    vh[ig] = make_double2(pot.x + v.x, pot.y + v.y);
+    vh[ig] = o;
+    if (gp.y != gp.x) {
+      rhog[gp.y] = cconj(rg);
+      vg_out[gp.y] = cconj(v);
+      vh[gp.y] = cconj(o);
+      e *= 2.0;
+    }
   }
-  const double s = block_sum(e, sh);
-  if (threadIdx.x == 0) epart[blockIdx.x] = s;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o);
+  if (grp == 0 && hl % 64 == 0) she[hl / 64] = e;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double r = 0.0;
+#pragma unroll
+    for (int w = 0; w < kPotG / 64; ++w) r += she[w];
+    epart[blockIdx.x] = r;
+  }
 }
 
 // LDA on the grid (POTENTIAL_XC, src/paw_potential.f90:1397-1401, and DFT,
 // src/paw_dft.f90:780-965, 2137-2195, 2824-2910): exc(r) partial sums, and
-// c(r) <- vxc(r) for the RTOG that follows
+// v(r) <- vxc(r) in place for the RTOG that follows
 __device__ inline void lda_point(double rho, double &exc, double &vxc) {
   const double rhot = fmax(rho, 1.0e-8);
   const double val = fmax(rhot, kRhoTMin);
@@ -256,14 +326,14 @@ __device__ inline void lda_point(double rho, double &exc, double &vxc) {
   }
 }
 
-__global__ void __launch_bounds__(kPotThreads) k_xc(int n, double2 *__restrict__ c, double *__restrict__ xpart) {
+__global__ void __launch_bounds__(kPotThreads) k_xc(int n, double *__restrict__ v, double *__restrict__ xpart) {
   __shared__ double sh[kPotThreads / 64];
   const int i = blockIdx.x * kPotThreads + threadIdx.x;
   double e = 0.0;
   if (i < n) {
     double vx;
-    lda_point(c[i].x, e, vx);
-    c[i] = make_double2(vx, 0.0);
+    lda_point(v[i], e, vx);
+    v[i] = vx;
   }
   const double s = block_sum(e, sh);
   if (threadIdx.x == 0) xpart[blockIdx.x] = s;
@@ -354,22 +424,22 @@ __global__ void k_grad_g(int ngl, const double *__restrict__ gvec, const double2
   }
 }
 
-// PBE on the grid: c = rho + core (real part), d[k] = d rho/dx_k; c <- vt,
+// PBE on the grid: c = rho + core, d[k] = d rho/dx_k (real arrays); c <- vt,
 // d[k] <- 2 de/d|grad rho|^2 d rho/dx_k (POTENTIAL_XC :1405-1470); exc partials
-__global__ void __launch_bounds__(kPotThreads) k_xc_gga(int n, double2 *__restrict__ c, double2 *__restrict__ d,
+__global__ void __launch_bounds__(kPotThreads) k_xc_gga(int n, double *__restrict__ c, double *__restrict__ d,
                                                         double *__restrict__ xpart) {
   __shared__ double sh[kPotThreads / 64];
   const int i = blockIdx.x * kPotThreads + threadIdx.x;
   double e = 0.0;
   if (i < n) {
-    const double gx = d[i].x, gy = d[(size_t)n + i].x, gz = d[2 * (size_t)n + i].x;
+    const double gx = d[i], gy = d[(size_t)n + i], gz = d[2 * (size_t)n + i];
     double vt, gv;
-    pbe_point(c[i].x, gx * gx + gy * gy + gz * gz, e, vt, gv);
-    c[i] = make_double2(vt, 0.0);
+    pbe_point(c[i], gx * gx + gy * gy + gz * gz, e, vt, gv);
+    c[i] = vt;
     const double s = 2.0 * gv;
-    d[i] = make_double2(s * gx, 0.0);
-    d[(size_t)n + i] = make_double2(s * gy, 0.0);
-    d[2 * (size_t)n + i] = make_double2(s * gz, 0.0);
+    d[i] = s * gx;
+    d[(size_t)n + i] = s * gy;
+    d[2 * (size_t)n + i] = s * gz;
   }
   const double s = block_sum(e, sh);
   if (threadIdx.x == 0) xpart[blockIdx.x] = s;
@@ -391,91 +461,135 @@ __global__ void k_div_g(int ngl, const double *__restrict__ gvec, const double2 
   v[ig] = o;
 }
 
-__global__ void k_zero_d(int n, double *x) {
-  if ((int)threadIdx.x < n) x[threadIdx.x] = 0.0;
-}
-
-__global__ void k_copy1(const double *a, double *b) {
-  if (threadIdx.x == 0) b[0] = a[0];
-}
-
-__global__ void k_add_c(int n, const double2 *__restrict__ a, double2 *__restrict__ b) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = make_double2(a[i].x + b[i].x, a[i].y + b[i].y);
-}
-
-// Per (atom, G block): VQLM(LM) and the Hartree/VBAR force terms
+// Per (atom group, G block): VQLM(LM) and the Hartree/VBAR force terms
 // (src/paw_potential.f90:1255-1290) and the pseudo-core force
 // (POTENTIAL_FPSCORE, :897-975), as block partial sums
 // apart[(a * nblk + block) * (lmrxx + 3) + {0..lmrxx-1: VQLM, lmrxx..+2: force}]
-__global__ void __launch_bounds__(kPotThreads) k_pot_atoms(PotGeo g, const double2 *__restrict__ rhog,
+//
+// The terms of G and -G are equal (conjugate coefficients, G odd), so a pair
+// is evaluated once and counts twice.  A thread keeps the sums of AG atoms
+// over ngi pairs in registers: a pair's coefficients, harmonics and tables
+// are read once per AG atoms, its phase factors come from the atoms' tables
+// in LDS, and the workgroup reduction runs once per (atom, ngi x 256 pairs)
+// instead of once per (atom, 256 G) with a sincos each.  365 -> 37 us at Si64.
+template <int LM> constexpr int pot_atoms() { return LM == 1 ? 4 : (LM == 4 ? 2 : 1); }
+template <int LM>
+__global__ void __launch_bounds__(kPotThreads) k_pot_atoms(PotGeo g, int ngi, const double2 *__restrict__ rhog,
                                                            const double2 *__restrict__ vg,
                                                            const double2 *__restrict__ vtot,
                                                            const double *__restrict__ scal,
                                                            double *__restrict__ apart) {
-  __shared__ double sh[kLmrxxMax + 3][kPotThreads / 64];
-  const int ig = blockIdx.x * kPotThreads + threadIdx.x;
-  const int a = blockIdx.y;
-  const int nval = g.lmrxx + 3;
-  double val[kLmrxxMax + 3];
-  for (int k = 0; k < nval; ++k) val[k] = 0.0;
-  if (ig < g.ngl) {
-    const int s = g.isp[a];
-    const int n = g.lmrx[s];
-    const double2 ea = eigr(g, a, ig);
+  constexpr int AG = pot_atoms<LM>(), NV = LM + 3;
+  extern __shared__ double2 sph[];         // AG atoms x 3 x nph
+  __shared__ double sh[AG * NV][kPotThreads / 64];
+  const int a0 = blockIdx.y * AG, na = min(AG, g.nat - a0);
+  for (int i = threadIdx.x; i < na * 3 * g.nph; i += kPotThreads) sph[i] = g.phase[(size_t)a0 * 3 * g.nph + i];
+  __syncthreads();
+  const int nh = g.full ? g.ngl : g.nh, nm = g.nph / 2;
+  double acc[AG][NV];
+#pragma unroll
+  for (int k = 0; k < AG; ++k)
+#pragma unroll
+    for (int v = 0; v < NV; ++v) acc[k][v] = 0.0;
+  for (int i = 0; i < ngi; ++i) {
+    const int h = (blockIdx.x * ngi + i) * kPotThreads + threadIdx.x;
+    if (h >= nh) break;
+    const int2 gp = pot_pair(g, h);
+    const int ig = gp.x;
+    const double wt = gp.x == gp.y ? 1.0 : 2.0;
+    const int3 n = make_int3(g.igvec[3 * ig] + nm, g.igvec[3 * ig + 1] + nm, g.igvec[3 * ig + 2] + nm);
+    const double gx = wt * g.gvec[3 * ig], gy = wt * g.gvec[3 * ig + 1], gz = wt * g.gvec[3 * ig + 2];
     const double2 rg = rhog[ig], v = vg[ig], vt = vtot[ig];
     const double2 r2b = {rg.x + (ig == g.ngamma ? scal[0] : 0.0), rg.y};
-    const double g0 = tab(g, 2, s, ig), v0 = tab(g, 3, s, ig);
-    // AVAL = (G0 conj(VG) + V0 conj(RHO2)) EIGR
-    const double2 b = {g0 * v.x + v0 * r2b.x, -(g0 * v.y + v0 * r2b.y)};
-    const double2 aval = {b.x * ea.x - b.y * ea.y, b.x * ea.y + b.y * ea.x};
-    double y[kLmrxxMax];
-    solid_ylm(g.lmrxx, g.gvec[3 * ig], g.gvec[3 * ig + 1], g.gvec[3 * ig + 2], y);
-    // VQLM(LM) += Re(CFAC(LM) YLMOFG(LM,G) AVAL)
-    for (int lm = 0; lm < n; ++lm) {
-      const double2 c = cfac_l(l_of(lm));
-      val[lm] = c.x * y[lm] * aval.x - c.y * y[lm] * aval.y;
+    double y[LM];
+    solid_ylm(LM, g.gvec[3 * ig], g.gvec[3 * ig + 1], g.gvec[3 * ig + 2], y);
+    int sp = -1;
+    double g0 = 0.0, v0 = 0.0, vb = 0.0, pc = 0.0;
+#pragma unroll
+    for (int k = 0; k < AG; ++k) {
+      if (k >= na) break;
+      const int a = a0 + k, s = g.isp[a];
+      if (s != sp) {
+        pc = tab(g, 0, s, ig);
+        vb = tab(g, 1, s, ig) * kY0;
+        g0 = tab(g, 2, s, ig);
+        v0 = tab(g, 3, s, ig);
+        sp = s;
+      }
+      const int nl = g.lmrx[s];
+      const double2 ea = pot_eigr(sph + (size_t)k * 3 * g.nph, g.nph, n);
+      // AVAL = (G0 conj(VG) + V0 conj(RHO2)) EIGR
+      const double2 b = {g0 * v.x + v0 * r2b.x, -(g0 * v.y + v0 * r2b.y)};
+      const double2 aval = {b.x * ea.x - b.y * ea.y, b.x * ea.y + b.y * ea.x};
+      // VQLM(LM) += Re(CFAC(LM) YLMOFG(LM,G) AVAL)
+#pragma unroll
+      for (int lm = 0; lm < LM; ++lm) {
+        const double2 c = cfac_l(l_of(lm));
+        if (lm < nl) acc[k][lm] += wt * (c.x * y[lm] * aval.x - c.y * y[lm] * aval.y);
+      }
+      // CSUM = sum_LM QLM(LM) CFAC(LM) YLMOFG(LM,G)
+      const double2 csum = comp_factor<LM>(g.qlm + (size_t)a * g.lmrxx, nl, y);
+      // CVAL = VBARG Y0 EIGR conj(RHO)
+      const double cval_im = vb * (ea.y * rg.x - ea.x * rg.y);
+      const double sv = cval_im + csum.x * aval.y + csum.y * aval.x;
+      // FPSCORE: -Im(conj(VTOT) PSCORG EIGR) Y0
+      const double sc = -pc * (vt.x * ea.y - vt.y * ea.x);
+      const double t = -sv + kY0 * sc;
+      acc[k][LM] += gx * t;
+      acc[k][LM + 1] += gy * t;
+      acc[k][LM + 2] += gz * t;
     }
-    // CSUM = sum_LM QLM(LM) CFAC(LM) YLMOFG(LM,G)
-    const double2 csum = comp_factor(g, a, n, y);
-    // CVAL = VBARG Y0 EIGR conj(RHO)
-    const double vb = tab(g, 1, s, ig) * kY0;
-    const double cval_im = vb * (ea.y * rg.x - ea.x * rg.y);
-    const double sv = cval_im + csum.x * aval.y + csum.y * aval.x;
-    // FPSCORE: -Im(conj(VTOT) PSCORG EIGR) Y0
-    const double pc = tab(g, 0, s, ig);
-    const double sc = -pc * (vt.x * ea.y - vt.y * ea.x);
-    const double t = -sv + kY0 * sc;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) val[g.lmrxx + k] = g.gvec[3 * ig + k] * t;
   }
-  // all values of the block at once: wave sums, then the waves in order
+  // all values of the block: rows of 16 lanes, the rows, then the waves in order
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int k = 0; k < nval; ++k) {
-    double v = val[k];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    if (lane == 0) sh[k][wv] = v;
-  }
+  for (int k = 0; k < AG; ++k)
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      double v = row16_sum(acc[k][q]);
+      v += __shfl_xor(v, 16);
+      v += __shfl_xor(v, 32);
+      if (lane == 0) sh[k * NV + q][wv] = v;
+    }
   __syncthreads();
-  if ((int)threadIdx.x < nval) {
+  const int o = threadIdx.x;
+  if (o < na * NV) {
     double r = 0.0;
-    for (int w = 0; w < kPotThreads / 64; ++w) r += sh[threadIdx.x][w];
-    apart[((size_t)a * gridDim.x + blockIdx.x) * nval + threadIdx.x] = r;
+    for (int w = 0; w < kPotThreads / 64; ++w) r += sh[o][w];
+    apart[((size_t)(a0 + o / NV) * gridDim.x + blockIdx.x) * NV + o % NV] = r;
   }
 }
 
-// Ordered reduction: output o sums in[o * stride * n + k * stride] over
-// k < n (one workgroup per output, fixed assignment of terms to threads)
-__global__ void __launch_bounds__(kPotThreads) k_sum_out(int n, int stride, const double *__restrict__ in,
-                                                         double scale, double *__restrict__ out) {
+// Ordered reductions into res, one workgroup per output: the NAT (LMRXX + 3)
+// per-atom values over nba blocks, then EHARTREE (with RHOB beside it) and EXC
+__global__ void __launch_bounds__(kPotThreads) k_pot_finish(int nval, int nat, int nba, int nbe, int nbx,
+                                                            const double *__restrict__ apart,
+                                                            const double *__restrict__ epart,
+                                                            const double *__restrict__ xpart,
+                                                            const double *__restrict__ scal, double vol, double dvol,
+                                                            double *__restrict__ res) {
   __shared__ double sh[kPotThreads / 64];
-  const int o = blockIdx.x;
-  const int c = o % stride, row = o / stride;
+  const int o = blockIdx.x, na = nval * nat;
+  const double *in = o < na ? apart + (size_t)(o / nval) * nba * nval + o % nval : (o == na ? epart : xpart);
+  const int n = o < na ? nba : (o == na ? nbe : nbx), stride = o < na ? nval : 1;
   double s = 0.0;
-  for (int k = threadIdx.x; k < n; k += kPotThreads) s += in[((size_t)row * n + k) * stride + c];
+  for (int k = threadIdx.x; k < n; k += kPotThreads) s += in[(size_t)k * stride];
   const double r = block_sum(s, sh);
-  if (threadIdx.x == 0) out[o] = scale * r;
+  if (threadIdx.x != 0) return;
+  res[o] = (o == na + 1 ? dvol : vol) * r;
+  if (o == na) res[na + 2] = scal[0];
+}
+
+// f(IC<LM>) with the full shell LM = lmrxx (1, 4, 9, 16 or 25)
+template <class F>
+void with_lm(int lmrxx, F &&f) {
+  switch (lmrxx) {
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 9: f(std::integral_constant<int, 9>{}); break;
+    case 16: f(std::integral_constant<int, 16>{}); break;
+    default: f(std::integral_constant<int, 25>{}); break;
+  }
 }
 
 }  // namespace
@@ -497,12 +611,24 @@ int vofrho_enqueue(pw_plan *p, int nat, int lmrxx, const int *isp, const double 
     if (p->pot_lmrx[s] > lmrxx) return pw_fail(PW_ERR_ARG, "POTENTIAL$VOFRHO: LMRX of a species exceeds LMRXX");
   PW_TRY(plan_device(p));
   const int nbg = (ngl + kPotThreads - 1) / kPotThreads;
+  // per-atom sums: G pairs per thread so that the grid holds about four
+  // workgroups per CU, at most 16 (the reduction is then a small part)
+  const int full = p->pot_sym ? 0 : 1, nh = full ? ngl : p->nh;
+  const int nbe = (nh + kPotG - 1) / kPotG;
+  int ag = 1;
+  with_lm(lmrxx, [&](auto lm) { ag = pot_atoms<decltype(lm)::value>(); });
+  const int ngrp = std::max(1, (nat + ag - 1) / ag);
+  const int ngi = (int)std::min<long>(16, std::max<long>(1, (long)nh * ngrp / ((long)kPotThreads * 1024)));
+  const int nba = (nh + kPotThreads * ngi - 1) / (kPotThreads * ngi);
+  const int nph = 2 * std::max(p->nmax[0], std::max(p->nmax[1], p->nmax[2])) + 1;
+  // atoms of a k_pot_g chunk: at most 48 KiB of phase tables in LDS
+  const int ac = std::max(1, std::min(16, (int)(49152 / ((size_t)3 * nph * sizeof(double2)))));
   const int nbr = (nrl + kPotThreads - 1) / kPotThreads;
   const int nval = lmrxx + 3;
   // work: grid (complex), rhog, vg, vh, vtot (sphere), partials, per-atom data
   const bool gga = p->pot_xc == 10;
-  const size_t need = (size_t)nrl * 16 + 4 * (size_t)ngl * 16 + (gga ? 3 * ((size_t)nrl + ngl) * 16 : 0) +
-                      ((size_t)nbg * (nval * (size_t)nat + 1) + nbr + 8) * 8 +
+  const size_t need = (size_t)nrl * 8 + 4 * (size_t)ngl * 16 + (gga ? 3 * ((size_t)nrl * 8 + (size_t)ngl * 16) : 0) +
+                      ((size_t)nba * nval * (size_t)nat + nbe + nbr + 8) * 8 + (size_t)nat * 3 * nph * 16 +
                       ((size_t)nat * nval + 3) * 8 + (size_t)nat * (8 + 3 * 8 + lmrxx * 8) + (size_t)nsp * 8 + 4096;
   if (need > p->pot_bytes) {
     if (p->d_pot) PW_HIP(hipFree(p->d_pot));
@@ -523,14 +649,15 @@ int vofrho_enqueue(pw_plan *p, int nat, int lmrxx, const int *isp, const double 
     p->h_pot_bytes = hneed;
   }
   char *w = (char *)p->d_pot;
-  double2 *grid = (double2 *)w; w += (size_t)nrl * 16;
   double2 *rhog = (double2 *)w; w += (size_t)ngl * 16;
   double2 *vg = (double2 *)w; w += (size_t)ngl * 16;
   double2 *vh = (double2 *)w; w += (size_t)ngl * 16;
   double2 *vtot = (double2 *)w; w += (size_t)ngl * 16;
-  double *epart = (double *)w; w += (size_t)nbg * 8;
+  double2 *phase = (double2 *)w; w += (size_t)nat * 3 * nph * 16;
+  double *grid = (double *)w; w += (size_t)nrl * 8;
+  double *epart = (double *)w; w += (size_t)nbe * 8;
   double *xpart = (double *)w; w += (size_t)nbr * 8;
-  double *apart = (double *)w; w += (size_t)nbg * nval * nat * 8;
+  double *apart = (double *)w; w += (size_t)nba * nval * nat * 8;
   double *scal = (double *)w; w += 8 * 8;
   double *res = (double *)w; w += hres * 8;   // per atom VQLM(LMRXX), force(3); EHARTREE, EXC, RHOB
   int *d_isp = (int *)w; w += (size_t)nat * 8;
@@ -539,8 +666,8 @@ int vofrho_enqueue(pw_plan *p, int nat, int lmrxx, const int *isp, const double 
   double *d_qlm = (double *)w; w += (size_t)nat * lmrxx * 8;
   w = (char *)p->d_pot + ((size_t)(w - (char *)p->d_pot) + 255) / 256 * 256;   // inside the 4096-byte slack
   // the gradient of rho + core on the grid and its Fourier coefficients (type 10)
-  double2 *grid3 = gga ? (double2 *)w : nullptr;
-  double2 *fg3 = gga ? grid3 + 3 * (size_t)nrl : nullptr;
+  double2 *fg3 = gga ? (double2 *)w : nullptr;
+  double *grid3 = gga ? (double *)(fg3 + 3 * (size_t)ngl) : nullptr;
   // per-atom data: 0-based species, b_k . R_a, QLM (staged in pinned memory)
   double *hbase = p->h_pot + hres;
   int *hisp = (int *)hbase;
@@ -579,41 +706,52 @@ int vofrho_enqueue(pw_plan *p, int nat, int lmrxx, const int *isp, const double 
   g.g2 = p->d_g2;
   g.tabs = p->d_pot_tabs;
   g.isp = d_isp;
-  g.gr = d_gr;
+  g.hg = p->d_hg;
+  g.nh = p->nh;
+  g.full = full;
+  g.phase = phase;
+  g.nph = nph;
   g.qlm = d_qlm;
   g.vol = p->vol;
   // rho(G) of the valence density
-  k_real_to_c<<<nbr, kPotThreads, 0, st>>>(nrl, rho, grid);
-  PW_TRY(fft_rtog_full(p, 1, rhog, grid, PW_PREC_FP64, st));
+  PW_TRY(fft_rtog_full(p, 1, rhog, rho, PW_PREC_FP64, st, true));
   // core, compensation, Hartree
-  k_zero_d<<<1, 64, 0, st>>>(8, scal);
-  k_pot_g<<<nbg, kPotThreads, 0, st>>>(g, rhog, vg, vh, epart, scal);
+  if (nat > 0) k_pot_phase<<<(nat * 3 * nph + 255) / 256, 256, 0, st>>>(nat, nph, d_gr, phase);
+  with_lm(lmrxx, [&](auto lm) {
+    k_pot_g<decltype(lm)::value><<<nbe, kPotG * kPotS, (size_t)ac * 3 * nph * sizeof(double2), st>>>(g, ac, rhog, vg, vh,
+                                                                                                     epart, scal);
+  });
   // density + core on the grid, XC, back to G
-  PW_TRY(fft_gtor_full(p, 1, rhog, grid, PW_PREC_FP64, st));
+  PW_TRY(fft_gtor_full(p, 1, rhog, grid, PW_PREC_FP64, st, true));
   if (gga) {
     // POTENTIAL_GRADIENT('RHO'), DFT type 10, POTENTIAL_GRADIENT('POT')
     k_grad_g<<<nbg, kPotThreads, 0, st>>>(ngl, p->d_gvec, rhog, fg3);
-    PW_TRY(fft_gtor_full(p, 3, fg3, grid3, PW_PREC_FP64, st));
+    PW_TRY(fft_gtor_full(p, 3, fg3, grid3, PW_PREC_FP64, st, true));
     k_xc_gga<<<nbr, kPotThreads, 0, st>>>(nrl, grid, grid3, xpart);
-    PW_TRY(fft_rtog_full(p, 1, vtot, grid, PW_PREC_FP64, st));
-    PW_TRY(fft_rtog_full(p, 3, fg3, grid3, PW_PREC_FP64, st));
+    PW_TRY(fft_rtog_full(p, 1, vtot, grid, PW_PREC_FP64, st, true, vh));
+    PW_TRY(fft_rtog_full(p, 3, fg3, grid3, PW_PREC_FP64, st, true));
     k_div_g<<<nbg, kPotThreads, 0, st>>>(ngl, p->d_gvec, fg3, vtot);
   } else {
     k_xc<<<nbr, kPotThreads, 0, st>>>(nrl, grid, xpart);
-    PW_TRY(fft_rtog_full(p, 1, vtot, grid, PW_PREC_FP64, st));
+    PW_TRY(fft_rtog_full(p, 1, vtot, grid, PW_PREC_FP64, st, true, vh));
   }
-  k_add_c<<<nbg, kPotThreads, 0, st>>>(ngl, vh, vtot);
-  // per-atom sums
+  // per-atom sums, then all ordered reductions
   if (nat > 0) {
-    k_pot_atoms<<<dim3(nbg, nat), kPotThreads, 0, st>>>(g, rhog, vg, vtot, scal, apart);
-    k_sum_out<<<nval * nat, kPotThreads, 0, st>>>(nbg, nval, apart, p->vol, res);
+    hipError_t err = hipSuccess;
+    with_lm(lmrxx, [&](auto lm) {
+      constexpr int LM = decltype(lm)::value;
+      const size_t lds = (size_t)pot_atoms<LM>() * 3 * nph * sizeof(double2);
+      if (lds > 65536)   // more than 341 G components along an axis
+        err = hipFuncSetAttribute((const void *)k_pot_atoms<LM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (err == hipSuccess)
+        k_pot_atoms<LM><<<dim3(nba, ngrp), kPotThreads, lds, st>>>(g, ngi, rhog, vg, vtot, scal, apart);
+    });
+    PW_HIP(err);
   }
-  k_sum_out<<<1, kPotThreads, 0, st>>>(nbg, 1, epart, p->vol, res + (size_t)nval * nat);
-  k_sum_out<<<1, kPotThreads, 0, st>>>(nbr, 1, xpart, p->vol / (double)nrl, res + (size_t)nval * nat + 1);
-  k_copy1<<<1, 64, 0, st>>>(scal, res + (size_t)nval * nat + 2);
+  k_pot_finish<<<nval * nat + 2, kPotThreads, 0, st>>>(nval, nat, nba, nbe, nbr, apart, epart, xpart, scal, p->vol,
+                                                       p->vol / (double)nrl, res);
   // v(r)
-  PW_TRY(fft_gtor_full(p, 1, vtot, grid, PW_PREC_FP64, st));
-  k_c_to_real<<<nbr, kPotThreads, 0, st>>>(nrl, grid, vofr);
+  PW_TRY(fft_gtor_full(p, 1, vtot, vofr, PW_PREC_FP64, st, true));
   PW_HIP(hipGetLastError());
   PW_HIP(hipMemcpyAsync(p->h_pot, res, hres * sizeof(double), hipMemcpyDeviceToHost, st));
   p->pot_nat = nat;
@@ -660,6 +798,18 @@ extern "C" int pw_potential_tables(pw_plan *p, int nsp, const int *lmrx, const d
   PW_HIP(hipMemcpy(p->d_pot_tabs, tabs, n * sizeof(double), hipMemcpyHostToDevice));
   p->pot_nsp = nsp;
   p->pot_lmrx = l;
+  // radial tables have T(G) = T(-G) (to the rounding of |G|)
+  p->pot_sym = true;
+  for (size_t k = 0; k < 4 * (size_t)nsp && p->pot_sym; ++k) {
+    const double *row = tabs + k * p->ngl;
+    for (const int2 &h : p->hg) {
+      const double a = row[h.x], b = row[h.y];
+      if (!(std::fabs(a - b) <= 1.0e-15 * std::max(std::fabs(a), std::fabs(b)))) {
+        p->pot_sym = false;
+        break;
+      }
+    }
+  }
   return PW_OK;
 }
 

@@ -25,7 +25,8 @@
 // diagonalised.  The
 // outer loop runs on the device: the convergence test sets a flag that makes
 // every later kernel of the batch return at once, so the host waits only
-// once per batch of iterations (batch = the previous call's count).
+// once per batch of iterations (batch = the previous call's count).  Sets
+// whose matrices fit in LDS are solved by one workgroup in one launch.
 #include <algorithm>
 #include <cmath>
 
@@ -923,6 +924,293 @@ __global__ void k_eig_scale(int n, const double *e, double *X, const OrthoState 
   X[idx] /= e[i] + e[j];
 }
 
+// ---------------------------------------------------------------------------
+// The whole solve in one workgroup, for the small sets whose matrices fit in
+// LDS: the preparation (Newton-Schulz, the P_k, the acceptance test) and all
+// outer iterations.  As a chain the solve is bound by launch latency: 45
+// dependent launches for 2 us of matrix instructions per iteration, most of a
+// CP step of Si8 (20 bands, 7 iterations).  One launch: 218 us in kernels (430
+// with the gaps) -> 44 us, the step 490 -> 325 us.
+//
+// Eight waves; a product's 16 x 16 tiles go one per wave, operands from LDS,
+// all fragments loaded before the first MFMA.  The term P_k G P_k of row block
+// I stays in one wave: G P_k(:,I) comes out of the MFMA in the layout in which
+// its transpose P_k(I,:) G is the A operand of the second product (G and P_k
+// symmetric), so nothing is exchanged between the two, and both read the same
+// fragments of P_k.  kSmallSub waves share the terms of a row block; their
+// sums are added in order.  The matrices have a compile-time row
+// length of 16 NT + 1 and their rows and columns n .. 4 ceil(n/4) - 1 are
+// zero: the products need no bounds (what a tile reads beyond that only
+// enters elements that are not written).
+// ---------------------------------------------------------------------------
+constexpr int kSmallThreads = 512, kSmallTiles = 2, kSmallSub = 4;
+constexpr int kSmallMats = 6;                   // LDS matrices beside the P_k
+// the pad keeps the rows up to 16 NT of the last matrix inside
+inline size_t small_lds(int n, int nterm) {
+  const int nt = (n + T16 - 1) / T16, ld = T16 * nt + 1, rows = (n + 3) & ~3;
+  return ((size_t)(kSmallMats + nterm) * rows * ld + (T16 * nt - rows) * ld + 64) * sizeof(double);
+}
+
+struct SmallArgs {
+  int n, nterm, nlev, nns, maxiter;
+  double c, q;                                  // Newton-Schulz start, Cayley shift
+  double tol, ptol_res, ptol_pow;
+  const double *chichi, *psipsi, *chipsi, *occ;
+  double *lam;                                  // in: the guess, out: the multipliers
+};
+
+// the tile (I, J) of A B (TA: A^T B)
+template <int NT, bool TA>
+__device__ inline dbl4 small_tile(const double *A, const double *B, int n, int I, int J) {
+  constexpr int ld = 16 * NT + 1;
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  double a[4 * NT], b[4 * NT];
+#pragma unroll
+  for (int s = 0; s < 4 * NT; ++s) {
+    const int k = 4 * s + lk, i = 16 * I + li;
+    a[s] = TA ? A[k * ld + i] : A[i * ld + k];
+    b[s] = B[k * ld + 16 * J + li];
+  }
+  dbl4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int s = 0; s < 4 * NT; ++s)
+    if (4 * s < n) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], acc, 0, 0, 0);
+  return acc;
+}
+// f(r, i, j) over the lane's elements of tile (I, J) inside the matrix
+template <class F>
+__device__ inline void small_each(int n, int I, int J, F &&f) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int i = 16 * I + lk + 4 * r, j = 16 * J + li;
+    if (i < n && j < n) f(r, i, j);
+  }
+}
+
+template <int NT>
+__global__ void __launch_bounds__(kSmallThreads) k_ortho_small(SmallArgs a, OrthoState *st) {
+  extern __shared__ double sm[];
+  constexpr int EL = (256 * NT * NT + kSmallThreads - 1) / kSmallThreads;   // elements per thread
+  constexpr int ld = 16 * NT + 1;
+  const int n = a.n, rows = (n + 3) & ~3, n2 = rows * ld;
+  double *red = sm;                             // 2 per wave
+  double *m0 = sm + 64, *m1 = m0 + n2, *m2 = m1 + n2, *m3 = m2 + n2, *m4 = m3 + n2, *m5 = m4 + n2, *P = m5 + n2;
+  const int t = threadIdx.x, wv = t >> 6, lane = t & 63, li = lane & 15, lk = lane >> 4;
+  const bool on = wv < NT * NT;
+  const int I = wv / NT, J = wv % NT;
+  auto finish = [&](int code, int iter) {
+    if (t != 0) return;
+    st->code = code;
+    st->iter = iter;
+    st->done = code >= 0 ? 1 : 0;
+  };
+  for (int e = t; e < (kSmallMats + a.nterm) * n2 + (16 * NT - rows) * ld; e += kSmallThreads) m0[e] = 0.0;
+  __syncthreads();
+  // preparation: B + qI in m0, X in m1/m2, T = (B + qI) X in m3
+  for (int e = t; e < n * n; e += kSmallThreads) {
+    const int i = e / n, j = e - i * n;
+    const double b = 0.5 * (a.chipsi[e] + a.chipsi[j * n + i]) + (i == j ? a.q : 0.0);
+    m0[i * ld + j] = b;
+    m1[i * ld + j] = (i == j ? 2.0 * a.c : 0.0) - a.c * a.c * b;
+  }
+  __syncthreads();
+  double *x = m1, *y = m2;
+  for (int k = 1; k < a.nns; ++k) {
+    if (on) {
+      const dbl4 v = small_tile<NT, false>(m0, x, n, I, J);
+      small_each(n, I, J, [&](int r, int i, int j) { m3[i * ld + j] = v[r]; });
+    }
+    __syncthreads();
+    if (on) {
+      const dbl4 v = small_tile<NT, false>(x, m3, n, I, J);
+      small_each(n, I, J, [&](int r, int i, int j) { y[i * ld + j] = 2.0 * x[i * ld + j] - v[r]; });
+    }
+    __syncthreads();
+    double *s = x;
+    x = y;
+    y = s;
+  }
+  // P_0 = M, A = I - 2qM in m4; level l doubles the P_k and squares A
+  double *ap = m4, *an = m5;
+  for (int e = t; e < n * n; e += kSmallThreads) {
+    const int i = e / n, j = e - i * n;
+    const double v = x[i * ld + j];
+    P[i * ld + j] = v;
+    ap[i * ld + j] = (i == j ? 1.0 : 0.0) - 2.0 * a.q * v;
+  }
+  __syncthreads();
+  for (int l = 0; l < a.nlev; ++l) {
+    const int half = 1 << l, nprod = half + (l + 1 < a.nlev ? 1 : 0);
+    for (int w = wv; w < nprod * NT * NT; w += kSmallThreads / 64) {
+      const int k = w / (NT * NT), tl = w - k * NT * NT, ti = tl / NT, tj = tl % NT;
+      double *dst = k < half ? P + (half + k) * n2 : an;
+      const dbl4 v = small_tile<NT, false>(ap, k < half ? P + k * n2 : ap, n, ti, tj);
+      small_each(n, ti, tj, [&](int r, int i, int j) { dst[i * ld + j] = v[r]; });
+    }
+    __syncthreads();
+    if (l + 1 < a.nlev) {
+      double *s = ap;
+      ap = an;
+      an = s;
+    }
+  }
+  {
+    // acceptance, as k_prep_part and the first k_series_sum: the residual of
+    // the last Newton-Schulz step and the row sums of |A^(2^(J-1))|
+    double r1 = 0.0, r2 = 0.0;
+    for (int e = t; e < n * n; e += kSmallThreads) {
+      const int i = e / n, j = e - i * n;
+      r1 = nanmax(r1, fabs(m3[i * ld + j] - (i == j ? 1.0 : 0.0)));
+    }
+    for (int i = t; i < n; i += kSmallThreads) {
+      double s = 0.0;
+      for (int j = 0; j < n; ++j) s += fabs(ap[i * ld + j]);
+      r2 = nanmax(r2, s);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      r1 = nanmax(r1, __shfl_xor(r1, o));
+      r2 = nanmax(r2, __shfl_xor(r2, o));
+    }
+    if (lane == 0) {
+      red[2 * wv] = r1;
+      red[2 * wv + 1] = r2;
+    }
+    __syncthreads();
+    for (int w = 0; w < kSmallThreads / 64; ++w) {
+      r1 = nanmax(r1, red[2 * w]);
+      r2 = nanmax(r2, red[2 * w + 1]);
+    }
+    if (!((double)n * r1 <= a.ptol_res && r2 <= a.ptol_pow)) {
+      finish(3, 0);
+      return;
+    }
+    __syncthreads();
+  }
+  // outer iterations: LAMBDA in m0, CHICHI in m5, HAUX in m1, T = LAMBDA^T
+  // HAUX in m2, GAMN in m3; the partial sums of the terms in m4, m1, m2, m3
+  double cp[4] = {0.0, 0.0, 0.0, 0.0}, pp[4] = {0.0, 0.0, 0.0, 0.0};
+  if (on)
+    small_each(n, I, J, [&](int r, int i, int j) {
+      cp[r] = 2.0 * a.chipsi[i * n + j];
+      pp[r] = a.psipsi[min(i, j) * n + max(i, j)] - (i == j ? 1.0 : 0.0);
+    });
+  double fa[EL], fb[EL];                        // the update's factors (src/paw_waves2.f90:1979-2005)
+  bool swap[EL];
+#pragma unroll
+  for (int u = 0; u < EL; ++u) {
+    const int e = t + kSmallThreads * u;
+    if (e >= n * n) continue;
+    const int i = e / n, j = e - i * n;
+    m0[i * ld + j] = a.lam[e];
+    m5[i * ld + j] = a.chichi[e];
+    const double oi = a.occ[i] + 1.0e-12, oj = a.occ[j] + 1.0e-12;
+    swap[u] = a.occ[i] < a.occ[j];
+    fa[u] = 2.0 * (swap[u] ? oj / (oj + oi) : oi / (oi + oj));
+    fb[u] = oi / oj;
+  }
+  __syncthreads();
+  const int rb = wv / kSmallSub, sub = wv % kSmallSub;
+  int code = -1, it = 1;
+  for (; it <= a.maxiter; ++it) {
+    if (on) {
+      const dbl4 v = small_tile<NT, false>(m5, m0, n, I, J);
+      small_each(n, I, J, [&](int r, int i, int j) { m1[i * ld + j] = v[r] + cp[r]; });
+    }
+    __syncthreads();
+    if (on) {
+      const dbl4 v = small_tile<NT, true>(m0, m1, n, I, J);
+      small_each(n, I, J, [&](int r, int i, int j) { m2[i * ld + j] = v[r]; });
+    }
+    __syncthreads();
+    // GAMN and the convergence test (src/paw_waves2.f90:1960-1975): NaN, any
+    // element at or above the bound, any far above it
+    bool isnan = false, above = false, huge = false;
+    if (on)
+      small_each(n, I, J, [&](int r, int i, int j) {
+        const double g = 0.5 * (m2[i * ld + j] + m2[j * ld + i]) + pp[r];
+        m3[i * ld + j] = g;
+        isnan |= g != g;
+        above |= !(fabs(g) < a.tol);
+        huge |= fabs(g) > 1.0e200;
+      });
+    int flags = (__any(isnan) ? 1 : 0) | (__any(above) ? 2 : 0) | (__any(huge) ? 4 : 0);
+    if (lane == 0) reinterpret_cast<int *>(red)[wv] = flags;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kSmallThreads / 64; ++w) flags |= reinterpret_cast<const int *>(red)[w];
+    if (flags != 2) {
+      code = (flags & 1) ? 1 : ((flags & 2) ? 2 : 0);
+      break;
+    }
+    // sum_k P_k G P_k: wave (row block, subset of the terms)
+    dbl4 out[NT];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) out[q] = dbl4{0.0, 0.0, 0.0, 0.0};
+    if (rb < NT) {
+      for (int k = sub; k < a.nterm; k += kSmallSub) {
+        const double *Pk = P + k * n2;
+        double f[NT][4 * NT];                   // P_k(4 s + lk, 16 q + li)
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+#pragma unroll
+          for (int s = 0; s < 4 * NT; ++s) f[q][s] = Pk[(4 * s + lk) * ld + 16 * q + li];
+        dbl4 g[NT];                             // (G P_k)(tile u, rb) = (P_k G)(rb, tile u)^T
+#pragma unroll
+        for (int u = 0; u < NT; ++u) g[u] = dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < 4 * NT; ++s) {
+          if (4 * s >= n) break;
+          double b = f[0][s];
+#pragma unroll
+          for (int q = 1; q < NT; ++q) b = rb == q ? f[q][s] : b;
+#pragma unroll
+          for (int u = 0; u < NT; ++u)
+            g[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(m3[(16 * u + li) * ld + 4 * s + lk], b, g[u], 0, 0, 0);
+        }
+#pragma unroll
+        for (int s = 0; s < 4 * NT; ++s) {
+          if (4 * s >= n) break;
+#pragma unroll
+          for (int q = 0; q < NT; ++q)
+            out[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(g[s / 4][s % 4], f[q][s], out[q], 0, 0, 0);
+        }
+      }
+    }
+    auto put = [&](double *dst) {
+#pragma unroll
+      for (int q = 0; q < NT; ++q)
+        small_each(n, rb, q, [&](int r, int i, int j) { dst[i * ld + j] = out[q][r]; });
+    };
+    if (rb < NT && sub < kSmallSub - 1) put(sub == 0 ? m4 : (sub == 1 ? m1 : m2));
+    __syncthreads();
+    if (rb < NT && sub == kSmallSub - 1) put(m3);
+    __syncthreads();
+    double nl[EL];
+#pragma unroll
+    for (int u = 0; u < EL; ++u) {
+      const int e = t + kSmallThreads * u;
+      if (e >= n * n) continue;
+      const int i = e / n, j = e - i * n;
+      const int o = swap[u] ? j * ld + i : i * ld + j;
+      const double c = 2.0 * a.q * (((m4[o] + m1[o]) + m2[o]) + m3[o]);
+      const double v = m0[o] - fa[u] * c;
+      nl[u] = swap[u] ? v * fb[u] : v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < EL; ++u) {
+      const int e = t + kSmallThreads * u;
+      if (e < n * n) m0[e / n * ld + e % n] = nl[u];
+    }
+    __syncthreads();
+  }
+  finish(code, it);                             // code -1: not converged in maxiter iterations
+  if (code == 0)
+    for (int e = t; e < n * n; e += kSmallThreads) a.lam[e] = m0[e / n * ld + e % n];
+}
+
 struct OrthoWork {
   double *bs, *m0, *m1, *gam, *x0, *x1, *t1, *t2, *lam2, *occ, *red, *bounds;
   double *apow[kMaxLevels];
@@ -951,7 +1239,8 @@ int ortho_work(pw_waveset *ws, OrthoWork &w) {
   static std::once_flag lds_once;
   static hipError_t lds_err = hipSuccess;
   std::call_once(lds_once, [] {
-    const void *fns[] = {(const void *)k_panel_batch, (const void *)k_series_panel};
+    const void *fns[] = {(const void *)k_panel_batch, (const void *)k_series_panel, (const void *)k_ortho_small<1>,
+                         (const void *)k_ortho_small<2>};
     for (const void *f : fns) {
       hipFuncAttributes fa{};
       hipError_t e = hipFuncGetAttributes(&fa, f);
@@ -1225,6 +1514,18 @@ int enqueue_iters_eig(pw_waveset *ws, const OrthoWork &w, double *const lbuf[2],
   return PW_OK;
 }
 
+// the reference's stop conditions (src/paw_waves2.f90:1935-1945, 1960-1975)
+int ortho_status(const OrthoState &hs) {
+  if (hs.code == 1) return pw_fail(PW_ERR_NOCONV, "WAVES_ORTHO_X: NaN in overlap");
+  if (hs.code == 2)
+    return pw_fail(PW_ERR_NOCONV, "WAVES_ORTHO_X: iteration loop for orthogonalization is about to diverge");
+  if (!hs.done)
+    return pw_fail(PW_ERR_NOCONV,
+                   "WAVES_ORTHO_X: loop for orthogonalization is not converged (specify SAFEORTHO=F, "
+                   "reduce the cutoff or the time step)");
+  return PW_OK;
+}
+
 // WAVES_ORTHO_X with S^-1 from the eigenvectors of B (the reference's form),
 // for a B that is not positive definite (inside the Lanczos bounds or
 // rejected by the series' acceptance test)
@@ -1250,13 +1551,7 @@ int ortho_x_eig(pw_waveset *ws, const OrthoWork &w, double *const lbuf[2], doubl
     hs = *hp;
     if (hs.done) break;
   }
-  if (hs.code == 1) return pw_fail(PW_ERR_NOCONV, "WAVES_ORTHO_X: NaN in overlap");
-  if (hs.code == 2)
-    return pw_fail(PW_ERR_NOCONV, "WAVES_ORTHO_X: iteration loop for orthogonalization is about to diverge");
-  if (!hs.done)
-    return pw_fail(PW_ERR_NOCONV,
-                   "WAVES_ORTHO_X: loop for orthogonalization is not converged (specify SAFEORTHO=F, "
-                   "reduce the cutoff or the time step)");
+  PW_TRY(ortho_status(hs));
   if ((hs.iter - 1) & 1) {
     k_copy_d<<<nblk, 256, 0, ws->stream>>>(n2, w.lam2, d_lam);
     PW_HIP(hipGetLastError());
@@ -1288,8 +1583,13 @@ int ortho_x_device(pw_waveset *ws, double *d_lam, const double *d_chichi, const 
   if (ws->d_occ) w.occ = ws->d_occ;   // the waveset's occupations are on the device already
   else PW_HIP(hipMemcpyAsync(w.occ, ws->occ.data(), n * sizeof(double), hipMemcpyHostToDevice, ws->stream));
   if (!ws->h_ortho_state) PW_HIP(hipHostMalloc(&ws->h_ortho_state, sizeof(OrthoState), hipHostMallocDefault));
-  k_symm<<<nblk, 256, 0, ws->stream>>>(n, d_chipsi, w.bs);
-  PW_HIP(hipGetLastError());
+  bool have_bs = false;
+  auto symm = [&]() -> int {
+    if (!have_bs) k_symm<<<nblk, 256, 0, ws->stream>>>(n, d_chipsi, w.bs);
+    have_bs = true;
+    PW_HIP(hipGetLastError());
+    return PW_OK;
+  };
   ws->ortho_lanczos = 0;
   double *lbuf[2] = {d_lam, w.lam2};
   for (int attempt = 0; attempt < 2; ++attempt) {
@@ -1297,6 +1597,7 @@ int ortho_x_device(pw_waveset *ws, double *d_lam, const double *d_chichi, const 
     // until the acceptance test rejects them
     if (!ws->lz_valid || attempt > 0) {
       double lo0, hi0;
+      PW_TRY(symm());
       PW_TRY(lanczos_bounds(ws, w.bs, w.bounds, &lo0, &hi0));
       ws->lz_lo = lo0;
       ws->lz_hi = hi0;
@@ -1309,6 +1610,7 @@ int ortho_x_device(pw_waveset *ws, double *d_lam, const double *d_chichi, const 
     if (!(P.lo > 0.0) || !(P.hi >= P.lo)) {
       // sym(CHIPSI) is not positive definite: the eigenvector form of S^-1
       ws->lz_valid = false;
+      PW_TRY(symm());
       return ortho_x_eig(ws, w, lbuf, d_lam, d_chichi, d_psipsi, d_chipsi, iter);
     }
     P.lo *= 0.97;
@@ -1331,6 +1633,7 @@ int ortho_x_device(pw_waveset *ws, double *d_lam, const double *d_chichi, const 
     P.nser = series_fits(n) ? std::min(P.nlev, kSeriesMaxLevels) : 0;
     if (P.nlev > kMaxLevels) {
       ws->lz_valid = false;
+      PW_TRY(symm());
       return ortho_x_eig(ws, w, lbuf, d_lam, d_chichi, d_psipsi, d_chipsi, iter);
     }
     // Newton-Schulz for (B+qI)^-1: |I - (B+qI)X_k| = e0^(2^k); stop at 1e-17
@@ -1342,6 +1645,48 @@ int ortho_x_device(pw_waveset *ws, double *d_lam, const double *d_chichi, const 
     ws->ortho_levels = P.nlev;
     ws->ortho_series = 1 << P.nser;
     ws->ortho_ns = P.nns;
+    OrthoState hs{};
+    OrthoState *hp = static_cast<OrthoState *>(ws->h_ortho_state);
+    // one workgroup for the whole solve where its matrices fit in LDS and a
+    // product has at most four tiles: 32 bands with 8 terms of the series, 20
+    // with 16.  The launches of the chain take 218 us in kernels and 430 with
+    // the gaps for 20 bands, this one 44; for 32 bands 230 and 500 against 64.
+    // Wider sets do not fit with their 8 terms.
+    if (P.nser == P.nlev && (n + T16 - 1) / T16 <= kSmallTiles && small_lds(n, 1 << P.nser) <= kLdsMax) {
+      const int nts = (n + T16 - 1) / T16;
+      auto *const small = nts == 1 ? k_ortho_small<1> : k_ortho_small<2>;
+      SmallArgs s{};
+      s.n = n;
+      s.nterm = 1 << P.nser;
+      s.nlev = P.nlev;
+      s.nns = P.nns;
+      s.maxiter = kMaxIter;
+      s.c = 2.0 / (P.lo + P.hi + 2.0 * P.q);
+      s.q = P.q;
+      s.tol = 1.0e-8;
+      s.ptol_res = 3.16e-6;
+      s.ptol_pow = kAcceptPower;
+      s.chichi = d_chichi;
+      s.psipsi = d_psipsi;
+      s.chipsi = d_chipsi;
+      s.occ = w.occ;
+      s.lam = d_lam;
+      (*small)<<<1, kSmallThreads, small_lds(n, s.nterm), ws->stream>>>(s, w.st);
+      PW_HIP(hipGetLastError());
+      PW_HIP(hipMemcpyAsync(hp, w.st, sizeof(OrthoState), hipMemcpyDeviceToHost, ws->stream));
+      PW_HIP(hipStreamSynchronize(ws->stream));
+      hs = *hp;
+      if (hs.code == 3 && attempt == 0) continue;
+      if (hs.code == 3) {
+        ws->lz_valid = false;
+        PW_TRY(symm());
+        return ortho_x_eig(ws, w, lbuf, d_lam, d_chichi, d_psipsi, d_chipsi, iter);
+      }
+      PW_TRY(ortho_status(hs));
+      *iter = hs.iter;
+      return PW_OK;
+    }
+    PW_TRY(symm());
     const int batch = std::max(2, std::min(ws->ortho_iter > 0 ? ws->ortho_iter : 8, kMaxIter));
     // the preparation and the first batch of iterations are one captured graph,
     // replayed while the bounds, the batch and the buffers stay the same
@@ -1384,8 +1729,6 @@ int ortho_x_device(pw_waveset *ws, double *d_lam, const double *d_chichi, const 
       ws->ortho_graph_misses++;
     }
     int launched = batch;
-    OrthoState hs{};
-    OrthoState *hp = static_cast<OrthoState *>(ws->h_ortho_state);
     for (;;) {
       PW_HIP(hipMemcpyAsync(hp, w.st, sizeof(OrthoState), hipMemcpyDeviceToHost, ws->stream));
       PW_HIP(hipStreamSynchronize(ws->stream));
@@ -1403,13 +1746,7 @@ int ortho_x_device(pw_waveset *ws, double *d_lam, const double *d_chichi, const 
       ws->lz_valid = false;
       return ortho_x_eig(ws, w, lbuf, d_lam, d_chichi, d_psipsi, d_chipsi, iter);
     }
-    if (hs.code == 1) return pw_fail(PW_ERR_NOCONV, "WAVES_ORTHO_X: NaN in overlap");
-    if (hs.code == 2)
-      return pw_fail(PW_ERR_NOCONV, "WAVES_ORTHO_X: iteration loop for orthogonalization is about to diverge");
-    if (!hs.done)
-      return pw_fail(PW_ERR_NOCONV,
-                     "WAVES_ORTHO_X: loop for orthogonalization is not converged (specify SAFEORTHO=F, "
-                     "reduce the cutoff or the time step)");
+    PW_TRY(ortho_status(hs));
     // iteration hs.iter converged after hs.iter-1 updates
     if ((hs.iter - 1) & 1) {
       k_copy_d<<<nblk, 256, 0, ws->stream>>>(n2, w.lam2, d_lam);

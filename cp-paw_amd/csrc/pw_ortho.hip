@@ -180,8 +180,10 @@ __host__ __device__ inline int panel_ldr(int n) { return n + 1 + ((1 - n) % 32 +
 
 constexpr size_t kLdsMax = 160 * 1024;
 inline size_t panel_lds(int n) { return (size_t)T16 * panel_ldr(n) * sizeof(double); }
-// the series needs two staged panels per workgroup
-inline bool series_fits(int n) { return 2 * panel_lds(n) + 1024 <= kLdsMax; }   // + the static LDS of the panel
+// the terms of the series side by side where their launch is bound by latency
+// and occupancy, up to the sets whose two 16-row panels fit in LDS; wider ones
+// take the Smith levels, half the products
+inline bool series_fits(int n) { return 2 * panel_lds(n) + 1024 <= kLdsMax; }
 
 // Batched products with one shared left operand, by row panels:
 //   C_z = A B_z,  B_z = B + z sb, C_z = C + z sc,  z < nz,
@@ -350,7 +352,7 @@ __global__ void __launch_bounds__(64 * kGemmWaves) k_gemm_pair(PairArgs a, Ortho
 
 // The Smith sum written out as a series (the Cayley series of S^-1):
 //   S^-1(G) = 2q sum_{k<K} A^k M G M A^k = 2q sum_k P_k G P_k^T,  P_k = A^k M,
-// with the P_k formed once per call.  k_series_panel: workgroup (row panel
+// with the P_k formed once per call.  k_series_terms: workgroup (row panel
 // I, term k) forms R = P_k(I,:) G into LDS and then the row panel
 // part_k(I,:) = R P_k (P_k is symmetric), so each term is a chain of two
 // row-panel products inside one workgroup.  k_series_sum adds the K terms of each element in
@@ -372,103 +374,7 @@ struct SeriesArgs {
   const double *P;             // K stacked n x n row-major matrices P_k
   const double *G;             // GAMN
   double *part;                // K stacked terms P_k G P_k^T
-  const double *bmax;          // block maxima of |GAMN| (k_gemm_pair<kPairGamma>), or null
-  int nbmax;
-  double tol;
 };
-
-__global__ void __launch_bounds__(64 * kPanelWaves) k_series_panel(SeriesArgs a, const OrthoState *st) {
-  if (stopped(st)) return;
-  if (a.bmax) {
-    // the convergence test of this iteration, as k_series_sum applies it
-    // next: when GAMN is converged (or NaN, or diverging) the terms go unused
-    // and the loop ends there, so the products are skipped
-    __shared__ double wm[kPanelWaves];
-    __shared__ int wn[kPanelWaves];
-    double m = 0.0;
-    int nan = 0;
-    for (int b = threadIdx.x; b < a.nbmax; b += blockDim.x) {
-      const double x = a.bmax[b];
-      if (x != x) nan = 1;
-      else m = fmax(m, x);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      m = fmax(m, __shfl_xor(m, o));
-      nan |= __shfl_xor(nan, o);
-    }
-    if ((threadIdx.x & 63) == 0) {
-      wm[threadIdx.x >> 6] = m;
-      wn[threadIdx.x >> 6] = nan;
-    }
-    __syncthreads();
-    m = 0.0;
-    nan = 0;
-#pragma unroll
-    for (int w = 0; w < kPanelWaves; ++w) {
-      m = fmax(m, wm[w]);
-      nan |= wn[w];
-    }
-    if (nan || m < a.tol || m > 1.0e200) return;
-  }
-  extern __shared__ double sm[];   // sA, sR: 16 x ldr each
-  const int n = a.n, nt = (n + T16 - 1) / T16, ldr = panel_ldr(n);
-  double *sA = sm, *sR = sm + T16 * ldr;
-  const size_t n2 = (size_t)n * n;
-  const int I0 = blockIdx.x * T16;
-  const double *Pk = a.P + (size_t)blockIdx.y * n2;
-  double *out = a.part + (size_t)blockIdx.y * n2;
-  const int wv = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-  // the B operand of the first product (first tile, first chunk) goes out
-  // with the A panel; that of the second as soon as the first's MFMAs are
-  // issued (both at once exceed the register budget of 9 waves per CU)
-  double b1[kKC];
-  if (wv < nt) load_bchunk<0>(b1, n, a.G, wv * T16, 0);
-  stage_panel(n, Pk + (size_t)I0 * n, n - I0, sA, ldr);
-  for (int e = threadIdx.x; e < T16 * (ldr - n); e += blockDim.x) {
-    const int i = e / (ldr - n);
-    sR[i * ldr + n + (e - i * (ldr - n))] = 0.0;
-  }
-  __syncthreads();
-  // R = P_k(I,:) G
-#pragma unroll 1
-  for (int jt = wv; jt < nt; jt += kPanelWaves) {
-    dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-    if (jt == wv) {
-      mfma_chunk(acc, b1, sA, ldr, 0);
-      panel_rest<0>(acc, n, sA, ldr, a.G, jt * T16, kKC);
-    } else {
-      panel_rest<0>(acc, n, sA, ldr, a.G, jt * T16, 0);
-    }
-    const int j = jt * T16 + li;
-    if (j >= n) continue;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) sR[(lk + 4 * r) * ldr + j] = acc[r];
-  }
-  double b2[kKC];
-  if (wv < nt) load_bchunk<0>(b2, n, Pk, wv * T16, 0);
-  __syncthreads();
-  // part_k(I,:) = R P_k   (P_k = A^k M is symmetric: the row-major read
-  // is the coalesced one)
-#pragma unroll 1
-  for (int jt = wv; jt < nt; jt += kPanelWaves) {
-    dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-    if (jt == wv) {
-      mfma_chunk(acc, b2, sR, ldr, 0);
-      panel_rest<0>(acc, n, sR, ldr, Pk, jt * T16, kKC);
-    } else {
-      panel_rest<0>(acc, n, sR, ldr, Pk, jt * T16, 0);
-    }
-    const int j = jt * T16 + li;
-    if (j >= n) continue;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = I0 + lk + 4 * r;
-      if (i < n) out[(size_t)i * n + j] = acc[r];
-    }
-  }
-}
 
 struct SumArgs {
   int n, nterm;
@@ -487,27 +393,14 @@ struct SumArgs {
 };
 
 // The convergence test of iteration it (src/paw_waves2.f90:1960-1975) from
-// the block maxima of |GAMN|: every workgroup reaches the same decision; the
-// first one records it.  Then the sum of the terms and the epilogue.
-template <int MODE>
-__global__ void __launch_bounds__(256) k_series_sum(SumArgs a, OrthoState *st) {
-  if (stopped(st)) return;
+// the block maxima of |GAMN|, by the 256 threads of a workgroup: every
+// workgroup reaches the same decision; the first one records it.  In the first
+// iteration also the acceptance test of the preparation (spectral bounds and
+// the Newton-Schulz inverse); a rejection (code 3) makes the host recompute
+// the bounds.  True when the loop ends here.
+__device__ inline bool series_ends(const SumArgs &a, OrthoState *st) {
   __shared__ double wm[4], wp2[4];
   __shared__ int wn[4];
-  const int n = a.n;
-  const size_t n2 = (size_t)n * n;
-  const int idx = blockIdx.x * 256 + threadIdx.x;
-  const bool in = idx < n * n;
-  const int i = in ? idx / n : 0, j = in ? idx - i * n : 0;
-  const bool swap = MODE == kSeriesLambda && in && a.occ[i] < a.occ[j];
-  // element (i,j), or (j,i) where the update takes the transposed element;
-  // the loads of the first group of terms go out with those of the block
-  // maxima, the adds run in the order k = 0, 1, ...
-  const double *src = a.part + (swap ? (size_t)j * n + i : (size_t)i * n + j);
-  constexpr int V = 16;
-  double v[V];
-#pragma unroll
-  for (int u = 0; u < V; ++u) v[u] = (in && u < a.nterm) ? src[(size_t)u * n2] : 0.0;
   double m = 0.0;
   int nan = 0;
   for (int b = threadIdx.x; b < a.nbmax; b += 256) {
@@ -527,9 +420,6 @@ __global__ void __launch_bounds__(256) k_series_sum(SumArgs a, OrthoState *st) {
   __syncthreads();
   m = fmax(fmax(wm[0], wm[1]), fmax(wm[2], wm[3]));
   nan = wn[0] | wn[1] | wn[2] | wn[3];
-  // first iteration: the acceptance test of the preparation (spectral bounds
-  // and the Newton-Schulz inverse); a rejection (code 3) makes the host
-  // recompute the bounds
   bool reject = false;
   if (a.pred) {
     __syncthreads();
@@ -552,17 +442,35 @@ __global__ void __launch_bounds__(256) k_series_sum(SumArgs a, OrthoState *st) {
     p2 = nanmax(nanmax(wp2[0], wp2[1]), nanmax(wp2[2], wp2[3]));
     reject = !((double)a.n_check * p1 <= a.ptol_res && p2 <= a.ptol_pow);
   }
-  // the convergence test of iteration it (src/paw_waves2.f90:1960-1975):
-  // every workgroup reaches the same decision; the first one records it
   const int code = reject ? 3 : (nan ? 1 : (m < a.tol ? 0 : (m > 1.0e200 ? 2 : -1)));
-  if (code >= 0) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      st->code = code;
-      if (code == 0) st->iter = a.it;
-      st->done = 1;
-    }
-    return;
+  if (code < 0) return false;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->code = code;
+    if (code == 0) st->iter = a.it;
+    st->done = 1;
   }
+  return true;
+}
+
+// The test, then the sum of the terms and the epilogue.
+template <int MODE>
+__global__ void __launch_bounds__(256) k_series_sum(SumArgs a, OrthoState *st) {
+  if (stopped(st)) return;
+  const int n = a.n;
+  const size_t n2 = (size_t)n * n;
+  const int idx = blockIdx.x * 256 + threadIdx.x;
+  const bool in = idx < n * n;
+  const int i = in ? idx / n : 0, j = in ? idx - i * n : 0;
+  const bool swap = MODE == kSeriesLambda && in && a.occ[i] < a.occ[j];
+  // element (i,j), or (j,i) where the update takes the transposed element;
+  // the loads of the first group of terms go out with those of the block
+  // maxima, the adds run in the order k = 0, 1, ...
+  const double *src = a.part + (swap ? (size_t)j * n + i : (size_t)i * n + j);
+  constexpr int V = 16;
+  double v[V];
+#pragma unroll
+  for (int u = 0; u < V; ++u) v[u] = (in && u < a.nterm) ? src[(size_t)u * n2] : 0.0;
+  if (series_ends(a, st)) return;
   if (!in) return;
   double sum = 0.0;
 #pragma unroll
@@ -600,6 +508,227 @@ __device__ inline double wave_sum(double s) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
   return s;
+}
+
+// ---------------------------------------------------------------------------
+// Row-panel chains: a workgroup carries a panel of 4 or 8 rows through two or
+// more products, the panel between them in LDS.  v_mfma_f64_4x4x4 (4 rows x 16
+// columns x 4 k, 16 cycles) splits a matrix into two to four times as many
+// workgroups as 16-row panels do at the same rate per cycle; what bounds them is the other
+// operand, n^2 doubles per workgroup from the L2 (3.3 us per product for 144
+// bands, of 1.0 for the matrix instructions).  Staging that operand through
+// LDS, and splitting the k range over the waves, both came out slower.
+//   k_series_terms  (P_k G) P_k, 8 rows: 15.7 -> 10.4 us per iteration for 144
+//                   bands and 8 terms (16-row panels filled 72 of 256 CUs),
+//                   8.0 -> 4.8 for 48, 39 -> 26 for 256, 157 -> 153 for 500
+//   k_ns_chain      one Newton-Schulz step, X' = 2X - (X (B + qI)) X: 144 bands
+//                   9.1 us against 11.4 for its two products as launches
+//   k_build_chain   P_k = M A^k, k < K, and the acceptance maxima: 144 bands,
+//                   K = 8: 32 us against 41 for the doubling launches
+// ---------------------------------------------------------------------------
+constexpr int kChainThreads = 1024;
+inline int chain_threads(int n) { return 64 * std::min(16, (n + T16 - 1) / T16); }
+// LDS row length of a panel: whole groups of eight k, == 8 or 24 (mod 32)
+// doubles, so that the sixteen (row, k pair) reads of a fragment fall into
+// distinct banks
+__host__ __device__ inline int chain_ld(int n) {
+  const int l = (n + 7) & ~7;
+  return l % 16 == 0 ? l + 8 : l;
+}
+
+// acc[f] += A(4f + i, :) B(:, col), the panel A in LDS (columns n .. zero);
+// lane l holds A row l % 4 and B column l % 16 at k pair l / 16, and of the
+// result row l / 16 and column l % 16.  op(k, value) maps the elements of B.
+template <int F, class Op>
+__device__ inline void chain_mul(const double *As, int ld, const double *__restrict__ B, int n, int col, double *acc,
+                                 Op &&op) {
+  constexpr int U = 6;                          // k pairs in flight: 12 loads
+  const int lane = threadIdx.x & 63, kq = 2 * (lane >> 4);
+  const double *ap = As + (lane & 3) * ld + kq;
+  const double *bp = B + min(col, n - 1);
+  const int full = n / 8;                       // groups of eight k inside the matrix
+  double alt[F];
+#pragma unroll
+  for (int f = 0; f < F; ++f) alt[f] = 0.0;
+  auto step = [&](int p, double b0, double b1) {
+    b0 = op(8 * p + kq, b0);
+    b1 = op(8 * p + kq + 1, b1);
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      const double *q = ap + 4 * f * ld + 8 * p;
+      const double a0 = q[0], a1 = q[1];
+      acc[f] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, b0, acc[f], 0, 0, 0);
+      alt[f] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, b1, alt[f], 0, 0, 0);
+    }
+  };
+  int p = 0;
+  for (; p + U <= full; p += U) {
+    double b[2 * U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const double *r = bp + (size_t)(8 * (p + u) + kq) * n;
+      b[2 * u] = r[0];
+      b[2 * u + 1] = r[n];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) step(p + u, b[2 * u], b[2 * u + 1]);
+  }
+  // the remaining groups, rows clamped (their A columns are zero)
+  for (; 8 * p < n; p += 2) {
+    double b[4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int k = 8 * (p + u) + kq;
+      b[2 * u] = bp[(size_t)min(k, n - 1) * n];
+      b[2 * u + 1] = bp[(size_t)min(k + 1, n - 1) * n];
+    }
+    step(p, b[0], b[1]);
+    if (8 * (p + 1) < n) step(p + 1, b[2], b[3]);
+  }
+#pragma unroll
+  for (int f = 0; f < F; ++f) acc[f] += alt[f];
+}
+struct ChainId {
+  __device__ double operator()(int, double v) const { return v; }
+};
+// f(col, column in range) for the column tiles of a wave
+template <class F>
+__device__ inline void chain_cols(int n, F &&f) {
+  const int nt = (n + T16 - 1) / T16, nw = blockDim.x >> 6;
+  for (int ct = threadIdx.x >> 6; ct < nt; ct += nw) f(16 * ct + (int)(threadIdx.x & 15));
+}
+// rows I0 .. I0 + R - 1 of M into LDS, zero outside
+template <int R>
+__device__ inline void chain_stage(const double *M, int n, int I0, double *s, int ld) {
+  for (int e = threadIdx.x; e < R * ld; e += blockDim.x) {
+    const int r = e / ld, k = e - r * ld;
+    s[e] = (k < n && I0 + r < n) ? M[(size_t)(I0 + r) * n + k] : 0.0;
+  }
+}
+
+// X' = 2X - U X, U = X (B + qI) of four rows; U is kept for the residual of
+// the last step ((B + qI) X is its transpose)
+__global__ void __launch_bounds__(kChainThreads) k_ns_chain(int n, double q, const double *Bs, const double *X,
+                                                            double *Xn, double *Uo) {
+  extern __shared__ double sm[];
+  const int ld = chain_ld(n), I0 = blockIdx.x * 4, row = (threadIdx.x & 63) >> 4;
+  double *sx = sm, *su = sm + 4 * ld;
+  chain_stage<4>(X, n, I0, sx, ld);
+  for (int e = threadIdx.x; e < 4 * ld; e += blockDim.x) su[e] = 0.0;
+  __syncthreads();
+  chain_cols(n, [&](int col) {
+    double acc[1] = {0.0};
+    chain_mul<1>(sx, ld, Bs, n, col, acc, ChainId{});
+    if (col >= n) return;
+    const double u = acc[0] + q * sx[row * ld + col];
+    su[row * ld + col] = u;
+    if (I0 + row < n) Uo[(size_t)(I0 + row) * n + col] = u;
+  });
+  __syncthreads();
+  chain_cols(n, [&](int col) {
+    double acc[1] = {0.0};
+    chain_mul<1>(su, ld, X, n, col, acc, ChainId{});
+    if (col < n && I0 + row < n) Xn[(size_t)(I0 + row) * n + col] = 2.0 * sx[row * ld + col] - acc[0];
+  });
+}
+
+// P_k = M A^k for 1 <= k < K, A = I - 2qM, four rows of M and of A carried
+// through all k (they share the loads of A); the acceptance maxima of these
+// rows: max |U - I| and the row sums of |A^h|, h = K/2
+__global__ void __launch_bounds__(kChainThreads) k_build_chain(int n, int K, double q, double *P, const double *U,
+                                                               double *pred) {
+  extern __shared__ double sm[];
+  __shared__ double red[2 * kChainThreads / 64];
+  const int ld = chain_ld(n), I0 = blockIdx.x * 4, row = (threadIdx.x & 63) >> 4;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const size_t n2 = (size_t)n * n;
+  double *cur = sm, *nxt = sm + 8 * ld;
+  double r1 = 0.0, r2 = 0.0;
+  for (int e = threadIdx.x; e < 4 * ld; e += blockDim.x) {
+    const int r = e / ld, k = e - r * ld, i = I0 + r;
+    const bool in = k < n && i < n;
+    const double m = in ? P[(size_t)i * n + k] : 0.0;
+    cur[e] = m;
+    cur[4 * ld + e] = in ? (i == k ? 1.0 : 0.0) - 2.0 * q * m : 0.0;
+    nxt[e] = 0.0;
+    nxt[4 * ld + e] = 0.0;
+    if (in) r1 = nanmax(r1, fabs(U[(size_t)i * n + k] - (i == k ? 1.0 : 0.0)));
+  }
+  __syncthreads();
+  for (int k = 1; k <= K; ++k) {
+    if (2 * k == K) {                           // cur holds the rows of A^k
+      for (int r = wv; r < 4; r += nw) {
+        double s = 0.0;
+        for (int j = lane; j < n; j += 64) s += fabs(cur[(4 + r) * ld + j]);
+        r2 = nanmax(r2, wave_sum(s));
+      }
+    }
+    if (k == K) break;
+    double *Pk = P + (size_t)k * n2;
+    chain_cols(n, [&](int col) {
+      double acc[2] = {0.0, 0.0};
+      chain_mul<2>(cur, ld, P, n, col, acc,
+                   [&](int kk, double m) { return (kk == col ? 1.0 : 0.0) - 2.0 * q * m; });
+      if (col >= n) return;
+      nxt[row * ld + col] = acc[0];
+      nxt[(4 + row) * ld + col] = acc[1];
+      if (I0 + row < n) Pk[(size_t)(I0 + row) * n + col] = acc[0];
+    });
+    __syncthreads();
+    double *s = cur;
+    cur = nxt;
+    nxt = s;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    r1 = nanmax(r1, __shfl_xor(r1, o));
+    r2 = nanmax(r2, __shfl_xor(r2, o));
+  }
+  if (lane == 0) {
+    red[2 * wv] = r1;
+    red[2 * wv + 1] = r2;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < nw; ++w) {
+      r1 = nanmax(r1, red[2 * w]);
+      r2 = nanmax(r2, red[2 * w + 1]);
+    }
+    pred[2 * blockIdx.x] = r1;
+    pred[2 * blockIdx.x + 1] = r2;
+  }
+}
+
+// Eight rows of the term P_k G P_k (P_k symmetric: the row-major read is the
+// coalesced one).  The terms are the fast index of the grid, so that with
+// eight of them an XCD reads one P_k.
+__global__ void __launch_bounds__(kChainThreads) k_series_terms(SeriesArgs a, int nterm, const OrthoState *st) {
+  if (stopped(st)) return;
+  extern __shared__ double sm[];
+  const int n = a.n, ld = chain_ld(n), row = (threadIdx.x & 63) >> 4;
+  const size_t n2 = (size_t)n * n;
+  double *sp = sm, *su = sm + 8 * ld;
+  const int k = blockIdx.x % nterm, I0 = 8 * (blockIdx.x / nterm);
+  const double *Pk = a.P + (size_t)k * n2;
+  double *out = a.part + (size_t)k * n2;
+  chain_stage<8>(Pk, n, I0, sp, ld);
+  for (int e = threadIdx.x; e < 8 * ld; e += blockDim.x) su[e] = 0.0;
+  __syncthreads();
+  chain_cols(n, [&](int col) {
+    double acc[2] = {0.0, 0.0};
+    chain_mul<2>(sp, ld, a.G, n, col, acc, ChainId{});
+    if (col >= n) return;
+    su[row * ld + col] = acc[0];
+    su[(4 + row) * ld + col] = acc[1];
+  });
+  __syncthreads();
+  chain_cols(n, [&](int col) {
+    double acc[2] = {0.0, 0.0};
+    chain_mul<2>(su, ld, Pk, n, col, acc, ChainId{});
+    if (col >= n) return;
+    if (I0 + row < n) out[(size_t)(I0 + row) * n + col] = acc[0];
+    if (I0 + 4 + row < n) out[(size_t)(I0 + 4 + row) * n + col] = acc[1];
+  });
 }
 
 // number of eigenvalues below x of the symmetric tridiagonal (al, be[1..k-1])
@@ -1239,8 +1368,8 @@ int ortho_work(pw_waveset *ws, OrthoWork &w) {
   static std::once_flag lds_once;
   static hipError_t lds_err = hipSuccess;
   std::call_once(lds_once, [] {
-    const void *fns[] = {(const void *)k_panel_batch, (const void *)k_series_panel, (const void *)k_ortho_small<1>,
-                         (const void *)k_ortho_small<2>};
+    const void *fns[] = {(const void *)k_panel_batch, (const void *)k_series_terms, (const void *)k_ns_chain,
+                         (const void *)k_build_chain, (const void *)k_ortho_small<1>, (const void *)k_ortho_small<2>};
     for (const void *f : fns) {
       hipFuncAttributes fa{};
       hipError_t e = hipFuncGetAttributes(&fa, f);
@@ -1288,9 +1417,10 @@ int panel_batch(pw_waveset *ws, const BatchArgs &a) {
   return PW_OK;
 }
 
-void series_panel(pw_waveset *ws, const SeriesArgs &a, int nterm, const OrthoState *st) {
-  const dim3 grid((a.n + T16 - 1) / T16, nterm);
-  k_series_panel<<<grid, 64 * kPanelWaves, 2 * panel_lds(a.n), ws->stream>>>(a, st);
+// LDS of two panels of `rows` rows
+inline size_t chain_lds(int n, int rows) { return (size_t)2 * rows * chain_ld(n) * sizeof(double); }
+void series_terms(pw_waveset *ws, const SeriesArgs &a, int nterm, const OrthoState *st) {
+  k_series_terms<<<(a.n + 7) / 8 * nterm, chain_threads(a.n), chain_lds(a.n, 8), ws->stream>>>(a, nterm, st);
 }
 
 template <int MODE>
@@ -1331,6 +1461,17 @@ struct OrthoParams {
   int nns;    // Newton-Schulz steps
 };
 
+// A Newton-Schulz step as one chain of two products instead of two launches:
+// the chain costs 3.3 us per product and 2.5 in all for 144 bands, where the
+// launches take 5.0 each and a gap; its time grows with n^2 on a quarter of the
+// CUs, 18.7 us against 13.6 for 256 bands.
+constexpr int kNsChainMaxN = 160;
+// The series matrices one after the other, K - 1 products in one launch,
+// instead of doubled in J launches: 32 us against 41 for 144 bands, 71 against
+// 82 for 256 and 248 against 280 for 500, all with K = 8; with 16 the doubling
+// needs one launch more, the chain 8 products.
+constexpr int kBuildChainMaxK = 8;
+
 // M, the series matrices P_k = A^k M, the powers A^(2^j) and the acceptance
 // test (everything before the outer loop)
 int enqueue_prep(pw_waveset *ws, const OrthoWork &w, const OrthoParams &P) {
@@ -1346,10 +1487,20 @@ int enqueue_prep(pw_waveset *ws, const OrthoWork &w, const OrthoParams &P) {
   double *mc = w.m0, *mn = w.m1;
   for (int k = 1; k < P.nns; ++k) {
     double *dst = (k + 1 == P.nns) ? w.pstk : mn;
-    gemm(ws, w.bs, 0, mc, 0, w.t1, 1.0, mc, P.q);       // T = (B+qI) X
-    gemm(ws, mc, 0, w.t1, 0, dst, -1.0, mc, 2.0);       // X' = 2X - X T
+    if (n <= kNsChainMaxN) {
+      k_ns_chain<<<(n + 3) / 4, chain_threads(n), chain_lds(n, 4), ws->stream>>>(n, P.q, w.bs, mc, dst, w.t1);
+    } else {
+      gemm(ws, w.bs, 0, mc, 0, w.t1, 1.0, mc, P.q);     // T = (B+qI) X
+      gemm(ws, mc, 0, w.t1, 0, dst, -1.0, mc, 2.0);     // X' = 2X - X T
+    }
     mn = mc;
     mc = dst;
+  }
+  if (ls == P.nlev && (1 << ls) <= kBuildChainMaxK) {
+    k_build_chain<<<(n + 3) / 4, chain_threads(n), chain_lds(n, 8), ws->stream>>>(n, 1 << ls, P.q, w.pstk, w.t1,
+                                                                                 w.pred);
+    PW_HIP(hipGetLastError());
+    return PW_OK;
   }
   // A = I - 2qM; level j doubles the series, P_{2^j + k} = A^(2^j) P_k for
   // k < 2^j, and squares the power, A^(2^(j+1)) = A^(2^j) A^(2^j)
@@ -1409,10 +1560,7 @@ int enqueue_iters(pw_waveset *ws, const OrthoWork &w, const OrthoParams &P, doub
       sa.P = w.pstk;
       sa.G = w.gam;
       sa.part = w.spart;
-      sa.bmax = w.red;
-      sa.nbmax = nt * nt;
-      sa.tol = eps;
-      series_panel(ws, sa, 1 << ls, w.st);
+      series_terms(ws, sa, 1 << ls, w.st);
     } else {
       gemm(ws, w.gam, 0, w.pstk, 0, w.t1, 1.0, nullptr, 0.0, w.st);
       gemm(ws, w.pstk, 0, w.t1, 0, w.spart, 1.0, nullptr, 0.0, w.st);

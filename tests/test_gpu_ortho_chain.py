@@ -1,0 +1,29 @@
+"""ORTHO_X by row-panel chains against the oracle: remainders of the panels of
+4 and 8 rows, of the column tiles of 16 and of the groups of 8 and 48 k, one
+column tile per wave and more (above 256 bands), the widest set with a
+Newton-Schulz step in one launch and the first one above it, 4 to 32 terms of
+the series (up to 8 built in one launch).  Both sides form the same iterates;
+the series is cut at 1.6e-11 of its first term and the bound is that of the
+other stand-alone solves, 1e-10.
+"""
+import numpy as np
+import pytest
+
+from harness import relerr
+from test_gpu_ortho_small import solve_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nb,spread", [(33, 1.1), (36, 6.0), (39, 60.0), (47, 1.1), (48, 6.0), (64, 1.1), (97, 6.0),
+                                       (100, 1.1), (144, 6.0), (160, 1.1), (161, 1.1), (255, 1.1), (256, 1.1),
+                                       (257, 1.1), (300, 6.0), (620, 1.1)])
+def test_ortho_x_row_panels(nb, spread):
+    import pwgpu
+    from oracle import waves as owv
+    occ, chichi, psipsi, chipsi = solve_case(nb, spread)
+    lam0 = 0.001 * np.random.default_rng(nb).normal(size=(nb, nb))
+    ref, it_ref = owv.ortho_x(occ, chichi, psipsi, chipsi, lam0.copy())
+    lam, it = pwgpu.ortho_x(occ, chichi, psipsi, chipsi, lam0)
+    assert it == it_ref
+    assert relerr(lam, ref) < 1e-10

@@ -29,12 +29,14 @@
 // whose matrices fit in LDS are solved by one workgroup in one launch.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "pw_common.h"
+#include "pw_device.h"
 
 namespace {
 
-typedef double dbl4 __attribute__((ext_vector_type(4)));
+typedef double dbl2u __attribute__((ext_vector_type(2), aligned(8)));
 
 constexpr int T16 = 16;
 constexpr int kMaxLevels = 12;
@@ -504,10 +506,11 @@ __global__ void k_symm(int n, const double *B, double *Bs) {
   Bs[idx] = 0.5 * (B[(size_t)i * n + j] + B[(size_t)j * n + i]);
 }
 
+// over the wave: inside the rows of 16 lanes by DPP, across them by two shuffles
 __device__ inline double wave_sum(double s) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  return s;
+  s = row16_sum(s);
+  s += __shfl_xor(s, 16);
+  return s + __shfl_xor(s, 32);
 }
 
 // ---------------------------------------------------------------------------
@@ -747,21 +750,24 @@ __device__ int sturm_count(int k, const double *al, const double *be, double x) 
 // Lanczos with two passes of classical Gram-Schmidt against all previous
 // vectors, then multisection on the Sturm sequence of the tridiagonal matrix.
 // out = {smallest, largest} Ritz value (inner bounds of the spectrum).
-// One workgroup of kLzThreads; the Krylov basis lives in LDS.
+// One workgroup of kLzThreads; the Krylov basis lives in LDS.  What bounds a
+// step is B from the L2 into one CU: 16-byte loads of two columns per lane, a
+// wave contiguous, sixteen rows in flight (8-byte loads, eight in flight:
+// 409 us for 256 bands and 30 steps, now 258; 144 bands 264 -> 192, 500 1057 -> 589).
 __global__ void __launch_bounds__(kLzThreads) k_lanczos(int n, int m, const double *__restrict__ B,
                                                         double *out) {
   extern __shared__ double sm[];
   double *V = sm;                          // [m+1][n]
   double *w = V + (size_t)(m + 1) * n;     // [n]
-  double *wp = w + n;                      // [G][n] partial matvec, G*n <= kLzThreads
-  double *c = wp + kLzThreads;             // [m+1]
+  double *wp = w + n;                      // [G][n] partial matvec, G*n <= 2 kLzThreads
+  double *c = wp + 2 * kLzThreads;         // [m+1]
   double *al = c + (m + 1);                // [m]
   double *be = al + m;                     // [m+1]
   __shared__ double red[kLzThreads / 64];
   __shared__ int kend_s;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   constexpr int NW = kLzThreads / 64;
-  const int G = max(1, kLzThreads / n);
+  const int np = (n + 1) / 2, G = min(16, kLzThreads / np);   // column pairs, row groups
   auto block_sum = [&](double s) -> double {
     s = wave_sum(s);
     if (lane == 0) red[wv] = s;
@@ -783,24 +789,42 @@ __global__ void __launch_bounds__(kLzThreads) k_lanczos(int n, int m, const doub
   __syncthreads();
   for (int k = 0; k < m; ++k) {
     const double *v = V + (size_t)k * n;
-    // w = B v (B symmetric: column reads are coalesced); G row groups per column
-    for (int e = t; e < G * n; e += kLzThreads) {
-      const int i = e % n, g = e / n;
+    // w = B v (B symmetric: column reads are coalesced); G row groups per
+    // column pair; the last pair of an odd n starts one column earlier
+    if (t < G * np) {
+      const int p = t % np, g = t / np, col = min(2 * p, n - 2);
       const int jlo = (int)((long)n * g / G), jhi = (int)((long)n * (g + 1) / G);
-      double a[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      double a0 = 0.0, a1 = 0.0, c0 = 0.0, c1 = 0.0;
       int j = jlo;
-      for (; j + 7 < jhi; j += 8) {
+      auto rows = [&](auto nu) {
+        constexpr int U = decltype(nu)::value;
+        for (; j + U <= jhi; j += U) {
+          dbl2u b[U];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) a[u] += B[(size_t)(j + u) * n + i] * v[j + u];
-      }
-      for (; j < jhi; ++j) a[0] += B[(size_t)j * n + i] * v[j];
-      wp[(size_t)g * n + i] = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+          for (int u = 0; u < U; ++u) b[u] = *reinterpret_cast<const dbl2u *>(B + (size_t)(j + u) * n + col);
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            double &s0 = u & 1 ? c0 : a0, &s1 = u & 1 ? c1 : a1;
+            s0 += b[u].x * v[j + u];
+            s1 += b[u].y * v[j + u];
+          }
+        }
+      };
+      rows(std::integral_constant<int, 16>{});
+      rows(std::integral_constant<int, 4>{});
+      rows(std::integral_constant<int, 1>{});
+      a0 += c0;
+      a1 += c1;
+      if (col == 2 * p) wp[g * n + col] = a0;
+      wp[g * n + col + 1] = a1;
     }
     __syncthreads();
     for (int i = t; i < n; i += kLzThreads) {
-      double r = 0.0;
-      for (int g = 0; g < G; ++g) r += wp[(size_t)g * n + i];
-      w[i] = r;
+      double r[2] = {0.0, 0.0};
+#pragma unroll
+      for (int g = 0; g < 16; ++g)
+        if (g < G) r[g & 1] += wp[g * n + i];
+      w[i] = r[0] + r[1];
     }
     __syncthreads();
     for (int pass = 0; pass < 2; ++pass) {
@@ -837,8 +861,9 @@ __global__ void __launch_bounds__(kLzThreads) k_lanczos(int n, int m, const doub
   }
   __syncthreads();
   const int kend = kend_s;
-  if (wv != 0) return;
-  // Gershgorin interval of the tridiagonal matrix (every lane of wave 0)
+  if (wv > 1) return;
+  // wave 0 the smallest, wave 1 the largest eigenvalue: Gershgorin interval of
+  // the tridiagonal matrix (every lane)
   double glo = 1.0e300, ghi = -1.0e300;
   for (int i = 0; i < kend; ++i) {
     const double r = (i > 0 ? fabs(be[i]) : 0.0) + (i + 1 < kend ? fabs(be[i + 1]) : 0.0);
@@ -846,28 +871,22 @@ __global__ void __launch_bounds__(kLzThreads) k_lanczos(int n, int m, const doub
     ghi = fmax(ghi, al[i] + r);
   }
   // multisection: each round splits the bracket into 65 parts, one lane per point
-  double res[2];
-  for (int side = 0; side < 2; ++side) {
-    double lo = glo, hi = ghi;
-    for (int round = 0; round < 9; ++round) {
-      const double x = lo + (hi - lo) * (double)(lane + 1) / 65.0;
-      const int cnt = sturm_count(kend, al, be, x);
-      // side 0: smallest eigenvalue = first point with count >= 1
-      // side 1: largest eigenvalue = first point with count >= kend
-      const bool above = side == 0 ? cnt >= 1 : cnt >= kend;
-      const unsigned long long mask = __ballot(above);
-      const int first = mask ? __ffsll((long long)mask) - 1 : 64;
-      const double nlo = lo + (hi - lo) * (double)first / 65.0;
-      const double nhi = lo + (hi - lo) * (double)(first + 1) / 65.0;
-      lo = nlo;
-      hi = nhi;
-    }
-    res[side] = 0.5 * (lo + hi);
+  const int side = wv;
+  double lo = glo, hi = ghi;
+  for (int round = 0; round < 9; ++round) {
+    const double x = lo + (hi - lo) * (double)(lane + 1) / 65.0;
+    const int cnt = sturm_count(kend, al, be, x);
+    // side 0: smallest eigenvalue = first point with count >= 1
+    // side 1: largest eigenvalue = first point with count >= kend
+    const bool above = side == 0 ? cnt >= 1 : cnt >= kend;
+    const unsigned long long mask = __ballot(above);
+    const int first = mask ? __ffsll((long long)mask) - 1 : 64;
+    const double nlo = lo + (hi - lo) * (double)first / 65.0;
+    const double nhi = lo + (hi - lo) * (double)(first + 1) / 65.0;
+    lo = nlo;
+    hi = nhi;
   }
-  if (lane == 0) {
-    out[0] = res[0];
-    out[1] = res[1];
-  }
+  if (lane == 0) out[side] = 0.5 * (lo + hi);
 }
 
 // Acceptance test of the spectral bounds (before the outer loop): the
@@ -1432,11 +1451,11 @@ void series_sum(pw_waveset *ws, const SumArgs &a, OrthoState *st) {
 int lanczos_bounds(pw_waveset *ws, const double *d_b, double *d_out, double *lo, double *hi) {
   const int n = ws->nb;
   if (n > kLzThreads) return pw_fail(PW_ERR_UNSUPPORTED, "WAVES_ORTHO_X: NB too large");
-  // LDS: (m+1) n + n + kLzThreads + 3m + 2 doubles, at most 144 KiB
-  const long budget = 144L * 1024 / 8 - n - kLzThreads - 3 * kLzMaxSteps - 2;
+  // LDS: (m+1) n + n + 2 kLzThreads + 3m + 2 doubles, at most 152 KiB
+  const long budget = 152L * 1024 / 8 - n - 2 * kLzThreads - 3 * kLzMaxSteps - 2;
   int m = std::min({n, kLzMaxSteps, (int)(budget / n) - 1});
   if (m < 2) return pw_fail(PW_ERR_UNSUPPORTED, "WAVES_ORTHO_X: NB too large for the Lanczos bounds");
-  const size_t lds = ((size_t)(m + 1) * n + n + kLzThreads + 3 * (size_t)m + 2) * sizeof(double);
+  const size_t lds = ((size_t)(m + 1) * n + n + 2 * kLzThreads + 3 * (size_t)m + 2) * sizeof(double);
   if (lds > 65536)
     PW_HIP(hipFuncSetAttribute((const void *)k_lanczos, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)lds));

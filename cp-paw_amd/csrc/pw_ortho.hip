@@ -1367,13 +1367,18 @@ struct OrthoWork {
   OrthoState *st;
 };
 
+// block-maxima slots: (n^2+255)/256 for the GAMN maxima, (n+3)/4 row groups
+// for the acceptance test (k_prep_part)
+inline size_t ortho_slots(size_t n) { return std::max((n * n + 255) / 256, (n + 3) / 4); }
+inline size_t ortho_need(size_t n) {
+  return (9 + kMaxLevels + 2 * ((size_t)1 << kSeriesMaxLevels)) * n * n + n + 4 * ortho_slots(n) + 64;
+}
+
 int ortho_work(pw_waveset *ws, OrthoWork &w) {
   const size_t n2 = (size_t)ws->nb * ws->nb;
-  // block-maxima slots: (n^2+255)/256 for the GAMN maxima, (n+3)/4 row groups
-  // for the acceptance test (k_prep_part)
-  const size_t nblk = std::max((n2 + 255) / 256, ((size_t)ws->nb + 3) / 4);
+  const size_t nblk = ortho_slots(ws->nb);
   const size_t kser = (size_t)1 << kSeriesMaxLevels;
-  const size_t need = (9 + kMaxLevels + 2 * kser) * n2 + ws->nb + 4 * nblk + 64;
+  const size_t need = ortho_need(ws->nb);
   if (need > ws->ortho_cap) {
     if (ws->d_ortho) PW_HIP(hipFree(ws->d_ortho));
     ws->d_ortho = nullptr;
@@ -1860,11 +1865,12 @@ int ortho_x_device(pw_waveset *ws, double *d_lam, const double *d_chichi, const 
     const OrthoGraphKey key{P.lo, P.hi, P.nlev, P.nns, batch, d_lam, d_chichi, d_psipsi, d_chipsi, ws->d_ortho};
     if (!ws->ortho_exec || !(ws->ortho_key == key)) {
       ortho_graph_release(ws);
-      // with other plans or wavesets alive (a request loop) the work is issued
-      // directly below; an existing graph is still replayed
+      // with other plans or wavesets alive (a request loop), and for a single
+      // solve (capture, instantiation and release cost more than the launches
+      // of the one replay save), the work is issued directly below; an existing graph is still replayed
       CaptureGate &gate = capture_gate();
       std::unique_lock<std::mutex> lk(gate.mu);
-      if (gate.plans <= 1 && gate.wavesets <= 1) {
+      if (!ws->ortho_once && gate.plans <= 1 && gate.wavesets <= 1) {
         PW_HIP(hipStreamBeginCapture(ws->stream, hipStreamCaptureModeRelaxed));
         int rq = enqueue_prep(ws, w, P);
         if (rq == PW_OK) rq = enqueue_iters(ws, w, P, lbuf, d_chichi, d_psipsi, d_chipsi, 1, batch);
@@ -1926,39 +1932,81 @@ int ortho_x_device(pw_waveset *ws, double *d_lam, const double *d_chichi, const 
 }
 
 // ---------------------------------------------------------------------------
-// C ABI: WAVES_ORTHO_X on host matrices (column-major NB x NB)
+// C ABI: WAVES_ORTHO_X on host matrices, column-major (pw_ortho_x) or row-major
+// (pw_ortho_x_rows) NB x NB.
+//
+// What bounded the call was the host: transposes by element loops on both
+// sides of the C entry (0.9 of 2.1 ms for 256 bands), the creation of a stream,
+// a graph that is replayed once.  The matrices are uploaded as they are and
+// transposed on the device, the solve runs on the thread's default stream with
+// its launches issued directly, all device memory is one allocation.
 // ---------------------------------------------------------------------------
+namespace {
+
+// out_m = transpose of in_m, m = blockIdx.z, by 32 x 32 tiles
+__global__ void __launch_bounds__(256) k_transpose_mats(int n, const double *__restrict__ in,
+                                                        double *__restrict__ out) {
+  __shared__ double s[32][33];
+  const size_t o = (size_t)blockIdx.z * n * n;
+  const int i0 = blockIdx.y * 32, j0 = blockIdx.x * 32, c = threadIdx.x & 31, r = threadIdx.x >> 5;
+  for (int q = r; q < 32; q += 8)
+    if (i0 + q < n && j0 + c < n) s[q][c] = in[o + (size_t)(i0 + q) * n + j0 + c];
+  __syncthreads();
+  for (int q = r; q < 32; q += 8)
+    if (j0 + q < n && i0 + c < n) out[o + (size_t)(j0 + q) * n + i0 + c] = s[c][q];
+}
+
+int ortho_x_host(int nb, const double *occ, const double *const src[4], double *lambda, int *iter, bool rows) {
+  pw_waveset ws;
+  OrthoState state{};
+  ws.nb = nb;
+  ws.stream = hipStreamPerThread;
+  ws.occ.assign(occ, occ + nb);
+  ws.h_ortho_state = &state;
+  ws.ortho_once = true;
+  const size_t n2 = (size_t)nb * nb, need = ortho_need(nb), mats = (rows ? 4 : 8) * n2;
+  double *base = nullptr;
+  PW_HIP(hipMalloc(&base, (need + mats) * sizeof(double)));
+  ws.d_ortho = base;
+  ws.ortho_cap = need;
+  double *d = base + need, *up = rows ? d : d + 4 * n2;
+  const dim3 grid((nb + 31) / 32, (nb + 31) / 32, 4);
+  int rc = PW_OK;
+  for (int m = 0; m < 4 && rc == PW_OK; ++m)
+    if (hipMemcpyAsync(up + m * n2, src[m], n2 * sizeof(double), hipMemcpyHostToDevice, ws.stream) != hipSuccess)
+      rc = pw_fail(PW_ERR_HIP, "pw_ortho_x: upload failed");
+  if (rc == PW_OK && !rows) {
+    k_transpose_mats<<<grid, 256, 0, ws.stream>>>(nb, up, d);
+    if (hipGetLastError() != hipSuccess) rc = pw_fail(PW_ERR_HIP, "pw_ortho_x: transposition failed");
+  }
+  if (rc == PW_OK) rc = ortho_x_device(&ws, d + 3 * n2, d, d + n2, d + 2 * n2, iter);
+  if (rc == PW_OK && !rows) {
+    k_transpose_mats<<<dim3(grid.x, grid.y, 1), 256, 0, ws.stream>>>(nb, d + 3 * n2, up);
+    if (hipGetLastError() != hipSuccess) rc = pw_fail(PW_ERR_HIP, "pw_ortho_x: transposition failed");
+  }
+  if (rc == PW_OK &&
+      hipMemcpyAsync(lambda, rows ? d + 3 * n2 : up, n2 * sizeof(double), hipMemcpyDeviceToHost, ws.stream) != hipSuccess)
+    rc = pw_fail(PW_ERR_HIP, "pw_ortho_x: download failed");
+  if (hipStreamSynchronize(ws.stream) != hipSuccess && rc == PW_OK)
+    rc = pw_fail(PW_ERR_HIP, "pw_ortho_x: stream synchronisation failed");
+  (void)hipFree(base);
+  return rc;
+}
+
+}  // namespace
+
 extern "C" int pw_ortho_x(int nb, const double *occ, const double *chichi, const double *psipsi,
                           const double *chipsi, double *lambda, int *iter) {
   if (nb <= 0 || !occ || !chichi || !psipsi || !chipsi || !lambda || !iter)
     return pw_fail(PW_ERR_ARG, "pw_ortho_x: bad argument");
-  pw_waveset ws;
-  ws.nb = nb;
-  PW_HIP(hipStreamCreateWithFlags(&ws.stream, hipStreamNonBlocking));
-  ws.occ.assign(occ, occ + nb);
-  const size_t n2 = (size_t)nb * nb;
-  std::vector<double> h(4 * n2);
-  const double *src[4] = {chichi, psipsi, chipsi, lambda};
-  for (int m = 0; m < 4; ++m)
-    for (int i = 0; i < nb; ++i)
-      for (int j = 0; j < nb; ++j) h[m * n2 + (size_t)i * nb + j] = src[m][(size_t)j * nb + i];
-  double *d = nullptr;
-  PW_HIP(hipMalloc(&d, 4 * n2 * sizeof(double)));
-  int rc = PW_OK;
-  if (hipMemcpy(d, h.data(), 4 * n2 * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
-    rc = pw_fail(PW_ERR_HIP, "pw_ortho_x: upload failed");
-  if (rc == PW_OK) rc = ortho_x_device(&ws, d + 3 * n2, d, d + n2, d + 2 * n2, iter);
-  if (rc == PW_OK && hipStreamSynchronize(ws.stream) != hipSuccess)
-    rc = pw_fail(PW_ERR_HIP, "pw_ortho_x: stream synchronisation failed");
-  if (rc == PW_OK && hipMemcpy(h.data() + 3 * n2, d + 3 * n2, n2 * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
-    rc = pw_fail(PW_ERR_HIP, "pw_ortho_x: download failed");
-  if (rc == PW_OK)
-    for (int i = 0; i < nb; ++i)
-      for (int j = 0; j < nb; ++j) lambda[(size_t)j * nb + i] = h[3 * n2 + (size_t)i * nb + j];
-  ortho_graph_release(&ws);
-  (void)hipFree(d);
-  if (ws.d_ortho) (void)hipFree(ws.d_ortho);
-  if (ws.h_ortho_state) (void)hipHostFree(ws.h_ortho_state);
-  (void)hipStreamDestroy(ws.stream);
-  return rc;
+  const double *const src[4] = {chichi, psipsi, chipsi, lambda};
+  return ortho_x_host(nb, occ, src, lambda, iter, false);
+}
+
+extern "C" int pw_ortho_x_rows(int nb, const double *occ, const double *chichi, const double *psipsi,
+                               const double *chipsi, double *lambda, int *iter) {
+  if (nb <= 0 || !occ || !chichi || !psipsi || !chipsi || !lambda || !iter)
+    return pw_fail(PW_ERR_ARG, "pw_ortho_x: bad argument");
+  const double *const src[4] = {chichi, psipsi, chipsi, lambda};
+  return ortho_x_host(nb, occ, src, lambda, iter, true);
 }

@@ -257,10 +257,9 @@ def ortho_x(occ, chichi, psipsi, chipsi, lam):
     """WAVES_ORTHO_X on the GPU (FP64); numpy (NB,NB) matrices, returns (lambda, iter)."""
     lib = _lib.load()
     nb = len(occ)
-    f = lambda m: np.ascontiguousarray(np.asarray(m, dtype=np.float64).T)
-    occ = np.ascontiguousarray(occ, dtype=np.float64)
-    a, b, c = f(chichi), f(psipsi), f(chipsi)
-    l = f(lam)
+    f = lambda m: np.ascontiguousarray(m, dtype=np.float64)
+    occ, a, b, c = f(occ), f(chichi), f(psipsi), f(chipsi)
+    l = np.array(lam, dtype=np.float64, order="C")
     it = ctypes.c_int()
-    check(lib.pw_ortho_x(nb, dptr(occ), dptr(a), dptr(b), dptr(c), dptr(l), ctypes.byref(it)))
-    return l.T.copy(), it.value
+    check(lib.pw_ortho_x_rows(nb, dptr(occ), dptr(a), dptr(b), dptr(c), dptr(l), ctypes.byref(it)))
+    return l, it.value

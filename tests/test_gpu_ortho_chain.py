@@ -27,3 +27,22 @@ def test_ortho_x_row_panels(nb, spread):
     lam, it = pwgpu.ortho_x(occ, chichi, psipsi, chipsi, lam0)
     assert it == it_ref
     assert relerr(lam, ref) < 1e-10
+
+
+@pytest.mark.parametrize("nb", [5, 32, 33, 65])
+def test_ortho_x_column_major(nb):
+    """The C entry on column-major matrices gives the bits of the row-major one
+    (the matrices are transposed on the device, edges of 32 x 32 tiles)."""
+    import ctypes
+
+    import pwgpu
+    from pwgpu import load
+    from pwgpu._lib import dptr
+    occ, chichi, psipsi, chipsi = solve_case(nb, 1.1)
+    lam0 = 0.001 * np.random.default_rng(nb).normal(size=(nb, nb))
+    ref, it_ref = pwgpu.ortho_x(occ, chichi, psipsi, chipsi, lam0)
+    col = [np.array(m.T, dtype=np.float64, order="C") for m in (chichi, psipsi, chipsi, lam0)]
+    it = ctypes.c_int()
+    assert load().pw_ortho_x(nb, dptr(occ), *[dptr(m) for m in col], ctypes.byref(it)) == 0
+    assert it.value == it_ref
+    assert np.array_equal(col[3].T, ref)

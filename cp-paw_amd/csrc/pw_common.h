@@ -383,8 +383,13 @@ int k_force(pw_waveset *ws, const double2 *psi, const double2 *phase, const doub
 int k_residual(pw_waveset *ws, const double2 *psibar, double *dst);
 int k_overlap(pw_waveset *ws, const double2 *psi1, const double2 *psi2, double *mat_host_or_dev, bool to_host, bool tid);
 // mat_dev = WAVES_OVERLAP(psi1, psi2) + WAVES_1COVERLAP(proj1, proj2) in one sequence
-int k_overlap_full(pw_waveset *ws, const double2 *psi1, const double2 *psi2, const double2 *proj1,
-                   const double2 *proj2, double *mat_dev);
+// one overlap matrix: psi1, psi2 with their projections (null: no one-centre part)
+constexpr int kOvlJobs = 3;
+struct OverlapJob {
+  const double2 *psi1, *psi2, *proj1, *proj2;
+  double *mat;
+};
+int k_overlap_full(pw_waveset *ws, const OverlapJob *jobs, int nj);
 int k_addopsi(pw_waveset *ws, double2 *psibar, const double2 *chi, const double *lam_dev);
 int k_addoproj(pw_waveset *ws, double2 *proj, const double2 *oproj, const double *lam_dev);
 int k_atom_matrix(pw_waveset *ws, const double2 *proj, double2 *out, const double2 *mats);
@@ -407,7 +412,7 @@ inline int half_pad(const pw_plan *p) { return (p->nh + 31) / 32 * 32; }
 int half_factors_room(pw_waveset *ws);
 int half_factors(pw_waveset *ws);
 int half_projections(pw_waveset *ws, const double2 *psi, double2 *proj);
-int half_overlap(pw_waveset *ws, const double2 *psi1, const double2 *psi2, const double4 *p1c, int nz, double *mat);
+int half_overlap(pw_waveset *ws, const OverlapJob *jobs, int nj, const double4 *p1c, int nz);
 int half_addpro(pw_waveset *ws, const ColOut &out, const double2 *x);
 int half_addopsi(pw_waveset *ws, double2 *psibar, const double2 *chi, const double *lam);
 int half_force(pw_waveset *ws, const double2 *psi, const double2 *ded, double *dst);

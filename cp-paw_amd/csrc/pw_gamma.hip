@@ -89,6 +89,7 @@ __device__ inline Bands2 split_pair(const Pair &v, bool self) {
 template <int NW>
 struct RowsP {
   HalfP p;
+  __device__ void job(int) {}
   struct Row {
     const double *f[2];
     const double2 *e[2];
@@ -137,8 +138,10 @@ struct RowsP {
 // 2 sum over the sphere of conj(c) c'
 template <int NW>
 struct RowsX {
-  const double2 *psi;
+  const double2 *psis[kOvlJobs];
   int ngl, nbh;
+  const double2 *psi;
+  __device__ void job(int j) { psi = psis[j]; }
   struct Row {
     size_t off;
     bool ok;
@@ -164,22 +167,31 @@ struct RowsX {
   }
 };
 
+// the band operands of up to kOvlJobs products of one launch
+struct HalfBands {
+  const double2 *psi[kOvlJobs];
+  int n;
+};
+
 // Workgroup: NW waves, 16 rows each, NC blocks of 16 real bands; K chunks of
 // 16 double-buffered in LDS with one barrier each, the operands of the next
 // chunk loaded into registers before the current chunk's MFMAs and stored
 // after them.
 template <class Rows, int NC, int NW>
-__global__ void __launch_bounds__(64 * NW, 2) k_half_row(Rows rows, const double2 *__restrict__ psi,
+__global__ void __launch_bounds__(64 * NW, 2) k_half_row(Rows rows, HalfBands bands,
                                                          const int2 *__restrict__ hg, int nh, int nrow, int ngl,
                                                          int nbh, int hsplit, int tr, int tb, int ns,
                                                          double *__restrict__ part) {
   constexpr int WR = 16 * NW, SA = hpad(WR), WC = 16 * NC, SB = hpad(WC);
   constexpr int NBT = (NC + NW - 1) / NW;      // (super band, hh) of the band operand per thread
   __shared__ double sA[2][HKR][SA], sB[2][HKR][SB];
-  const XcdTile xt = xcd_tile(tr * tb, ns);
+  const XcdTile xt = xcd_tile(tr * tb * bands.n, ns);
   if (!xt.valid) return;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6, li = lane & 15, lk = lane >> 4, hh = t & 7;
-  const int r0 = (xt.inner % tr) * WR, b0 = (xt.inner / tr) * (8 * NC);
+  const int job = xt.inner / (tr * tb), tile = xt.inner - job * tr * tb;
+  const int r0 = (tile % tr) * WR, b0 = (tile / tr) * (8 * NC);
+  const double2 *__restrict__ psi = bands.psi[job];
+  rows.job(job);
   const int h0 = xt.shared * hsplit, h1 = min(nh, h0 + hsplit);
   const int nchunk = (h1 - h0 + HK - 1) / HK;
   dbl4 acc[NC];
@@ -237,7 +249,7 @@ __global__ void __launch_bounds__(64 * NW, 2) k_half_row(Rows rows, const double
     }
     if (more) store((c + 1) & 1, self);
   }
-  double *dst = part + (size_t)xt.shared * nrow * (2 * nbh);
+  double *dst = part + ((size_t)job * ns + xt.shared) * nrow * (2 * nbh);
 #pragma unroll
   for (int q = 0; q < NC; ++q) {
     const int n = 2 * b0 + 16 * q + li;
@@ -251,13 +263,20 @@ __global__ void __launch_bounds__(64 * NW, 2) k_half_row(Rows rows, const double
 
 // WAVES_OVERLAP + WAVES_1COVERLAP: the NB x NB matrix from the split partials
 // of the real-band product (scaled) and the one-centre runs (c1, c2) of
-// k_overlap1c in z order.  One thread per (row n, super band j): two elements.
+// k_overlap1c in z order.  One thread per (row n, super band j): two elements;
+// blockIdx.y is the matrix.
+struct HalfMats {
+  double *mat[kOvlJobs];
+};
 __global__ void __launch_bounds__(kRedC * kRedS) k_half_finish(const double2 *__restrict__ part, int ns, int nb,
                                                                double scale, const double4 *__restrict__ part1c,
-                                                               int nz, double *mat) {
+                                                               int nz, HalfMats mats) {
   __shared__ double2 red[kRedS][kRedC];
   const int c = threadIdx.x % kRedC, sl = threadIdx.x / kRedC;
   const int nbh = nb / 2, n = nb * nbh, idx = blockIdx.x * kRedC + c;
+  part += (size_t)blockIdx.y * ns * n;
+  if (part1c) part1c += (size_t)blockIdx.y * nz * nbh * nbh;
+  double *mat = mats.mat[blockIdx.y];
   const bool in = idx < n;
   double2 acc = czero();
   if (in) {
@@ -605,24 +624,24 @@ constexpr int kHalfMinChunks = 2;   // K chunks per G split of a row product at 
 // part[split][nrow][2 nbh] = rows x bands; the split count follows the
 // autotuned number of waves (about two per SIMD by default)
 template <int NW, class Rows>
-int run_half_row(pw_waveset *ws, const Rows &rows, int nrow, const double2 *psi, int *ns_out, const char *name) {
+int run_half_row(pw_waveset *ws, const Rows &rows, int nrow, const HalfBands &bands, int *ns_out, const char *name) {
   pw_plan *p = ws->plan;
   const int nbh = ws->nbh, nh = p->nh;
   const int ct = (2 * nbh + 15) / 16;              // blocks of 16 real bands, at most 9 per workgroup
   const int tb = (ct + 8) / 9, nc = (ct + tb - 1) / tb;
   const int tr = (nrow + 16 * NW - 1) / (16 * NW);
   const int chunks = (nh + HK - 1) / HK;
-  const int want = std::max(1, ws->tune_split_waves / NW / std::max(1, tr * tb));
+  const int want = std::max(1, ws->tune_split_waves / NW / std::max(1, tr * tb * bands.n));
   int ns = std::max(1, std::min(want, chunks / kHalfMinChunks));
   const int hsplit = (chunks + ns - 1) / ns * HK;
   ns = (nh + hsplit - 1) / hsplit;
-  PW_TRY(ws_part(ws, (size_t)ns * nrow * 2 * nbh * sizeof(double)));
+  PW_TRY(ws_part(ws, (size_t)bands.n * ns * nrow * 2 * nbh * sizeof(double)));
   {
     ScopeTimer tm(ws, name);
-    const unsigned grid = xcd_blocks(tr * tb, ns);
+    const unsigned grid = xcd_blocks(tr * tb * bands.n, ns);
 #define PW_LAUNCH(NC)                                                                                       \
   case NC:                                                                                                  \
-    k_half_row<Rows, NC, NW><<<grid, 64 * NW, 0, ws->stream>>>(rows, psi, p->d_hg, nh, nrow, p->ngl, nbh,   \
+    k_half_row<Rows, NC, NW><<<grid, 64 * NW, 0, ws->stream>>>(rows, bands, p->d_hg, nh, nrow, p->ngl, nbh,   \
                                                                hsplit, tr, tb, ns, ws->d_part);             \
     break;
     switch (nc) {
@@ -704,7 +723,7 @@ int half_factors(pw_waveset *ws) {
 int half_projections(pw_waveset *ws, const double2 *psi, double2 *proj) {
   RowsP<4> rows{half_p(ws)};
   int ns = 0;
-  PW_TRY(run_half_row<4>(ws, rows, ws->npro, psi, &ns, "projections"));
+  PW_TRY(run_half_row<4>(ws, rows, ws->npro, HalfBands{{psi}, 1}, &ns, "projections"));
   const size_t n = (size_t)ws->npro * ws->nbh;
   ScopeTimer tm(ws, "reduce");
   k_reduce_split<double2><<<(n + kRedC - 1) / kRedC, kRedC * kRedS, 0, ws->stream>>>((const double2 *)ws->d_part, ns,
@@ -713,22 +732,34 @@ int half_projections(pw_waveset *ws, const double2 *psi, double2 *proj) {
   return PW_OK;
 }
 
-// mat = Omega sum conj(c_i) c_j (+ the one-centre runs p1c); a workgroup of
-// three waves when that wastes fewer 16-row blocks than four
-int half_overlap(pw_waveset *ws, const double2 *psi1, const double2 *psi2, const double4 *p1c, int nz, double *mat) {
+// mat = Omega sum conj(c_i) c_j (+ the one-centre runs p1c) for the matrices of
+// jobs; a workgroup of three waves when that wastes fewer 16-row blocks than
+// four.  One launch each for all matrices: they share the reads of the wave
+// functions in an XCD's L2, and a small set's are bound by launches.  The three
+// of a CP step: Si8 13.4 + 9.4 (finishing passes) -> 5.3 + 3.7 us, Si64 (144
+// bands) 108 -> 89 and one finishing pass of 9.8.
+int half_overlap(pw_waveset *ws, const OverlapJob *jobs, int nj, const double4 *p1c, int nz) {
   const int nb = 2 * ws->nbh, mt = (nb + 15) / 16;
-  int ns = 0;
-  if ((mt + 2) / 3 * 3 < (mt + 3) / 4 * 4) {
-    RowsX<3> rows{psi1, ws->plan->ngl, ws->nbh};
-    PW_TRY(run_half_row<3>(ws, rows, nb, psi2, &ns, "overlap"));
-  } else {
-    RowsX<4> rows{psi1, ws->plan->ngl, ws->nbh};
-    PW_TRY(run_half_row<4>(ws, rows, nb, psi2, &ns, "overlap"));
+  HalfBands bands{};
+  HalfMats mats{};
+  bands.n = nj;
+  for (int j = 0; j < nj; ++j) {
+    bands.psi[j] = jobs[j].psi2;
+    mats.mat[j] = jobs[j].mat;
   }
+  auto rows = [&](auto r) {
+    for (int j = 0; j < nj; ++j) r.psis[j] = jobs[j].psi1;
+    r.ngl = ws->plan->ngl;
+    r.nbh = ws->nbh;
+    return r;
+  };
+  int ns = 0;
+  if ((mt + 2) / 3 * 3 < (mt + 3) / 4 * 4) PW_TRY(run_half_row<3>(ws, rows(RowsX<3>{}), nb, bands, &ns, "overlap"));
+  else PW_TRY(run_half_row<4>(ws, rows(RowsX<4>{}), nb, bands, &ns, "overlap"));
   ScopeTimer tm(ws, "reduce");
   const int n = nb * ws->nbh;
-  k_half_finish<<<(n + kRedC - 1) / kRedC, kRedC * kRedS, 0, ws->stream>>>((const double2 *)ws->d_part, ns, nb,
-                                                                            0.5 * ws->plan->vol, p1c, nz, mat);
+  k_half_finish<<<dim3((n + kRedC - 1) / kRedC, nj), kRedC * kRedS, 0, ws->stream>>>(
+      (const double2 *)ws->d_part, ns, nb, 0.5 * ws->plan->vol, p1c, nz, mats);
   PW_HIP(hipGetLastError());
   return PW_OK;
 }

@@ -306,23 +306,38 @@ __global__ void k_unravel_pw(int nbh, int nb, const double2 *t, const double2 *t
 
 // ---------------------------------------------------------------------------
 // one-centre overlap (WAVES_1COVERLAP, src/paw_waves2.f90:856-1022), added to mat
-// c1 = sum_k conj(p1_ki) p2a_kj, c2 = sum_k p1_ki p2a_kj.  The projector index
-// k is split over blockIdx.z in runs of k1c rows; part[z][i][j] = (c1, c2)
-// of the run, summed in z order by k_overlap_finish.
+// c1 = sum_k conj(p1_ki) p2a_kj, c2 = sum_k p1_ki p2a_kj, p2a = DO p2 of each
+// atom, formed while its rows are staged.  The projector index k is split over
+// blockIdx.z in runs of k1c rows, up to kOvlJobs matrices side by side;
+// part[job][z][i][j] = (c1, c2) of the run, summed in z order by the finishing
+// kernels.  Launch-bound: three matrices took six launches with DO p2 in
+// launches of its own, Si8 (10 super bands) 26 us, now 8.9; Si64 (72) 33 -> 15.
 // ---------------------------------------------------------------------------
 constexpr int k1c = 64;
-__global__ void __launch_bounds__(256) k_overlap1c(int npro, int nbh, const double2 *p1, const double2 *p2a,
-                                                   double4 *part) {
+struct Ovl1c {
+  const double2 *p1[kOvlJobs], *p2[kOvlJobs];
+};
+__global__ void __launch_bounds__(256) k_overlap1c(ProjGeo q, int npro, int nbh, int nz, const int2 *tab,
+                                                   const double2 *mats, Ovl1c a, double4 *part) {
   __shared__ double2 sa[k1c][17];
   __shared__ double2 sb[k1c][17];
   const int ti = threadIdx.x / 16, tj = threadIdx.x % 16;
-  const int i0 = blockIdx.x * 16, j0 = blockIdx.y * 16, k0 = blockIdx.z * k1c;
+  const int job = blockIdx.z / nz, k0 = (blockIdx.z - job * nz) * k1c;
+  const int i0 = blockIdx.x * 16, j0 = blockIdx.y * 16;
   const int i = i0 + ti, j = j0 + tj;
+  const double2 *p1 = a.p1[job], *p2 = a.p2[job];
   for (int w = threadIdx.x; w < k1c * 16; w += 256) {
     const int k = w / 16, c = w % 16;
     const bool ok = k0 + k < npro;
     sa[k][c] = (ok && i0 + c < nbh) ? p1[(size_t)(k0 + k) * nbh + i0 + c] : czero();
-    sb[k][c] = (ok && j0 + c < nbh) ? p2a[(size_t)(k0 + k) * nbh + j0 + c] : czero();
+    const int2 t = tab[min(k0 + k, npro - 1)];
+    const int base = q.ipro0[t.x], lmnx = q.lmnx[q.atom_isp[t.x]];
+    const double2 *m = mats + ((size_t)t.x * q.lmnxx + t.y) * q.lmnxx;
+    const double2 *src = p2 + (size_t)base * nbh + min(j0 + c, nbh - 1);
+    double2 s = czero();
+#pragma unroll 8
+    for (int u = 0; u < lmnx; ++u) s = cadd(s, cmul(m[u], src[(size_t)u * nbh]));
+    sb[k][c] = (ok && j0 + c < nbh) ? s : czero();
   }
   __syncthreads();
   double2 c1 = czero(), c2 = czero();
@@ -1894,7 +1909,10 @@ int k_force(pw_waveset *ws, const double2 *psi, const double2 *phase, const doub
 int k_overlap(pw_waveset *ws, const double2 *psi1, const double2 *psi2, double *mat, bool, bool) {
   pw_plan *p = ws->plan;
   const int nbh = ws->nbh, nbhp = (nbh + 15) / 16 * 16;
-  if (ws->prec == PW_PREC_FP64) return half_overlap(ws, psi1, psi2, nullptr, 0, mat);
+  if (ws->prec == PW_PREC_FP64) {
+    const OverlapJob job{psi1, psi2, nullptr, nullptr, mat};
+    return half_overlap(ws, &job, 1, nullptr, 0);
+  }
   double2 *red = nullptr;
   {
     const size_t bytes = runs_bytes(nbh, p->ngl);
@@ -1914,26 +1932,12 @@ int k_overlap(pw_waveset *ws, const double2 *psi1, const double2 *psi2, double *
   return PW_OK;
 }
 
-// mat_dev = WAVES_OVERLAP(psi1, psi2) + WAVES_1COVERLAP(proj1, proj2): the
-// one-centre partials first (DO*proj2 in d_xproj, the partials in the small
-// scratch), then the G-split product with its reduction deferred, then one
-// k_overlap_finish pass (four launches)
-int k_overlap_full(pw_waveset *ws, const double2 *psi1, const double2 *psi2, const double2 *proj1,
-                   const double2 *proj2, double *mat) {
+// one matrix in the mixed form: the G-split product with its reduction
+// deferred, then one k_overlap_finish pass
+static int overlap_mixed(pw_waveset *ws, const OverlapJob &o, const double4 *p1c, int nz) {
   pw_plan *p = ws->plan;
-  ProjGeo q = make_pgeo(ws);
-  const int nbh = ws->nbh, nbhp = (nbh + 15) / 16 * 16, nz = (ws->npro + k1c - 1) / k1c;
-  PW_TRY(ws_small(ws, (size_t)nz * nbh * nbh * sizeof(double4)));
-  double4 *p1c = (double4 *)ws->d_small;
-  {
-    ScopeTimer tm(ws, "overlap1c");
-    k_atom_mat<<<dim3(ws->nat, (ws->lmnxx * nbh + 63) / 64), 64, 0, ws->stream>>>(q, proj2, ws->d_domat,
-                                                                                   ws->d_xproj);
-    dim3 grid((nbh + 15) / 16, (nbh + 15) / 16, nz);
-    k_overlap1c<<<grid, 256, 0, ws->stream>>>(ws->npro, nbh, proj1, ws->d_xproj, p1c);
-    PW_HIP(hipGetLastError());
-  }
-  if (ws->prec == PW_PREC_FP64) return half_overlap(ws, psi1, psi2, p1c, nz, mat);
+  const int nbh = ws->nbh, nbhp = (nbh + 15) / 16 * 16;
+  const double2 *psi1 = o.psi1, *psi2 = o.psi2;
   RowPart rp;
   {
     const size_t bytes = runs_bytes(nbh, p->ngl);
@@ -1950,9 +1954,33 @@ int k_overlap_full(pw_waveset *ws, const double2 *psi1, const double2 *psi2, con
   {
     ScopeTimer tm(ws, "reduce");
     k_overlap_finish<<<(nbh * nbh + kRedC - 1) / kRedC, kRedC * kRedS, 0, ws->stream>>>(
-        rp.part, rp.ns, rp.n, rp.scale, nbh, nbhp, ws->nb, p1c, nz, mat);
+        rp.part, rp.ns, rp.n, rp.scale, nbh, nbhp, ws->nb, p1c, nz, o.mat);
     PW_HIP(hipGetLastError());
   }
+  return PW_OK;
+}
+
+// matrices of one kind: mat = WAVES_OVERLAP(psi1, psi2) + WAVES_1COVERLAP(proj1,
+// proj2), up to kOvlJobs of them: the one-centre partials in one launch (in the
+// small scratch), then the product and its finishing pass, in FP64 one launch
+// each for all matrices
+int k_overlap_full(pw_waveset *ws, const OverlapJob *jobs, int nj) {
+  const int nbh = ws->nbh, nz = (ws->npro + k1c - 1) / k1c;
+  PW_TRY(ws_small(ws, (size_t)nj * nz * nbh * nbh * sizeof(double4)));
+  double4 *p1c = (double4 *)ws->d_small;
+  {
+    ScopeTimer tm(ws, "overlap1c");
+    Ovl1c a{};
+    for (int j = 0; j < nj; ++j) {
+      a.p1[j] = jobs[j].proj1;
+      a.p2[j] = jobs[j].proj2;
+    }
+    dim3 grid((nbh + 15) / 16, (nbh + 15) / 16, nz * nj);
+    k_overlap1c<<<grid, 256, 0, ws->stream>>>(make_pgeo(ws), ws->npro, nbh, nz, ws->d_ipro_tab, ws->d_domat, a, p1c);
+    PW_HIP(hipGetLastError());
+  }
+  if (ws->prec == PW_PREC_FP64) return half_overlap(ws, jobs, nj, p1c, nz);
+  for (int j = 0; j < nj; ++j) PW_TRY(overlap_mixed(ws, jobs[j], p1c + (size_t)j * nz * nbh * nbh, nz));
   return PW_OK;
 }
 

@@ -375,6 +375,18 @@ __host__ __device__ constexpr int fft_lprod(const Fft1D &f, int st) {
   return L;
 }
 
+// threads of the yz passes: kYZ, for the large FP64 planes twice as many.  One
+// such plane fills a CU's LDS (104 KiB for 80 x 80), so the workgroup is all
+// that hides the latency of its stages; with 512 threads a stage of 72 x 72
+// takes two rounds of butterflies, 57 % full, with 1024 one: 72 x 72 planes of
+// 72 super bands 188 -> 178 us (density 98 -> 94), 80 x 80 of 128 307 -> 279;
+// 704 threads (one full round) 183, 281 and 101.  FP32 planes share a CU by
+// threes: 384 and 704 threads are slower there (88 and 94 us against 82).
+template <typename T2, int NY, int NZ>
+constexpr int yz_threads() {
+  return sizeof(T2) == 16 && NY * NZ >= 48 * 48 ? 1024 : kYZ;
+}
+
 template <int N> constexpr int nstage_ct() { return fft_inplace_ct(N).nstage; }
 
 // the plane's scalar lengths as constants
@@ -409,11 +421,12 @@ __host__ __device__ constexpr int tw_off_ct(int n, int st) {
 }
 
 // pencils p = tid mod npen with offsets p * ps (pmap == nullptr) or pmap[p]
-// (a negative entry: no pencil); every thread below (kYZ / npen) npen takes
-// part (npen <= kYZ)
+// (a negative entry: no pencil); every thread below (NT / npen) npen takes
+// part (npen <= NT)
+template <int NT>
 __device__ inline PenSet pen_set(int npen, int ps, const int *pmap) {
   PenSet s;
-  const int t = threadIdx.x, step = npen > 0 ? kYZ / npen : 0;
+  const int t = threadIdx.x, step = npen > 0 ? NT / npen : 0;
   const int q = npen > 0 ? t / npen : 0, p = t - q * npen;
   const int off = npen > 0 && t < step * npen ? (pmap ? pmap[p] : p * ps) : -1;
   if (off >= 0) {
@@ -429,7 +442,7 @@ __device__ inline PenSet pen_set(int npen, int ps, const int *pmap) {
 }
 
 // the stage twiddle table of length N from root[m] = exp(+2 pi i m / N)
-template <typename T2, int N>
+template <typename T2, int N, int NT>
 __device__ inline void tw_table_ct(const T2 *root, T2 *tab) {
   constexpr Fft1D f = fft_inplace_ct(N);
   int off = 0, L = 1;
@@ -437,7 +450,7 @@ __device__ inline void tw_table_ct(const T2 *root, T2 *tab) {
     const int R = f.radix[st];
     L *= R;
     const int cnt = (L / R) * (R - 1);
-    for (int e = threadIdx.x; e < cnt; e += kYZ) {
+    for (int e = threadIdx.x; e < cnt; e += NT) {
       const int j = e / (R - 1), q = e - j * (R - 1) + 1;
       tab[off + e] = root[j * q * (N / L)];
     }
@@ -628,10 +641,10 @@ __device__ inline void dens_reg_store(const Geo &g, int nr3, const double (&accr
 template <typename T2, int NY, int NZ>
 __device__ inline void yz_forward_ct(const Geo &g, const T2 *col, T2 *pl, const PenSet &py, const PenSet &pz,
                                      const T2 *tby, const T2 *tbz) {
-  constexpr int P = NY | 1;
-  for (int i = threadIdx.x; i < P * NZ; i += kYZ) pl[i] = czero<T2>();
+  constexpr int P = NY | 1, NT = yz_threads<T2, NY, NZ>();
+  for (int i = threadIdx.x; i < P * NZ; i += NT) pl[i] = czero<T2>();
   __syncthreads();
-  for (int s = threadIdx.x; s < g.nstripe; s += kYZ) pl[g.stripe_pos[s]] = col[s];
+  for (int s = threadIdx.x; s < g.nstripe; s += NT) pl[g.stripe_pos[s]] = col[s];
   __syncthreads();
   ct_dit<T2, NY, 0, nstage_ct<NY>(), +1, 1>(pl, py, tby);
   ct_dit<T2, NZ, 0, nstage_ct<NZ>() - 1, +1, P>(pl, pz, tbz);
@@ -743,16 +756,17 @@ __device__ inline void dens_reg_store_ct(const PenSet &pz, const double (&accr)[
 template <int NY, int NZ>
 constexpr bool dens_reg_ct() {
   constexpr Fft1D f = fft_inplace_ct(NZ);
-  return f.radix[f.nstage - 1] <= kRegR && NZ / f.radix[f.nstage - 1] <= 2 * (kYZ / NY);
+  return f.radix[f.nstage - 1] <= kRegR && NZ / f.radix[f.nstage - 1] <= 2 * (kYZ / NY);   // (of kYZ threads: more have fewer each)
 }
 
 // ---- yz pass of WAVES_VPSI: psi(x,y,z) * V(r), back to the stripes ----------------
 // One workgroup per (x, band); vt = V as [x][z][y] in the work precision.
 template <typename T2, bool BIG, int NY = 0, int NZ = 0>
-__global__ void __launch_bounds__(kYZ) k_yz_vpsi(Geo g, Fft1D fy, Fft1D fz, const T2 *twy, const T2 *twz,
+__global__ void __launch_bounds__((yz_threads<T2, NY, NZ>())) k_yz_vpsi(Geo g, Fft1D fy, Fft1D fz, const T2 *twy, const T2 *twz,
                                                  T2 *stripes, const typename Prec<T2>::T *vt) {
   typedef typename Prec<T2>::T T;
   yz_fix<NY, NZ>(g);
+  constexpr int NT = yz_threads<T2, NY, NZ>();
   extern __shared__ unsigned char smem_raw[];
   const int n23 = g.nr2 * g.nr3;
   T2 *pl = reinterpret_cast<T2 *>(smem_raw);
@@ -761,9 +775,9 @@ __global__ void __launch_bounds__(kYZ) k_yz_vpsi(Geo g, Fft1D fy, Fft1D fz, cons
   T2 *col = stripes + ((size_t)band * g.nr1 + x) * g.nstripe;
   const T *vx = vt + (size_t)x * n23;
   if constexpr (NY > 0 && NZ > 0) {
-    tw_table_ct<T2, NY>(twy, ty);
-    tw_table_ct<T2, NZ>(twz, tz);
-    const PenSet py = pen_set(g.nypen, 0, g.ypen), pz = pen_set(NY, 1, nullptr);
+    tw_table_ct<T2, NY, NT>(twy, ty);
+    tw_table_ct<T2, NZ, NT>(twz, tz);
+    const PenSet py = pen_set<NT>(g.nypen, 0, g.ypen), pz = pen_set<NT>(NY, 1, nullptr);
     yz_forward_ct<T2, NY, NZ>(g, col, pl, py, pz, ty, tz);
     z_last_vpsi_ct<T2, NY, NZ>(pl, pz, tz, vx);
     ct_dif<T2, NZ, nstage_ct<NZ>() - 2, -1, NY | 1>(pl, pz, tz);
@@ -780,7 +794,7 @@ __global__ void __launch_bounds__(kYZ) k_yz_vpsi(Geo g, Fft1D fy, Fft1D fz, cons
     fft_dif<T2, BIG>(pl, fz, fz.nstage - 1, g.nr2, g.mnr2, g.pitch, 1, nullptr, tz, -1, true);
     fft_dif<T2, BIG>(pl, fy, fy.nstage, g.nzp, g.mnzp, 1, 0, zpos, ty, -1, true);
   }
-  for (int s = threadIdx.x; s < g.nstripe; s += kYZ) col[s] = pl[g.stripe_pos[s]];
+  for (int s = threadIdx.x; s < g.nstripe; s += NT) col[s] = pl[g.stripe_pos[s]];
 }
 
 // ---- yz pass of WAVES_DENSITY: sum over a group of bands ----------------------
@@ -790,11 +804,12 @@ __global__ void __launch_bounds__(kYZ) k_yz_vpsi(Geo g, Fft1D fy, Fft1D fz, cons
 template <typename T2, bool REG> struct DensWaves { static constexpr int v = 1; };
 template <> struct DensWaves<float2, true> { static constexpr int v = 4; };
 template <typename T2, bool BIG, bool REG, int NY = 0, int NZ = 0>
-__global__ void __launch_bounds__(kYZ) __attribute__((amdgpu_waves_per_eu(DensWaves<T2, REG>::v))) k_yz_dens(Geo g, Fft1D fy, Fft1D fz, const T2 *twy, const T2 *twz,
+__global__ void __launch_bounds__((yz_threads<T2, NY, NZ>())) __attribute__((amdgpu_waves_per_eu(DensWaves<T2, REG>::v))) k_yz_dens(Geo g, Fft1D fy, Fft1D fz, const T2 *twy, const T2 *twz,
                                                  const T2 *stripes, int nb, int bpg, const double *occ2,
                                                  double *part) {
   static_assert(!(REG && BIG), "the register band sum takes radices up to kRegR");
   yz_fix<NY, NZ>(g);
+  constexpr int NT = yz_threads<T2, NY, NZ>();
   extern __shared__ unsigned char smem_raw[];
   const int n23 = g.nr2 * g.nr3;
   double *acc = reinterpret_cast<double *>(smem_raw);
@@ -810,12 +825,12 @@ __global__ void __launch_bounds__(kYZ) __attribute__((amdgpu_waves_per_eu(DensWa
   const int bstart = grp * bpg, bend = min(nb, bstart + bpg);
   double *dst = part + ((size_t)grp * g.nr1 + x) * n23;
   if (!REG)
-    for (int i = threadIdx.x; i < n23; i += kYZ) acc[i] = 0.0;
+    for (int i = threadIdx.x; i < n23; i += NT) acc[i] = 0.0;
   if constexpr (NY > 0 && NZ > 0) {
     if constexpr (!REG || dens_reg_ct<NY, NZ>()) {
-      tw_table_ct<T2, NY>(twy, ty);
-      tw_table_ct<T2, NZ>(twz, tz);
-      const PenSet py = pen_set(g.nypen, 0, g.ypen), pz = pen_set(NY, 1, nullptr);
+      tw_table_ct<T2, NY, NT>(twy, ty);
+      tw_table_ct<T2, NZ, NT>(twz, tz);
+      const PenSet py = pen_set<NT>(g.nypen, 0, g.ypen), pz = pen_set<NT>(NY, 1, nullptr);
       for (int band = bstart; band < bend; ++band) {
         const double s1 = occ2[2 * band], s2 = occ2[2 * band + 1];
         if (s1 == 0.0 && s2 == 0.0) continue;   // uniform across the workgroup
@@ -855,7 +870,7 @@ __global__ void __launch_bounds__(kYZ) __attribute__((amdgpu_waves_per_eu(DensWa
   }
   if constexpr (!REG) {
     __syncthreads();
-    for (int i = threadIdx.x; i < n23; i += kYZ) dst[i] = acc[i];
+    for (int i = threadIdx.x; i < n23; i += NT) dst[i] = acc[i];
   }
 }
 
@@ -1096,7 +1111,7 @@ int vpsi_t(pw_plan *p, int nb, const double2 *psi, const double *v, double2 *hps
     PW_TRY(with_yz(p, [&](auto ny, auto nz) -> int {
       constexpr int NY = decltype(ny)::value, NZ = decltype(nz)::value;
       PW_TRY(yz_lds(k_yz_vpsi<T2, false, NY, NZ>, lds));
-      k_yz_vpsi<T2, false, NY, NZ><<<dim3(p->nr1, nb), kYZ, lds, s>>>(
+      k_yz_vpsi<T2, false, NY, NZ><<<dim3(p->nr1, nb), yz_threads<T2, NY, NZ>(), lds, s>>>(
           g, p->fyz[0], p->fyz[1], twid<T2>(p, 1), twid<T2>(p, 2), (T2 *)p->d_stripe_buf, (const T *)p->d_vt);
       return PW_OK;
     }));
@@ -1129,20 +1144,20 @@ int density_t(pw_plan *p, int nb, const double2 *psi, const double *occ2, double
     PW_HIP(hipMalloc(&p->d_dens_part, need));
     p->dens_bytes = need;
   }
-#define PW_DENS(BIG, REG, ...)                                                                             \
+#define PW_DENS(TH, BIG, REG, ...)                                                                          \
   do {                                                                                                     \
     PW_TRY(yz_lds(k_yz_dens<T2, BIG, REG, ##__VA_ARGS__>, lds));                                           \
-    k_yz_dens<T2, BIG, REG, ##__VA_ARGS__><<<dim3(p->nr1, ngrp), kYZ, lds, s>>>(g, p->fyz[0], p->fyz[1], twid<T2>(p, 1),  \
-                                                                 twid<T2>(p, 2), (const T2 *)p->d_stripe_buf, \
-                                                                 nb, bpg, occ2, (double *)p->d_dens_part);  \
+    k_yz_dens<T2, BIG, REG, ##__VA_ARGS__><<<dim3(p->nr1, ngrp), TH, lds, s>>>(                            \
+        g, p->fyz[0], p->fyz[1], twid<T2>(p, 1), twid<T2>(p, 2), (const T2 *)p->d_stripe_buf, nb, bpg,     \
+        occ2, (double *)p->d_dens_part);                                                                   \
   } while (0)
   if (yz_big(p)) {
-    PW_DENS(true, false);
+    PW_DENS(kYZ, true, false);
   } else {
     PW_TRY(with_yz(p, [&](auto ny, auto nz) -> int {
-      constexpr int NY = decltype(ny)::value, NZ = decltype(nz)::value;
-      if (reg) PW_DENS(false, true, NY, NZ);
-      else PW_DENS(false, false, NY, NZ);
+      constexpr int NY = decltype(ny)::value, NZ = decltype(nz)::value, TH = yz_threads<T2, NY, NZ>();
+      if (reg) PW_DENS(TH, false, true, NY, NZ);
+      else PW_DENS(TH, false, false, NY, NZ);
       return PW_OK;
     }));
   }

@@ -309,7 +309,7 @@ struct pw_waveset {
   std::vector<double> hfac_pos;
   bool hfac_valid = false;
   bool pro_sym = true;
-  int4 *d_ipro4 = nullptr;     // per projector: F row, atom, l, 0
+  int4 *d_ipro4 = nullptr;     // per projector: offsets of its rows in F and E of d_hfac, l mod 2, 0
   double2 *d_phase = nullptr;  // nat*3*(2*nmaxx+1)
   int nphase = 0;              // 2*nmaxx+1
   std::vector<double> phase_pos;   // positions of the tables in d_phase

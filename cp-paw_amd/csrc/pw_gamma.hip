@@ -14,9 +14,12 @@
 // FP64 MFMA bound: 3.5 GFLOP per projector product at Si64 (512 projectors,
 // 144 bands, 23 847 G) is 48 us at the rate of a large FP64 product.  Measured
 // there against the complex products over the whole sphere: projections 287
-// -> 88 us, ADDPRO 328 -> 107, forces 272 -> 96, one band overlap 109 -> 36,
-// ADDOPSI 101 -> 39.  The rest is the staging between the MFMAs (LDS stores
-// and one barrier per 16 K) and the G-split partial sums.
+// -> 79 us, ADDPRO 328 -> 101, forces 272 -> 87, the three band overlaps of a
+// step 327 -> 82, ADDOPSI 101 -> 37.  The rest is the staging between the MFMAs:
+// the matrix units are busy 50 to 62 % of the time and vector instructions take
+// 13 to 20 %, which do not overlap.  With selects on every load, 64-bit products
+// in the addresses and (-i)^l by a switch the same kernels took 88, 107, 96, 89
+// and 39 us.
 #include <algorithm>
 
 #include "pw_device.h"
@@ -31,13 +34,20 @@ constexpr int HKR = 2 * HK;  // real K of a staged chunk
 // stores (one column, rows hh) spread over the banks
 constexpr int hpad(int w) { return w + ((17 - w % 32) + 32) % 32; }
 
-// Projector factors on the half list, P(i,h) = (-i)^l F(k,h) E(atom,h)
+// Projector factors on the half list, P(i,h) = (-i)^(l mod 2) F(k,h) E(atom,h);
+// F carries the sign of the even power, (-1)^(l/2)
 struct HalfP {
   const double *f;     // [NSP*LMNXX][NHP]
   const double2 *e;    // [NAT][NHP]
-  const int4 *tab;     // per projector: F row, atom, l, 0
+  const int4 *tab;     // per projector: offsets of its F and E rows, l mod 2, 0
   int npro, nhp;
+  __device__ const double *frow(int4 t) const { return f + (unsigned)t.x; }
+  __device__ const double2 *erow(int4 t) const { return e + (unsigned)t.y; }
 };
+// z (-i)^odd
+__device__ inline double2 rot_odd(double2 z, int odd) {
+  return make_double2(odd ? z.y : z.x, odd ? -z.x : z.y);
+}
 
 __global__ void k_half_f(ProjGeo q, int nsp, int nh, int nhp, const int2 *__restrict__ hg, double *f) {
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -48,6 +58,7 @@ __global__ void k_half_f(ProjGeo q, int nsp, int nh, int nhp, const int2 *__rest
   if (h < nh && lmn < q.lmnx[isp]) {
     const int ig = hg[h].x;
     v = q.ylm[(size_t)q.lmn_lm[k] * q.ngl + ig] * q.pro[(size_t)(q.ibpro[isp] + q.lmn_ln[k]) * q.ngl + ig];
+    if (q.lmn_l[k] & 2) v = -v;
   }
   f[idx] = v;
 }
@@ -59,24 +70,29 @@ __global__ void k_half_e(ProjGeo q, int nh, int nhp, const int2 *__restrict__ hg
   e[idx] = h < nh ? eigr_of(q, atom, hg[h].x) : czero();
 }
 
-// psi of one super band at (G, -G) -> s and d; the self pair G = 0 has s = psi, d = 0
+// psi of one super band at (G, -G).  The loads are unconditional (clamped
+// indices): what is out of range meets a zero of the other operand or enters
+// elements that are not written.  On these kernels every vector instruction
+// counts: the FP64 matrix instructions keep the SIMD unit from issuing others,
+// and matrix and vector time added up to 72 % in all of them.
 struct Pair {
   double2 p, m;
 };
-__device__ inline void load_pair(const double2 *__restrict__ psi, size_t off, int2 g, bool ok, Pair &v) {
-  v.p = ok ? psi[off + g.x] : czero();
-  v.m = (ok && g.x != g.y) ? psi[off + g.y] : czero();
+__device__ inline void load_pair(const double2 *__restrict__ psi, size_t off, int2 g, Pair &v) {
+  v.p = psi[off + g.x];
+  v.m = psi[off + g.y];
 }
-// the rows (re, im) of the two real bands: a = 2 c1, b = 2 c2
+// the rows (re, im) of the two real bands: a = 2 c1, b = 2 c2; at the self pair
+// G = 0 twice that, which the other operand makes good
 struct Bands2 {
   double are, aim, bre, bim;
 };
-__device__ inline Bands2 split_pair(const Pair &v, bool self) {
+__device__ inline Bands2 split_pair(const Pair &v) {
   Bands2 r;
   r.are = v.p.x + v.m.x;
   r.bre = v.p.y + v.m.y;
-  r.aim = self ? 0.0 : v.p.y - v.m.y;
-  r.bim = self ? 0.0 : v.m.x - v.p.x;
+  r.aim = v.p.y - v.m.y;
+  r.bim = v.m.x - v.p.x;
   return r;
 }
 
@@ -93,8 +109,7 @@ struct RowsP {
   struct Row {
     const double *f[2];
     const double2 *e[2];
-    int l[2];
-    bool ok[2];
+    int odd[2];
   };
   struct Pre {
     double f[2];
@@ -104,15 +119,14 @@ struct RowsP {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int r = r0 + (threadIdx.x >> 3) + 8 * NW * i;
-      w.ok[i] = r < p.npro;
-      const int4 t = p.tab[w.ok[i] ? r : 0];
-      w.f[i] = p.f + (size_t)t.x * p.nhp;
-      w.e[i] = p.e + (size_t)t.y * p.nhp;
-      w.l[i] = t.z;
+      const int4 t = p.tab[min(r, p.npro - 1)];
+      w.f[i] = p.frow(t);
+      w.e[i] = p.erow(t);
+      w.odd[i] = t.z;
     }
   }
   // h < NHP: the tables are zero beyond NH
-  __device__ void fetch(const Row &w, int h, int2, bool, Pre &v) const {
+  __device__ void fetch(const Row &w, int h, int2, Pre &v) const {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       v.f[i] = w.f[i][h];
@@ -120,13 +134,13 @@ struct RowsP {
     }
   }
   template <int SA>
-  __device__ void store(const Row &w, const Pre &v, bool, double (*sA)[SA]) const {
+  __device__ void store(const Row &w, const Pre &v, bool self, bool, double (*sA)[SA]) const {
     const int hh = threadIdx.x & 7;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int r = (threadIdx.x >> 3) + 8 * NW * i;
-      const double s = w.ok[i] ? v.f[i] : 0.0;
-      const double2 z = rot_mil(make_double2(s * v.e[i].x, s * v.e[i].y), w.l[i]);
+      const double s = self ? 0.5 * v.f[i] : v.f[i];
+      const double2 z = rot_odd(make_double2(s * v.e[i].x, s * v.e[i].y), w.odd[i]);
       sA[hh][r] = z.x;
       sA[HK + hh][r] = z.y;
     }
@@ -134,8 +148,9 @@ struct RowsP {
 };
 
 // 16 NW real bands of psi (8 NW super bands), one (super band, hh) per
-// thread; the G = 0 term counts twice: sum over the pairs of A X is then
-// 2 sum over the sphere of conj(c) c'
+// thread; the G = 0 term counts twice (both operands hold twice their bands
+// there, hence the half): sum over the pairs of A X is then 2 sum over the
+// sphere of conj(c) c'.  Zero beyond the split's pairs.
 template <int NW>
 struct RowsX {
   const double2 *psis[kOvlJobs];
@@ -144,26 +159,23 @@ struct RowsX {
   __device__ void job(int j) { psi = psis[j]; }
   struct Row {
     size_t off;
-    bool ok;
   };
   struct Pre {
     Pair v;
   };
   __device__ void init(Row &w, int r0) const {
-    const int b = r0 / 2 + (threadIdx.x >> 3);
-    w.ok = b < nbh;
-    w.off = (size_t)(w.ok ? b : 0) * ngl;
+    w.off = (size_t)min(r0 / 2 + (int)(threadIdx.x >> 3), nbh - 1) * ngl;
   }
-  __device__ void fetch(const Row &w, int, int2 g, bool in, Pre &p) const { load_pair(psi, w.off, g, w.ok && in, p.v); }
+  __device__ void fetch(const Row &w, int, int2 g, Pre &p) const { load_pair(psi, w.off, g, p.v); }
   template <int SA>
-  __device__ void store(const Row &, const Pre &p, bool self, double (*sA)[SA]) const {
+  __device__ void store(const Row &, const Pre &p, bool self, bool in, double (*sA)[SA]) const {
     const int hh = threadIdx.x & 7, n = 2 * (threadIdx.x >> 3);
-    const Bands2 r = split_pair(p.v, self);
-    const double w = self ? 2.0 : 1.0;
+    const Bands2 r = split_pair(p.v);
+    const double w = in ? (self ? 0.5 : 1.0) : 0.0;
     sA[hh][n] = w * r.are;
     sA[hh][n + 1] = w * r.bre;
-    sA[HK + hh][n] = r.aim;
-    sA[HK + hh][n + 1] = r.bim;
+    sA[HK + hh][n] = w * r.aim;
+    sA[HK + hh][n + 1] = w * r.bim;
   }
 };
 
@@ -201,25 +213,24 @@ __global__ void __launch_bounds__(64 * NW, 2) k_half_row(Rows rows, HalfBands ba
   rows.init(rw, r0);
   typename Rows::Pre pa;
   Pair pb[NBT];
+  size_t off[NBT];
+#pragma unroll
+  for (int i = 0; i < NBT; ++i) off[i] = (size_t)min(b0 + min((t >> 3) + 8 * NW * i, 8 * NC - 1), nbh - 1) * ngl;
   // index of chunk c for this thread's hh (clamped into the half list)
   auto idx = [&](int c) { return hg[min(h0 + c * HK + hh, nh - 1)]; };
   auto fetch = [&](int c, int2 g) {
-    const int h = h0 + c * HK + hh;
-    const bool in = h < h1;
-    rows.fetch(rw, h, g, in, pa);
+    rows.fetch(rw, h0 + c * HK + hh, g, pa);
 #pragma unroll
-    for (int i = 0; i < NBT; ++i) {
-      const int bl = (t >> 3) + 8 * NW * i, b = b0 + bl;
-      load_pair(psi, (size_t)min(b, nbh - 1) * ngl, g, in && bl < 8 * NC && b < nbh, pb[i]);
-    }
+    for (int i = 0; i < NBT; ++i) load_pair(psi, off[i], g, pb[i]);
   };
-  auto store = [&](int buf, bool self) {
-    rows.store(rw, pa, self, sA[buf]);
+  auto store = [&](int c, bool self) {
+    const int buf = c & 1;
+    rows.store(rw, pa, self, h0 + c * HK + hh < h1, sA[buf]);
 #pragma unroll
     for (int i = 0; i < NBT; ++i) {
       const int bl = (t >> 3) + 8 * NW * i;
       if (NC % NW != 0 && bl >= 8 * NC) break;
-      const Bands2 r = split_pair(pb[i], self);
+      const Bands2 r = split_pair(pb[i]);
       sB[buf][hh][2 * bl] = r.are;
       sB[buf][hh][2 * bl + 1] = r.bre;
       sB[buf][HK + hh][2 * bl] = r.aim;
@@ -247,7 +258,7 @@ __global__ void __launch_bounds__(64 * NW, 2) k_half_row(Rows rows, HalfBands ba
 #pragma unroll
       for (int q = 0; q < NC; ++q) acc[q] = mfma4(av, b[k][16 * q + li], acc[q]);
     }
-    if (more) store((c + 1) & 1, self);
+    if (more) store(c + 1, self);
   }
   double *dst = part + ((size_t)job * ns + xt.shared) * nrow * (2 * nbh);
 #pragma unroll
@@ -336,23 +347,22 @@ struct PlaneP {
   struct Pre {
     double f;
     double2 e;
-    int l;
+    int odd;
   };
   __device__ int4 entry(int k0) const {
-    const int k = k0 + ((threadIdx.x & 255) >> 4);
-    const int4 t = p.tab[min(k, p.npro - 1)];
-    return make_int4(t.x, t.y, t.z, k < p.npro);
+    return p.tab[min(k0 + (int)((threadIdx.x & 255) >> 4), p.npro - 1)];
   }
-  __device__ void fetch(int4 t, int, int h, int2, bool, Pre &v) const {
-    v.f = t.w ? p.f[(size_t)t.x * p.nhp + h] : 0.0;
-    v.e = p.e[(size_t)t.y * p.nhp + h];
-    v.l = t.z;
+  __device__ void fetch(int4 t, int, int h, int2, Pre &v) const {
+    v.odd = t.z;
+    if (threadIdx.x >= 256) return;               // whole waves (124 -> 101 us for Si64)
+    v.f = p.frow(t)[h];
+    v.e = p.erow(t)[h];
   }
   template <int SB>
-  __device__ void store(const Pre &v, bool, double (*re)[SB], double (*im)[SB]) const {
+  __device__ void store(const Pre &v, double (*re)[SB], double (*im)[SB]) const {
     const int t = threadIdx.x;
     if (t >= 256) return;
-    const double2 z = rot_mil(make_double2(v.f * v.e.x, v.f * v.e.y), v.l);
+    const double2 z = rot_odd(make_double2(v.f * v.e.x, v.f * v.e.y), v.odd);
     re[t >> 4][t & 15] = z.x;
     im[t >> 4][t & 15] = z.y;
   }
@@ -366,19 +376,18 @@ struct PlaneX {
     Pair v;
   };
   __device__ int4 entry(int) const { return make_int4(0, 0, 0, 0); }
-  __device__ void fetch(int4, int k0, int, int2 g, bool in, Pre &p) const {
+  __device__ void fetch(int4, int k0, int, int2 g, Pre &p) const {
     const int b = k0 / 2 + ((threadIdx.x & 127) >> 4);
-    load_pair(chi, (size_t)min(b, nbh - 1) * ngl, g, in && b < nbh, p.v);
+    load_pair(chi, (size_t)min(b, nbh - 1) * ngl, g, p.v);
   }
   template <int SB>
-  __device__ void store(const Pre &p, bool self, double (*re)[SB], double (*im)[SB]) const {
+  __device__ void store(const Pre &p, double (*re)[SB], double (*im)[SB]) const {
     const int t = threadIdx.x, k = 2 * (t >> 4), h = t & 15;
     if (t >= 128) return;
-    // the real bands c = half the sums, at G = 0 the sum itself
-    const Bands2 r = split_pair(p.v, self);
-    const double w = self ? 1.0 : 0.5;
-    re[k][h] = w * r.are;
-    re[k + 1][h] = w * r.bre;
+    // the real bands c = half the sums
+    const Bands2 r = split_pair(p.v);
+    re[k][h] = 0.5 * r.are;
+    re[k + 1][h] = 0.5 * r.bre;
     im[k][h] = 0.5 * r.aim;
     im[k + 1][h] = 0.5 * r.bim;
   }
@@ -404,37 +413,36 @@ __global__ void __launch_bounds__(1024) k_half_col(Plane pl, const double2 *__re
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6, li = lane & 15, lk = lane >> 4;
   const int h0 = blockIdx.x * 16, b0 = blockIdx.y * 8 * nt, nw = 8 * nt;
   const int hs = h0 + (t & 15);
-  const bool hin = hs < nh;
   const int2 g = hg[min(hs, nh - 1)];
-  const bool self = g.x == g.y;
   // this thread's coefficients: element e = t + i blockDim of the chunk's 16 x nw
   constexpr int NA = 2 * RTW;
-  int ka[NA], ba[NA];
-  bool oka[NA];
+  // (those of rows beyond nk are zero, those of bands beyond nbh go unused),
+  // its place in the row and in LDS
+  int ka[NA], da[NA], oa[NA];
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
     const int e = t + i * blockDim.x;
     ka[i] = e / nw;
-    ba[i] = e - ka[i] * nw;
-    oka[i] = ka[i] < 16 && b0 + ba[i] < nbh;
+    const int bl = e - ka[i] * nw;
+    oa[i] = (ka[i] & 15) * nbh + min(b0 + bl, nbh - 1);
+    da[i] = ka[i] * SA + 16 * (bl >> 3) + (bl & 3) + ((bl >> 2) & 1) * 8;
   }
   double2 va[NA];
   typename Plane::Pre pre;
   auto fetch = [&](int k0, int4 ent) {
-    pl.fetch(ent, k0, hs, g, hin, pre);
+    pl.fetch(ent, k0, hs, g, pre);
+    const double2 *xc = x + (size_t)k0 * nbh;
 #pragma unroll
-    for (int i = 0; i < NA; ++i)
-      va[i] = (oka[i] && k0 + ka[i] < nk) ? x[(size_t)(k0 + ka[i]) * nbh + b0 + ba[i]] : czero();
+    for (int i = 0; i < NA; ++i) va[i] = k0 + ka[i] < nk ? xc[oa[i]] : czero();
   };
   auto store = [&](int buf) {
-    pl.store(pre, self, sRe + 16 * buf, sIm + 16 * buf);
+    pl.store(pre, sRe + 16 * buf, sIm + 16 * buf);
+    double *d = sA + buf * 16 * SA;
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
       if (ka[i] >= 16) continue;
-      const int bl = ba[i];
-      double *d = sA + ((size_t)buf * 16 + ka[i]) * SA + 16 * (bl >> 3) + (bl & 3) + ((bl >> 2) & 1) * 8;
-      d[0] = va[i].x;
-      d[4] = va[i].y;
+      d[da[i]] = va[i].x;
+      d[da[i] + 4] = va[i].y;
     }
   };
   dbl4 ar[RTW], ai[RTW];
@@ -512,24 +520,26 @@ __global__ void __launch_bounds__(64 * kFW, 2) k_half_force(HalfP p, const doubl
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6, li = lane & 15, lk = lane >> 4;
   const int r0 = xt.inner * WR, h0 = xt.shared * WH;
   const int hb = t & (WH - 1), bb = t / WH;               // band operand: (pair, super band of the chunk)
-  const int hs = h0 + hb;
-  const int2 g = hg[min(hs, nh - 1)];
-  const bool self = g.x == g.y, hin = hs < nh;
+  const int2 g = hg[min(h0 + hb, nh - 1)];              // (the columns beyond NH and the term G = 0 get no weight)
   constexpr int NA = WR * 8 / (64 * kFW);
   const int ba = t & 7;
+  const double2 *da[NA];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) da[i] = ded + (size_t)min(r0 + (t >> 3) + 8 * kFW * i, p.npro - 1) * nbh;
   double2 va[NA];
   Pair pb;
   auto fetch = [&](int c) {
-    const int b = 8 * c + bb;
-    load_pair(psi, (size_t)min(b, nbh - 1) * ngl, g, hin && b < nbh, pb);
+    load_pair(psi, (size_t)min(8 * c + bb, nbh - 1) * ngl, g, pb);
+    const int bk = 8 * c + ba, bc = min(bk, nbh - 1);
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      const int r = r0 + (t >> 3) + 8 * kFW * i, bk = 8 * c + ba;
-      va[i] = (r < p.npro && bk < nbh) ? ded[(size_t)r * nbh + bk] : czero();
+    for (int i = 0; i < NA; ++i) va[i] = da[i][bc];
+    if (bk >= nbh) {                                      // rows of the contraction beyond the bands
+#pragma unroll
+      for (int i = 0; i < NA; ++i) va[i] = czero();
     }
   };
   auto store = [&](int buf) {
-    const Bands2 x = split_pair(pb, self);
+    const Bands2 x = split_pair(pb);
     sRe[buf][2 * bb][hb] = x.are;
     sRe[buf][2 * bb + 1][hb] = x.bre;
     sIm[buf][2 * bb][hb] = x.aim;
@@ -597,9 +607,9 @@ __global__ void __launch_bounds__(64 * kFW, 2) k_half_force(HalfP p, const doubl
 #pragma unroll
         for (int q = 0; q < kFHT; ++q) {
           const int h = h0 + 16 * q + li;                 // < NHP: zero tables beyond NH
-          const double s = p.f[(size_t)tb.x * p.nhp + h];
-          const double2 e = p.e[(size_t)tb.y * p.nhp + h];
-          const double2 pv = rot_mil(make_double2(s * e.x, s * e.y), tb.z);
+          const double s = p.frow(tb)[h];
+          const double2 e = p.erow(tb)[h];
+          const double2 pv = rot_odd(make_double2(s * e.x, s * e.y), tb.z);
           // Re(i p conj(d)) = p.x d.y - p.y d.x
           const double cc = pv.x * ai[rt][q][r] - pv.y * ar[rt][q][r];
           f[0] += cc * gx[q];
@@ -737,7 +747,7 @@ int half_projections(pw_waveset *ws, const double2 *psi, double2 *proj) {
 // four.  One launch each for all matrices: they share the reads of the wave
 // functions in an XCD's L2, and a small set's are bound by launches.  The three
 // of a CP step: Si8 13.4 + 9.4 (finishing passes) -> 5.3 + 3.7 us, Si64 (144
-// bands) 108 -> 89 and one finishing pass of 9.8.
+// bands) 108 -> 82 and one finishing pass of 9.8.
 int half_overlap(pw_waveset *ws, const OverlapJob *jobs, int nj, const double4 *p1c, int nz) {
   const int nb = 2 * ws->nbh, mt = (nb + 15) / 16;
   HalfBands bands{};

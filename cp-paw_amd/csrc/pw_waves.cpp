@@ -459,11 +459,12 @@ extern "C" int pw_waves_create(pw_plan *plan, int nb, int nat, int nsp, const in
   up(&ws->d_lmn_l, ws->lmn_l);
   {
     std::vector<int> tab, tab4;
+    const size_t nhp = half_pad(plan);   // 32-bit offsets: see the check in setr8a PRO
     for (int a = 0; a < nat; ++a)
       for (int l = 0; l < ws->lmnx[ws->isp[a]]; ++l) {
         const int k = ws->isp[a] * ws->lmnxx + l;
         tab.insert(tab.end(), {a, l});
-        tab4.insert(tab4.end(), {k, a, ws->lmn_l[k], 0});
+        tab4.insert(tab4.end(), {(int)(unsigned)(k * nhp), (int)(unsigned)(a * nhp), ws->lmn_l[k] & 1, 0});
       }
     up((int **)&ws->d_ipro_tab, tab);
     up((int **)&ws->d_ipro4, tab4);
@@ -609,8 +610,9 @@ extern "C" int pw_waves_setr8a(pw_waveset *ws, const char *id, int len, const do
     PW_HIP(hipMemcpy(ws->d_pro, val, (size_t)len * sizeof(double), hipMemcpyHostToDevice));
     ws->pfac_valid = false;
     ws->hfac_valid = false;
-    // radial tables have PRO(G) = PRO(-G) (to the rounding of |G|)
-    ws->pro_sym = true;
+    // radial tables have PRO(G) = PRO(-G) (to the rounding of |G|); the factor
+    // tables on the G pairs take 32-bit row offsets
+    ws->pro_sym = (size_t)std::max(ws->nat, ws->nsp * ws->lmnxx) * half_pad(p) <= 0xffffffffull;
     for (int k = 0; k < ws->nbarepro && ws->pro_sym; ++k) {
       const double *row = val + (size_t)k * p->ngl;
       for (const int2 &h : p->hg) {

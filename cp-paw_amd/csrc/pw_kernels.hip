@@ -460,15 +460,19 @@ __device__ inline void fold_lambda(const double *lam, int nb, int i, int j, doub
 // on the device): A(i,k) in lane i + 16(k/8), element k%8; B(k,j) in lane
 // j + 16(k/8), element k%8; C(i,j) in lane j + 16(i/4), element i%4.
 // Operands live in LDS as six planes (re h,m,l, im h,m,l), K contiguous per
-// row/column, rows padded to 80 B so that the 16-byte operand reads of 16
-// lanes cover all 64 banks once.
+// row/column, rows of 64 B with their 16-byte runs swapped by the row index
+// (plane_slot).
 // ---------------------------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int KB = 32;        // K of one MFMA = K of one staged chunk
-constexpr int KBP = KB + 8;   // LDS row stride in bf16
+constexpr int KBP = KB;       // LDS row stride in bf16
+// the four runs of a row swapped by the row: half of the LDS cycles of the
+// padded rows were bank conflicts, Si64 projections 56.4 -> 54.7 us, ADDPRO 79.2
+// -> 77.0, forces 97.3 -> 93.6
+__device__ inline int plane_slot(int row, int k8) { return 8 * (k8 ^ ((row >> 1) & 3)); }
 constexpr int NPL = 6;        // planes per complex operand
 
 __device__ inline flt4 mfma_bf(const bf16x8 &a, const bf16x8 &b, flt4 c) {
@@ -552,12 +556,12 @@ __device__ inline void cmfma_bf_nb(flt4 &cr, flt4 &ci, const bf16x8 *a, const bf
 
 __device__ inline void store_planes(__bf16 (*pl)[KBP], int plane_rows, int row, int k8, const Planes8 &v) {
 #pragma unroll
-  for (int q = 0; q < NPL; ++q) *reinterpret_cast<bf16x8 *>(&pl[q * plane_rows + row][8 * k8]) = v.p[q];
+  for (int q = 0; q < NPL; ++q) *reinterpret_cast<bf16x8 *>(&pl[q * plane_rows + row][plane_slot(row, k8)]) = v.p[q];
 }
 
 __device__ inline void load_planes(const __bf16 (*pl)[KBP], int plane_rows, int row, int k8, bf16x8 *v) {
 #pragma unroll
-  for (int q = 0; q < NPL; ++q) v[q] = *reinterpret_cast<const bf16x8 *>(&pl[q * plane_rows + row][8 * k8]);
+  for (int q = 0; q < NPL; ++q) v[q] = *reinterpret_cast<const bf16x8 *>(&pl[q * plane_rows + row][plane_slot(row, k8)]);
 }
 
 // Projector functions of the mixed form from two factor tables,
@@ -867,8 +871,8 @@ template <class Gen, class GB, int NCB, int NW>
 __global__ void __launch_bounds__(64 * NW) k_rowgemm_bf(Gen gen, GB gb, int nrow, int ngl, int nbh, int gsplit,
                                                         int tr, int tb, int ns, double2 *__restrict__ part) {
   constexpr int WR = 16 * NW, NB16 = 16 * NCB;
-  __shared__ __bf16 sA[NPL * WR][KBP];
-  __shared__ __bf16 sB[NPL * NB16][KBP];
+  __shared__ __align__(16) __bf16 sA[NPL * WR][KBP];
+  __shared__ __align__(16) __bf16 sB[NPL * NB16][KBP];
   const XcdTile xt = xcd_tile(tr * tb, ns);
   if (!xt.valid) return;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6, li = lane & 15, lk = lane >> 4;
@@ -1037,8 +1041,8 @@ struct SrcChiCols {          // [chi_k(G); conj(chi_k(-G))] along K = 2 NBH, row
 template <class GA, class GB, int NRB, int NW>
 __global__ void __launch_bounds__(64 * NW) k_colgemm_bf(GA ga, GB gb, int nk, int ngl, int nbh, ColOut out) {
   constexpr int WG = 16 * NW, NB16 = 16 * NRB;
-  __shared__ __bf16 sB[NPL * WG][KBP];
-  __shared__ __bf16 sA[NPL * NB16][KBP];
+  __shared__ __align__(16) __bf16 sB[NPL * WG][KBP];
+  __shared__ __align__(16) __bf16 sA[NPL * NB16][KBP];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6, li = lane & 15, lk = lane >> 4;
   const int g0 = blockIdx.x * WG, b0 = blockIdx.y * NB16;
   dbl4 accr[NRB], acci[NRB];   // FP64 sums of per-chunk FP32 MFMA sums
@@ -1121,7 +1125,7 @@ __global__ void __launch_bounds__(64 * NW) k_force_bf(GA ga, GB gb, int npro, in
                                                       const double *__restrict__ gvec, int nrt, int ngt,
                                                       double *__restrict__ part) {
   constexpr int WG = 16 * NW, NB16 = 16 * NRB;
-  __shared__ __bf16 sB[NPL * WG][KBP];
+  __shared__ __align__(16) __bf16 sB[NPL * WG][KBP];
   __shared__ __align__(16) __bf16 sA[NPL * NB16][KBP];
   // per-wave row sums of the epilogue reuse the A staging area (free after the K loop)
   static_assert(sizeof(double) * NW * NB16 * 3 <= sizeof(__bf16) * NPL * NB16 * KBP, "sF fits in sA");

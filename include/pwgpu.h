@@ -209,6 +209,10 @@ int pw_waves_density(pw_waveset *ws, const void *psi_dev, double *rho_dev);
 int pw_ortho_x(int nb, const double *occ, const double *chichi,
                const double *psipsi, const double *chipsi, double *lambda,
                int *iter);
+/* the same on row-major matrices */
+int pw_ortho_x_rows(int nb, const double *occ, const double *chichi,
+               const double *psipsi, const double *chipsi, double *lambda,
+               int *iter);
 
 /* ---- density -> potential (POTENTIAL$VOFRHO) --------------------------------
  * Replaces the core of POTENTIAL$VOFRHO (src/paw_potential.f90:324-896:

@@ -375,16 +375,19 @@ __host__ __device__ constexpr int fft_lprod(const Fft1D &f, int st) {
   return L;
 }
 
-// threads of the yz passes: kYZ, for the large FP64 planes twice as many.  One
-// such plane fills a CU's LDS (104 KiB for 80 x 80), so the workgroup is all
-// that hides the latency of its stages; with 512 threads a stage of 72 x 72
-// takes two rounds of butterflies, 57 % full, with 1024 one: 72 x 72 planes of
-// 72 super bands 188 -> 178 us (density 98 -> 94), 80 x 80 of 128 307 -> 279;
-// 704 threads (one full round) 183, 281 and 101.  FP32 planes share a CU by
-// threes: 384 and 704 threads are slower there (88 and 94 us against 82).
+// threads of the yz passes: kYZ, twice as many where one FP64 plane fills a
+// CU's LDS (104 KiB for 80 x 80) and its workgroup is all that hides the latency
+// of the stages; 512 threads also take two rounds of butterflies per stage of 72
+// x 72, 57 % full, 1024 one: 72 x 72 planes of 72 super bands 188 -> 178 us
+// (density 98 -> 94), 80 x 80 of 128 307 -> 279; 704 threads (one full round)
+// 183, 281 and 101.  Where two planes share a CU (64 x 64, one full round of
+// 512) 1024 threads are slower: V psi of 24 H2O 140 us against 117.  FP32 planes
+// share a CU by threes: 384 and 704 threads are slower there (88 and 94 us
+// against 82).
 template <typename T2, int NY, int NZ>
 constexpr int yz_threads() {
-  return sizeof(T2) == 16 && NY * NZ >= 48 * 48 ? 1024 : kYZ;
+  constexpr int lds = ((NY | 1) * NZ + NY + NZ) * (int)sizeof(T2);
+  return sizeof(T2) == 16 && 2 * lds > 160 * 1024 ? 1024 : kYZ;
 }
 
 template <int N> constexpr int nstage_ct() { return fft_inplace_ct(N).nstage; }

@@ -33,11 +33,18 @@ __host__ __device__ constexpr Fft1D pencil_stages(int n) {
   return f;
 }
 
-// pencils per workgroup: at most 40 KiB of exchange buffer, 16 to 64 (FP64) or 128 (FP32)
+// pencils per workgroup: at most 40 KiB of exchange buffer, 16 to 64 (FP64) or
+// 128 (FP32); lengths of three stages have two buffers, together at most 48 KiB
+// (with 40 each two workgroups fit on a CU: RTOG of 95 x 30^3 in FP32 51 us, now
+// 33, in FP64 51 -> 39; 60^3 37 -> 29, 66^3 48 -> 34, 70^3 46 -> 35; 42 and 84
+// keep their tile)
 template <typename T2, int N>
 constexpr int pencil_tile() {
+  const int nbuf = pencil_stages<T2>(N).nstage > 2 ? 2 : 1;
   int p = 16;
-  while (2 * p * N * (int)sizeof(T2) <= 40960 && 2 * p * (int)sizeof(T2) <= 1024) p *= 2;
+  while (2 * p * N * (int)sizeof(T2) <= 40960 && 2 * p * N * nbuf * (int)sizeof(T2) <= 49152 &&
+         2 * p * (int)sizeof(T2) <= 1024)
+    p *= 2;
   return p;
 }
 

@@ -16,7 +16,8 @@
 //   (or too ill-conditioned for the series) S^-1 is applied as the reference
 //   does, through the eigenvectors of B, which one workgroup computes by
 //   cyclic Jacobi rotations (ortho_x_eig).  The P_k are formed once
-//   per call by doubling (one row-panel batch launch per level); each outer
+//   per call (up to 8 in one launch, more by doubling, one row-panel batch
+//   launch per level); each outer
 //   iteration then applies the series in two launches (row-panel chains
 //   P_k G P_k, then the ordered sum over k with the convergence test and the
 //   LAMBDA update).  Only terms beyond 2^5 would continue by the Smith
@@ -1820,8 +1821,8 @@ int ortho_x_device(pw_waveset *ws, double *d_lam, const double *d_chichi, const 
     OrthoState hs{};
     OrthoState *hp = static_cast<OrthoState *>(ws->h_ortho_state);
     // one workgroup for the whole solve where its matrices fit in LDS and a
-    // product has at most four tiles: 32 bands with 8 terms of the series, 20
-    // with 16.  The launches of the chain take 218 us in kernels and 430 with
+    // product has at most four tiles: 32 bands with 8 terms of the series, 24
+    // with 16, 16 with 32.  The launches of the chain take 218 us in kernels and 430 with
     // the gaps for 20 bands, this one 44; for 32 bands 230 and 500 against 64.
     // Wider sets do not fit with their 8 terms.
     if (P.nser == P.nlev && (n + T16 - 1) / T16 <= kSmallTiles && small_lds(n, 1 << P.nser) <= kLdsMax) {

@@ -1,5 +1,5 @@
-"""ORTHO_X in one workgroup (up to 32 bands with 8 terms of the series, 20
-with 16) against the oracle: one and two 16 x 16 tiles per edge
+"""ORTHO_X in one workgroup (up to 32 bands with 8 terms of the series, 24
+with 16, 16 with 32) against the oracle: one and two 16 x 16 tiles per edge
 and their remainders, the widest set, the first one above it (launch chain),
 and spectra of sym(CHIPSI) that ask for 4 to 32 terms.  Both sides form the
 same iterates; the series is cut at 1.6e-11 of its first term and the bound is

@@ -250,6 +250,7 @@ struct pw_waveset {
   bool lz_valid = false;
   int ortho_lanczos = 0;       // Lanczos runs in the last ORTHO_X call
   int ortho_eigen = 0;         // ORTHO_X solves through the eigenvectors of sym(CHIPSI) (B not positive definite)
+  int ortho_passes = 0;        // passes over the series' terms in the last ORTHO_X call
   bool ortho_once = false;     // a single solve: no graph is captured for it
   int ortho_graph_misses = 0;  // ORTHO_X solves issued without a graph (other objects alive)
   // launch shapes chosen by pw_waves_autotune

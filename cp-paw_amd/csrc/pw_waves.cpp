@@ -885,6 +885,7 @@ extern "C" int pw_waves_geti4(pw_waveset *ws, const char *id, int *val) {
   else if (s == "SPLITWAVES") *val = ws->tune_split_waves;
   else if (s == "COLWAVES") *val = ws->tune_col_waves;
   else if (s == "DENSBLOCKS") *val = ws->tune_dens_blocks;
+  else if (s == "ORTHOPASSES") *val = ws->ortho_passes;
   else if (s == "ORTHOLANCZOS") *val = ws->ortho_lanczos;
   else if (s == "ORTHOEIGEN") *val = ws->ortho_eigen;
   else if (s == "ORTHOGRAPHMISSES") *val = ws->ortho_graph_misses;

@@ -150,7 +150,10 @@ int pw_waves_getr8a(pw_waveset *ws, const char *id, int len, double *val);
 int pw_waves_getr8(pw_waveset *ws, const char *id, double *val);
 /* "ORTHOITER" (iterations of the last WAVES_ORTHO_X), "NPRO", "NBH",
  * "LMNXX", "ORTHOLEVELS" (squared-Smith levels of the last solve), "ORTHONS"
- * (Newton-Schulz steps of the last solve), "ORTHOLANCZOS" (Lanczos runs for
+ * (Newton-Schulz steps of the last solve), "ORTHOPASSES" (passes over the
+ * terms of the series in the last solve, one per update of the multipliers; 0
+ * without such terms: a solve through the eigenvectors, or of sets too wide
+ * for them, above 609 bands), "ORTHOLANCZOS" (Lanczos runs for
  * the spectral bounds in the last solve: 0 when the previous bounds were
  * accepted), "ORTHOEIGEN" (solves so far through the eigenvectors of
  * sym(CHIPSI), taken when it is not positive definite), "ORTHOGRAPHMISSES"

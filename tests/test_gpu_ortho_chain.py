@@ -46,3 +46,16 @@ def test_ortho_x_column_major(nb):
     assert load().pw_ortho_x(nb, dptr(occ), *[dptr(m) for m in col], ctypes.byref(it)) == 0
     assert it.value == it_ref
     assert np.array_equal(col[3].T, ref)
+
+
+@pytest.mark.parametrize("nb", [20, 48, 146])
+def test_no_terms_where_the_loop_ends(nb):
+    """The series is applied once per update of the multipliers: not in the
+    iteration whose GAMN is converged, in one workgroup and by panels."""
+    from test_gpu_gamma import both
+    print(f"case series passes nb={nb}", flush=True)
+    s, o, w = both(nb, 3)
+    for f in (w.etot, w.propagate, w.orthogonalize):
+        f()
+    assert w.geti4("ORTHOITER") > 1 and w.geti4("ORTHOEIGEN") == 0
+    assert w.geti4("ORTHOPASSES") == w.geti4("ORTHOITER") - 1

@@ -524,6 +524,7 @@ int ws_reset_run(pw_waveset *ws) {
   f.d_atom_isp = ws->d_atom_isp; f.d_ipro0 = ws->d_ipro0; f.d_ibpro = ws->d_ibpro; f.d_lmnx = ws->d_lmnx;
   f.d_lmn_ln = ws->d_lmn_ln; f.d_lmn_lm = ws->d_lmn_lm; f.d_lmn_l = ws->d_lmn_l; f.d_ipro_tab = ws->d_ipro_tab;
   f.d_ipro4 = ws->d_ipro4;
+  f.pro_sym = ws->pro_sym;   // a property of the table in d_pro
   f.d_phase = ws->d_phase; f.d_small_mats = ws->d_small_mats;
   f.d_res = ws->d_res; f.h_res = ws->h_res;
   f.d_pfac = ws->d_pfac; f.pfac_bytes = ws->pfac_bytes;

@@ -102,3 +102,34 @@ def test_residual_convergence():
     assert by_r["converged"] == 1 and by_e["converged"] == 1
     assert 0.0 < by_r["residual"] < 1.0e-5
     assert abs(by_r["etot"] - by_e["etot"]) < 1.0e-5
+
+
+@pytest.mark.gpu
+def test_reset_set_keeps_its_projector_table():
+    """A set that is reset for the next request keeps the PRO table on the
+    device, and with it the choice of the products: a table with PRO(G) !=
+    PRO(-G) takes those over the whole sphere also when the next run does not
+    set it again.  1e-11 as in the tests of the products."""
+    import ctypes
+
+    import pwgpu
+    from harness import oracle_waveset, relerr
+    print("case reset set with PRO(G) != PRO(-G)", flush=True)
+    s = model.tiny(nb=16, nat=3)
+    o = oracle_waveset(s)
+    rng = np.random.default_rng(1)
+    o.pro = o.pro * rng.uniform(0.5, 1.5, o.pro.shape)
+    o.psi0 = rng.normal(size=o.psi0.shape) + 1j * rng.normal(size=o.psi0.shape)
+    o.psim = o.psi0.copy()
+    plane = pwgpu.PlaneWave(s.rbas, s.epw_psi, s.epw_rho)
+    w = pwgpu.Waves.from_system(plane, s, psi=o.psi0)
+    w.setr8a("PRO", o.pro)
+    reset = w.lib._Z12ws_reset_runP10pw_waveset      # internal: the request loop calls it
+    reset.argtypes = [ctypes.c_void_p]
+    assert reset(w.handle) == 0
+    for kind, key, val in w.system_inputs(s, o.psi0):
+        if key != "PRO":
+            getattr(w, "set" + kind)(key, val)
+    o.etot(s.pos)
+    w.etot()
+    assert relerr(w.getc8a("PROJ"), o.proj) < 1e-11

@@ -365,7 +365,7 @@ extern "C" int pw_waves_footprint(pw_plan *plan, int nb, int nat, int nsp, const
   b += (long long)(21 + 6) * nb * nb * 8;           // NB x NB matrices, ORTHO_X work
   b += 3 * ((npro + 63) / 64) * nbh * nbh * 32;     // one-centre overlaps of three matrices
   b += ngl * 48 + (long long)nat * lmnxx * lmnxx * 32;
-  if (prec == PW_PREC_FP64) b += (nsp * lmnxx * 8 + nat * 16) * (ngl / 2 + 33);  // projector factors on the G pairs
+  b += (nsp * lmnxx * 8 + nat * 16) * (ngl / 2 + 33);   // projector factors on the G pairs (mixed form: for ORTHOERR)
   if (prec == PW_PREC_MIXED) b += (nsp * lmnxx * 12 + nat * 24) * nglp;  // projector factors, FP64 and FP32
   *bytes = b + b / 10 + (8ll << 20);
   return PW_OK;

@@ -104,6 +104,34 @@ def test_residual_convergence():
     assert abs(by_r["etot"] - by_e["etot"]) < 1.0e-5
 
 
+def test_footprint_counts_the_factor_tables_of_a_mixed_set():
+    """A mixed set holds its own projector factors and, once ORTHOERR is read,
+    those of the FP64 products too: against the FP64 set it has FP32 stripes
+    and V, and its own factors on top."""
+    import ctypes
+
+    import pwgpu
+    from pwgpu import _lib
+    lib = _lib.load()
+    s = model.si_supercell(16)
+    plane = pwgpu.PlaneWave(s.rbas, s.epw_psi, s.epw_rho)
+    isp = (np.asarray(s.isp) + 1).astype(np.int32)
+    lnx = np.array([len(l) for l in s.lox_list], dtype=np.int32)
+    lox = np.array(s.lox_list[0], dtype=np.int32)
+    size = {}
+    for prec in (0, 1):
+        b = ctypes.c_longlong()
+        _lib.check(lib.pw_waves_footprint(plane.handle, s.nb, s.nat, 1, _lib.iptr(isp), _lib.iptr(lnx),
+                                          int(lnx.max()), _lib.iptr(lox), prec, ctypes.byref(b)))
+        size[prec] = b.value
+    nbh, nglp = (s.nb + 1) // 2, (plane.ngl + 63) // 64 * 64
+    lmnx = sum(2 * l + 1 for l in s.lox_list[0])
+    fp32 = 8 * (nbh * plane.geti4("NSTRIPE") * plane.nr[0] + plane.nrl)
+    own = (12 * lmnx + 24 * s.nat) * nglp
+    plane.close()
+    assert size[1] >= size[0] + (own - fp32) * 11 // 10 - 16
+
+
 @pytest.mark.gpu
 def test_reset_set_keeps_its_projector_table():
     """A set that is reset for the next request keeps the PRO table on the

@@ -382,9 +382,8 @@ int k_addpro_opsi(pw_waveset *ws, double2 *opsi, const double2 *psi0, const doub
 int k_force(pw_waveset *ws, const double2 *psi, const double2 *phase, const double2 *dedproj, double *dst);
 // max over super bands of |HPSI - (1+a) m/dt^2 (psi(+) - psibar)| into dst (device)
 int k_residual(pw_waveset *ws, const double2 *psibar, double *dst);
-int k_overlap(pw_waveset *ws, const double2 *psi1, const double2 *psi2, double *mat_host_or_dev, bool to_host, bool tid);
-// mat_dev = WAVES_OVERLAP(psi1, psi2) + WAVES_1COVERLAP(proj1, proj2) in one sequence
-// one overlap matrix: psi1, psi2 with their projections (null: no one-centre part)
+// one overlap matrix, WAVES_OVERLAP(psi1, psi2) + WAVES_1COVERLAP(proj1, proj2); up
+// to kOvlJobs of them in one sequence
 constexpr int kOvlJobs = 3;
 struct OverlapJob {
   const double2 *psi1, *psi2, *proj1, *proj2;

@@ -288,22 +288,6 @@ __global__ void __launch_bounds__(64 * NW) k_force_m(ProjGeo q, const int2 *ipta
   }
 }
 
-
-// unravel super-wave products into the NB x NB real matrix (row-major),
-// WAVES_OVERLAP (src/paw_waves2.f90:805-848); t, tm already times Omega
-__global__ void k_unravel_pw(int nbh, int nb, const double2 *t, const double2 *tm, double *mat) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= nbh * nbh) return;
-  const int i = idx / nbh, j = idx % nbh;
-  const double re = 0.5 * t[idx].x, im = 0.5 * t[idx].y;
-  const double rem = 0.5 * tm[idx].x, imm = 0.5 * tm[idx].y;
-  const int ia = 2 * i, ja = 2 * j;
-  mat[(size_t)ia * nb + ja] = re + rem;
-  mat[(size_t)ia * nb + ja + 1] = im + imm;
-  mat[(size_t)(ia + 1) * nb + ja] = -im + imm;
-  mat[(size_t)(ia + 1) * nb + ja + 1] = re - rem;
-}
-
 // ---------------------------------------------------------------------------
 // one-centre overlap (WAVES_1COVERLAP, src/paw_waves2.f90:856-1022), added to mat
 // c1 = sum_k conj(p1_ki) p2a_kj, c2 = sum_k p1_ki p2a_kj, p2a = DO p2 of each
@@ -355,8 +339,9 @@ __global__ void __launch_bounds__(256) k_overlap1c(ProjGeo q, int npro, int nbh,
 
 // WAVES_OVERLAP's matrix in one pass from the G-split partials of the
 // stacked product (rows 0..nbhp-1: T, rows nbhp..: TM): the sums of
-// k_reduce_split, the unravel of k_unravel_pw and, with part1c, the
-// one-centre sum over the runs of k_overlap1c in z order.
+// k_reduce_split, the unravel of the super waves into the NB x NB real matrix
+// (row-major; src/paw_waves2.f90:805-848) and, with part1c, the one-centre sum
+// over the runs of k_overlap1c in z order.
 __global__ void __launch_bounds__(kRedC * kRedS) k_overlap_finish(const double2 *__restrict__ part, int ns, size_t n,
                                                                   double scale, int nbh, int nbhp, int nb,
                                                                   const double4 *__restrict__ part1c, int nz,
@@ -1606,9 +1591,6 @@ int wave_runs(pw_waveset *ws, const double2 *psi, bool minus, size_t off, SplitR
   return PW_OK;
 }
 
-// out[r][b] = scale sum_G A(r,G) psi[b][G]: split over G (about two waves per
-// SIMD), deterministic reduction of the splits.  out == nullptr puts the
-// result behind the partials and returns it in *res.
 // G-split partials left for the caller's own reduction (defer != nullptr)
 struct RowPart {
   const double2 *part = nullptr;
@@ -1617,9 +1599,11 @@ struct RowPart {
   double scale = 1.0;
 };
 
+// out[r][b] = scale sum_G A(r,G) psi[b][G]: split over G (about two waves per
+// SIMD), deterministic reduction of the splits
 template <int NW, class Gen>
 int run_rowgemm(pw_waveset *ws, const Gen &gen, int nrow, const double2 *psi, double scale,
-                double2 *out, double2 **res, const char *name) {
+                double2 *out, const char *name) {
   const int ngl = ws->plan->ngl, nbh = ws->nbh;
   int nblk, tb;
   band_tiles(nbh, &nblk, &tb);
@@ -1629,9 +1613,8 @@ int run_rowgemm(pw_waveset *ws, const Gen &gen, int nrow, const double2 *psi, do
   const int gsplit = ((ngl + ns - 1) / ns + KC - 1) / KC * KC;
   ns = (ngl + gsplit - 1) / gsplit;
   const size_t n = (size_t)nrow * nbh;
-  PW_TRY(ws_part(ws, (size_t)(ns + (out ? 0 : 1)) * n * sizeof(double2)));
+  PW_TRY(ws_part(ws, (size_t)ns * n * sizeof(double2)));
   double2 *part = (double2 *)ws->d_part;
-  if (!out) out = part + (size_t)ns * n;
   {
     ScopeTimer tm(ws, name);
     const unsigned grid = xcd_blocks(tr * tb, ns);
@@ -1647,7 +1630,6 @@ int run_rowgemm(pw_waveset *ws, const Gen &gen, int nrow, const double2 *psi, do
                                                                                          out);
     PW_HIP(hipGetLastError());
   }
-  if (res) *res = out;
   return PW_OK;
 }
 
@@ -1669,7 +1651,7 @@ int run_colgemm(pw_waveset *ws, const GA &ga, const GB &gb, int nk, const ColOut
 // split-BF16x3 counterpart of run_rowgemm (G splits are whole 32-chunks)
 template <int NW, class Gen>
 int run_rowgemm_bf(pw_waveset *ws, const Gen &gen, int nrow, const BandRuns &gb, double scale,
-                   double2 *out, double2 **res, const char *name, RowPart *defer = nullptr) {
+                   double2 *out, const char *name, RowPart *defer = nullptr) {
   const int ngl = ws->plan->ngl, nbh = ws->nbh;
   int nblk, tb;
   band_tiles(nbh, &nblk, &tb);
@@ -1679,9 +1661,8 @@ int run_rowgemm_bf(pw_waveset *ws, const Gen &gen, int nrow, const BandRuns &gb,
   const int gsplit = ((ngl + ns - 1) / ns + KB - 1) / KB * KB;
   ns = (ngl + gsplit - 1) / gsplit;
   const size_t n = (size_t)nrow * nbh;
-  PW_TRY(ws_part(ws, (size_t)(ns + (out ? 0 : 1)) * n * sizeof(double2)));
+  PW_TRY(ws_part(ws, (size_t)ns * n * sizeof(double2)));
   double2 *part = (double2 *)ws->d_part;
-  if (!out) out = part + (size_t)ns * n;
   {
     ScopeTimer tm(ws, name);
     const unsigned grid = xcd_blocks(tr * tb, ns);
@@ -1702,7 +1683,6 @@ int run_rowgemm_bf(pw_waveset *ws, const Gen &gen, int nrow, const BandRuns &gb,
                                                                                          out);
     PW_HIP(hipGetLastError());
   }
-  if (res) *res = out;
   return PW_OK;
 }
 
@@ -1820,13 +1800,13 @@ int k_projections(pw_waveset *ws, const double2 *psi, const double2 *phase, doub
     BandRuns gb;
     PW_TRY(wave_runs(ws, psi, false, 0, &gb.s));
     RowPf gen{pfac_of(ws)};
-    return run_rowgemm_bf<4>(ws, gen, ws->npro, gb, ws->plan->vol, proj, nullptr, "projections");
+    return run_rowgemm_bf<4>(ws, gen, ws->npro, gb, ws->plan->vol, proj, "projections");
   }
   if (ws->pro_sym) return half_projections(ws, psi, proj);
   ProjGeo q = make_pgeo(ws);
   q.phase = phase;
   GenProj gen{q, ws->d_ipro_tab};
-  return run_rowgemm<4>(ws, gen, ws->npro, psi, ws->plan->vol, proj, nullptr, "projections");
+  return run_rowgemm<4>(ws, gen, ws->npro, psi, ws->plan->vol, proj, "projections");
 }
 
 // psi = (src or psi) + sum_i |p_i> x_i, then times num / m(G) when scaled
@@ -1907,37 +1887,10 @@ int k_force(pw_waveset *ws, const double2 *psi, const double2 *phase, const doub
   return PW_OK;
 }
 
-// mat_dev (row-major NB x NB) = WAVES_OVERLAP(psi1, psi2)
-// T = Omega sum_G conj(psi1_i) psi2_j and TM = Omega sum_G psi1_i psi2_j(-G)
-//   = Omega sum_G psi1_i(-G) psi2_j(G), one GEMM over stacked rows
-int k_overlap(pw_waveset *ws, const double2 *psi1, const double2 *psi2, double *mat, bool, bool) {
-  pw_plan *p = ws->plan;
-  const int nbh = ws->nbh, nbhp = (nbh + 15) / 16 * 16;
-  if (ws->prec == PW_PREC_FP64) {
-    const OverlapJob job{psi1, psi2, nullptr, nullptr, mat};
-    return half_overlap(ws, &job, 1, nullptr, 0);
-  }
-  double2 *red = nullptr;
-  {
-    const size_t bytes = runs_bytes(nbh, p->ngl);
-    PW_TRY(ws_split(ws, 3 * bytes));   // outside a runs scope all three go to the scratch
-    OvlRuns gen;
-    gen.nbhp = nbhp;
-    BandRuns gb;
-    PW_TRY(wave_runs(ws, psi1, false, 0, &gen.rows));
-    PW_TRY(wave_runs(ws, psi1, true, bytes, &gen.minus));
-    if (psi2 == psi1) gb.s = gen.rows;
-    else PW_TRY(wave_runs(ws, psi2, false, 2 * bytes, &gb.s));
-    PW_TRY(run_rowgemm_bf<2>(ws, gen, 2 * nbhp, gb, p->vol, nullptr, &red, "overlap"));
-  }
-  k_unravel_pw<<<(nbh * nbh + 255) / 256, 256, 0, ws->stream>>>(nbh, ws->nb, red, red + (size_t)nbhp * nbh,
-                                                                  mat);
-  PW_HIP(hipGetLastError());
-  return PW_OK;
-}
-
-// one matrix in the mixed form: the G-split product with its reduction
-// deferred, then one k_overlap_finish pass
+// one matrix in the mixed form: T = Omega sum_G conj(psi1_i) psi2_j and TM =
+// Omega sum_G psi1_i psi2_j(-G) = Omega sum_G psi1_i(-G) psi2_j(G) as one G-split
+// product over stacked rows with its reduction deferred, then one
+// k_overlap_finish pass
 static int overlap_mixed(pw_waveset *ws, const OverlapJob &o, const double4 *p1c, int nz) {
   pw_plan *p = ws->plan;
   const int nbh = ws->nbh, nbhp = (nbh + 15) / 16 * 16;
@@ -1953,7 +1906,7 @@ static int overlap_mixed(pw_waveset *ws, const OverlapJob &o, const double4 *p1c
     PW_TRY(wave_runs(ws, psi1, true, bytes, &gen.minus));
     if (psi2 == psi1) gb.s = gen.rows;
     else PW_TRY(wave_runs(ws, psi2, false, 2 * bytes, &gb.s));
-    PW_TRY(run_rowgemm_bf<2>(ws, gen, 2 * nbhp, gb, p->vol, nullptr, nullptr, "overlap", &rp));
+    PW_TRY(run_rowgemm_bf<2>(ws, gen, 2 * nbhp, gb, p->vol, nullptr, "overlap", &rp));
   }
   {
     ScopeTimer tm(ws, "reduce");

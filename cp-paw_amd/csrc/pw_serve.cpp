@@ -59,7 +59,7 @@ using Clock = std::chrono::steady_clock;
 
 // launch shapes per system shape, shared by all jobs of the process
 std::mutex g_tune_mu;
-std::map<std::tuple<int, int, int, int, int>, std::array<int, 3>> g_tuned;
+std::map<std::tuple<int, int, int, int, int, bool>, std::array<int, 3>> g_tuned;
 
 }  // namespace
 
@@ -247,7 +247,8 @@ void worker(pw_server *s) {
 // ---------------------------------------------------------------------------
 // autotuner: G-split width of the projection/overlap GEMMs and the band
 // grouping of the density pass, timed with HIP events on the waveset's
-// stream; the choice is cached per (NGL, NBH, NPRO, NR1, prec)
+// stream; the choice is cached per (NGL, NBH, NPRO, NR1, prec, PRO(G) =
+// PRO(-G)): the last one decides which products run
 // ---------------------------------------------------------------------------
 extern "C" int pw_waves_autotune(pw_waveset *ws) {
   if (!ws) return pw_fail(PW_ERR_ARG, "pw_waves_autotune: null waveset");
@@ -255,7 +256,7 @@ extern "C" int pw_waves_autotune(pw_waveset *ws) {
   if (!ws->have_psi0 || ws->r0.empty())
     return pw_fail(PW_ERR_STATE, "pw_waves_autotune: PSI0 and R0 must be set");
   pw_plan *p = ws->plan;
-  const auto key = std::make_tuple(p->ngl, ws->nbh, ws->npro, p->nr1, ws->prec);
+  const auto key = std::make_tuple(p->ngl, ws->nbh, ws->npro, p->nr1, ws->prec, ws->pro_sym);
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find(key);
@@ -286,16 +287,22 @@ extern "C" int pw_waves_autotune(pw_waveset *ws) {
   if (rc == PW_OK) {
     // G-split width of the row products: more splits fill the GPU, fewer
     // shrink the partial sums their ordered reduction reads back; timed on
-    // the projections and one band overlap (the two row-product shapes),
-    // reductions included, into the Gram-Schmidt scratch matrix
+    // the projections and the three overlaps of a step (launched together, the
+    // FP64 ones divide the splits between them), reductions included, into
+    // matrices that no result is read from
     double tbest = 1e30;
-    double *mat = ws->d_small_mats + (size_t)4 * ws->nb * ws->nb;
+    auto mat = [&](int k) { return ws->d_small_mats + (size_t)k * ws->nb * ws->nb; };
+    const OverlapJob jobs[3] = {{ws->d_psim, ws->d_psim, ws->d_oproj, ws->d_oproj, mat(3)},
+                                {ws->d_psi0, ws->d_psim, ws->d_oproj, ws->d_oproj, mat(4)},
+                                {ws->d_psi0, ws->d_psi0, ws->d_oproj, ws->d_oproj, mat(5)}};
     for (int cand : {256, 512, 1024, 2048, 4096}) {
       ws->tune_split_waves = cand;
       const double t = timed([&] {
-        int r = k_projections(ws, ws->d_psi0, ws->d_phase, ws->d_oproj);
-        if (r == PW_OK) r = k_overlap(ws, ws->d_psi0, ws->d_psi0, mat, false, true);
-        return r;
+        int r = k_runs_scope(ws, true);
+        if (r == PW_OK) r = k_projections(ws, ws->d_psi0, ws->d_phase, ws->d_oproj);
+        if (r == PW_OK) r = k_overlap_full(ws, jobs, 3);
+        const int e = k_runs_scope(ws, false);
+        return r != PW_OK ? r : e;
       });
       if (t < tbest) { tbest = t; best_split = cand; }
     }

@@ -161,3 +161,31 @@ def test_reset_set_keeps_its_projector_table():
     o.etot(s.pos)
     w.etot()
     assert relerr(w.getc8a("PROJ"), o.proj) < 1e-11
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [0, 1])
+def test_autotune_times_the_launches_of_a_step(prec):
+    """The row products are timed as a step launches them, the three overlaps
+    with their one-centre parts together, and the choice is kept apart for
+    sets whose PRO table takes other products."""
+    import pwgpu
+    print(f"case autotune prec={prec}", flush=True)
+    s = model.tiny(nb=22 + 2 * prec, nat=5)
+    plane = pwgpu.PlaneWave(s.rbas, s.epw_psi, s.epw_rho)
+
+    def launches(asym):
+        w = pwgpu.Waves.from_system(plane, s, prec=prec)
+        if asym:
+            pro = s.pro_table(plane.getr8a("G2"))
+            w.setr8a("PRO", pro * np.random.default_rng(2).uniform(0.5, 1.5, pro.shape))
+        w.profile()
+        w.autotune()
+        n = [w.kernel_time(k)[1] for k in ("projections", "overlap1c")]
+        w.close()
+        return n
+
+    for asym in (False, True):
+        proj, one = launches(asym)
+        assert proj > 3 and one > 0, asym
+        assert launches(asym)[1] == 0, asym      # the second set of the shape takes the kept choice

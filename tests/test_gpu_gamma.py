@@ -54,3 +54,57 @@ def test_products_whole_sphere(nb):
     assert relerr(w.getc8a("PSI0"), o.psi0) < 1e-11
     assert relerr(w.getc8a("PROJ"), o.proj) < 1e-11
     assert relerr(w.getc8a("HPSI"), o.hpsi) < 1e-11
+
+
+def step(monkeypatch, s, o, w):
+    """One CP step on both sides; the oracle's overlap matrices (MAT, OMAT, OOMAT) as well."""
+    from oracle import waves as owv
+    seen = {}
+    solve = owv.ortho_x
+
+    def ortho_x(occ, chichi, psipsi, chipsi, lam):
+        seen.update(MAT=psipsi, OMAT=chipsi, OOMAT=chichi)
+        return solve(occ, chichi, psipsi, chipsi, lam)
+
+    monkeypatch.setattr(owv, "ortho_x", ortho_x)
+    o.etot(s.pos)
+    o.propagate()
+    o.orthogonalize(s.pos, s.pos)
+    for f in (w.etot, w.propagate, w.orthogonalize):
+        f()
+    return seen
+
+
+@pytest.mark.parametrize("nb,nat", [(18, 2), (146, 2), (260, 3)])
+def test_overlaps_of_a_step(nb, nat, monkeypatch):
+    """The three overlap matrices of a step side by side in one launch, at the
+    remainders of the band tiles; 1e-11 on the matrices and 1e-9 on the
+    multipliers as in the step tests."""
+    print(f"case gamma overlaps of a step nb={nb} nat={nat}", flush=True)
+    s, o, w = both(nb, nat)
+    for k, m in step(monkeypatch, s, o, w).items():
+        assert relerr(w.getr8a(k), m) < 1e-11, k
+    assert w.geti4("ORTHOITER") == o.ortho_iter
+    assert relerr(w.getc8a("RLAM0").real, o.rlam0) < 1e-9
+
+
+@pytest.mark.parametrize("nb", [16, 146])
+def test_step_whole_sphere(nb, monkeypatch):
+    """Forces and a step with PRO(G) != PRO(-G): OPSI and the overlaps with it,
+    and the forces as the plain sum over the sphere, without the INVERTG
+    average of dE/dP, which changes nothing where P(-G) = conj(P(G)) and which
+    the kernels leave out."""
+    from oracle import waves as owv
+    print(f"case gamma step, PRO(G) != PRO(-G), nb={nb}", flush=True)
+    monkeypatch.setattr(owv, "dedpro", lambda plane, psi, ded: np.conj(ded) @ psi)
+    s, o, w = both(nb, 3, asym=True)
+    mats = step(monkeypatch, s, o, w)
+    assert relerr(w.getr8a("FORCE"), o.force) < 1e-10
+    for k, m in mats.items():
+        assert relerr(w.getr8a(k), m) < 1e-11, k
+    assert relerr(w.getc8a("RLAM0").real, o.rlam0) < 1e-9
+    o.switch()
+    w.switch()
+    o.etot(s.pos)
+    w.etot()
+    assert relerr(w.getr8a("FORCE"), o.force) < 1e-9

@@ -126,15 +126,10 @@ template <> struct XTile<float2> { static constexpr int n = 32; };
 // (VOFRHO's transforms) they had all run on one XCD, 21 and 17 us for the
 // passes of the Si64 density sphere against 9 and 8.
 __device__ inline void x_block(int ngroups, int nb, int &group, int &band) {
-  const int id = blockIdx.x, whole = nb / 8 * 8, r = id - whole * ngroups;
-  if (r >= 0) {
-    band = whole + r / ngroups;
-    group = r % ngroups;
-    return;
-  }
-  const int j = id / 8;
-  band = id % 8 + 8 * (j / ngroups);
-  group = j % ngroups;
+  const unsigned id = blockIdx.x, whole = (unsigned)nb & ~7u, n8 = whole * ngroups;
+  const unsigned j = id < n8 ? id / 8 : id - n8, q = j / (unsigned)ngroups;
+  band = (int)(id < n8 ? id % 8 + 8 * q : whole + q);
+  group = (int)(j - q * ngroups);
 }
 inline dim3 x_grid(int ngroups, int nb) { return dim3((unsigned)(nb * ngroups)); }
 // LDS pitch of the x passes' stripe tiles: odd, so that the tile's transposes
@@ -180,13 +175,14 @@ __global__ void __launch_bounds__(kBlock) k_xfwd(Geo g, Fft1D f, const T2 *tw, c
   }
 }
 
-// ---- x pass, inverse: stripes -> sphere (gather, scale, optional G^2/2 psi) ---
-// add_kin: 0 nothing, 1 + G^2/2 psi, kAddPlain + psi
-constexpr int kAddPlain = 2;
+// ---- x pass, inverse: stripes -> sphere (gather, scale, optional term) --------
+// add: + G^2/2 psi (V psi), in rows + psi (RTOG's added coefficients).  Which of
+// the two is fixed per instance: chosen per element, it cost 1.5 of 48.5 us for
+// 64 bands of 80^3 in FP64.
 template <typename T2, int NX = 0, bool ROW = false>
 __global__ void __launch_bounds__(kBlock) k_xinv(Geo g, Fft1D f, const T2 *tw, const T2 *stripes,
                                                  double2 *out, const double2 *psi, double scale,
-                                                 int add_kin, int nb) {
+                                                 int add, int nb) {
   constexpr int PX = XTile<T2>::n;
   if constexpr (NX > 0) g.nr1 = NX;
   int grp, band;
@@ -219,8 +215,8 @@ __global__ void __launch_bounds__(kBlock) k_xinv(Geo g, Fft1D f, const T2 *tw, c
     const int ig = g.stripe_g[e];
     T2 v = r[(g.stripe_s[e] - s0) * xp + g.stripe_x[e]];
     double2 o = make_double2((double)v.x * scale, (double)v.y * scale);
-    if (add_kin) {
-      const double h = add_kin == kAddPlain ? 1.0 : 0.5 * g.g2[ig];
+    if (add) {
+      const double h = ROW ? 1.0 : 0.5 * g.g2[ig];
       const double2 p = ps[ig];
       o.x += h * p.x;
       o.y += h * p.y;
@@ -1190,7 +1186,7 @@ int rtog_t(pw_plan *p, int nb, double2 *fofg, const void *fofr, T2 *stripes, T2 
   const Geo g = make_geo(p);
   PW_TRY(run_pencils<T2>(p, 2, -1, nb, z_pencils(p, fofr, planes, false, real), s));
   PW_TRY(run_pencils<T2>(p, 1, -1, nb, y_pencils(p, planes, stripes, false), s));
-  return run_inverse_x<T2, true>(p, g, nb, fofg, add, 1.0 / (double)p->nrl, add ? kAddPlain : 0, stripes, s);
+  return run_inverse_x<T2, true>(p, g, nb, fofg, add, 1.0 / (double)p->nrl, add ? 1 : 0, stripes, s);
 }
 
 // full-grid transforms in batches of at most c bands through the given

@@ -518,16 +518,18 @@ __device__ inline double wave_sum(double s) {
 }
 
 // ---------------------------------------------------------------------------
-// Row-panel chains: a workgroup carries a panel of 4 or 8 rows through two or
+// Row-panel chains: a workgroup carries a panel of 4, 8 or 16 rows through two or
 // more products, the panel between them in LDS.  v_mfma_f64_4x4x4 (4 rows x 16
 // columns x 4 k, 16 cycles) splits a matrix into two to four times as many
-// workgroups as 16-row panels do at the same rate per cycle; what bounds them is the other
-// operand, n^2 doubles per workgroup from the L2 (3.3 us per product for 144
-// bands, of 1.0 for the matrix instructions).  Staging that operand through
-// LDS, and splitting the k range over the waves, both came out slower.
-//   k_series_terms  (P_k G) P_k, 8 rows: 15.7 -> 10.4 us per iteration for 144
-//                   bands and 8 terms (16-row panels filled 72 of 256 CUs),
-//                   8.0 -> 4.8 for 48, 39 -> 26 for 256, 157 -> 153 for 500
+// workgroups as v_mfma_f64_16x16x4 does at the same rate per cycle; what bounds
+// them is the other operand, n^2 doubles per workgroup from the L2 (3.3 us per
+// product for 144 bands, of 1.0 for the matrix instructions).  Staging that
+// operand through LDS, and splitting the k range over the waves, both came out
+// slower.
+//   k_series_terms  (P_k G) P_k, 8 or 16 rows, against 16 rows with 16x16x4: 15.8
+//                   -> 11.0 us per iteration for 144 bands and 8 terms (16 rows
+//                   filled 72 of 256 CUs), 8.0 -> 4.8 for 48, 39.8 -> 24.8 for
+//                   256, 88.6 -> 73.0 for 400, 157 -> 117 for 500
 //   k_ns_chain      one Newton-Schulz step, X' = 2X - (X (B + qI)) X: 144 bands
 //                   9.1 us against 11.4 for its two products as launches
 //   k_build_chain   P_k = M A^k, k < K, and the acceptance maxima: 144 bands,
@@ -535,12 +537,13 @@ __device__ inline double wave_sum(double s) {
 // ---------------------------------------------------------------------------
 constexpr int kChainThreads = 1024;
 inline int chain_threads(int n) { return 64 * std::min(16, (n + T16 - 1) / T16); }
-// LDS row length of a panel: whole groups of eight k, == 8 or 24 (mod 32)
-// doubles, so that the sixteen (row, k pair) reads of a fragment fall into
-// distinct banks
+// LDS row length of a panel: whole groups of eight k and four doubles more, 8 or
+// 24 (mod 32) banks, so that the 16-byte reads of (k, k + 1) in the four rows of
+// a fragment fall into distinct banks.  With whole rows 8 or 24 (mod 32) doubles
+// long every other LDS cycle was a conflict: passes of 16 rows took 87.7 us instead of
+// 73.0 for 400 bands and 8 terms, of 8 rows 26.9 instead of 24.8 for 256.
 __host__ __device__ inline int chain_ld(int n) {
-  const int l = (n + 7) & ~7;
-  return l % 16 == 0 ? l + 8 : l;
+  return ((n + 7) & ~7) + 4;
 }
 
 // acc[f] += A(4f + i, :) B(:, col), the panel A in LDS (columns n .. zero);
@@ -706,29 +709,31 @@ __global__ void __launch_bounds__(kChainThreads) k_build_chain(int n, int K, dou
   }
 }
 
-// Eight rows of the term P_k G P_k (P_k symmetric: the row-major read is the
+// 4 F rows of the term P_k G P_k (P_k symmetric: the row-major read is the
 // coalesced one).  The terms are the fast index of the grid, so that with
 // eight of them an XCD reads one P_k.  The convergence test of this iteration
 // comes first, as k_series_sum applies it next: when GAMN is converged, NaN or
 // diverging the terms go unused and the loop ends there, so the products are
 // skipped.  Its loads go out with those of the panel; it costs 0.3 us per
-// iteration and saves most of the last one: all passes of a solve of 12
+// iteration and saves most of the last one (8 rows): all passes of a solve of 12
 // iterations 130 -> 127 us for 144 bands and 8 terms, of 14 iterations 355 -> 339
 // for 256; 96 bands 79 -> 77, 48 bands 49 -> 50.  After the first product
 // instead of before it, 256 bands took 351.
+template <int F>
 __global__ void __launch_bounds__(kChainThreads) k_series_terms(SeriesArgs a, int nterm, OrthoState *st) {
   if (stopped(st)) return;
   extern __shared__ double sm[];
   __shared__ int wflag[kChainThreads / 64];
   const int n = a.n, ld = chain_ld(n), row = (threadIdx.x & 63) >> 4;
   const size_t n2 = (size_t)n * n;
-  double *sp = sm, *su = sm + 8 * ld;
-  const int k = blockIdx.x % nterm, I0 = 8 * (blockIdx.x / nterm);
+  constexpr int R = 4 * F;
+  double *sp = sm, *su = sm + R * ld;
+  const int k = blockIdx.x % nterm, I0 = R * (blockIdx.x / nterm);
   const double *Pk = a.P + (size_t)k * n2;
   double *out = a.part + (size_t)k * n2;
   const double x0 = (int)threadIdx.x < a.nbmax ? a.bmax[threadIdx.x] : 0.0;
-  chain_stage<8>(Pk, n, I0, sp, ld);
-  for (int e = threadIdx.x; e < 8 * ld; e += blockDim.x) su[e] = 0.0;
+  chain_stage<R>(Pk, n, I0, sp, ld);
+  for (int e = threadIdx.x; e < R * ld; e += blockDim.x) su[e] = 0.0;
   bool isnan = false, above = false, huge = false;
   auto test = [&](double x) {
     isnan |= x != x;
@@ -745,19 +750,20 @@ __global__ void __launch_bounds__(kChainThreads) k_series_terms(SeriesArgs a, in
   if (__any(flag & 5) || !__any(flag & 2)) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) st->passes++;
   chain_cols(n, [&](int col) {
-    double acc[2] = {0.0, 0.0};
-    chain_mul<2>(sp, ld, a.G, n, col, acc, ChainId{});
+    double acc[F] = {};
+    chain_mul<F>(sp, ld, a.G, n, col, acc, ChainId{});
     if (col >= n) return;
-    su[row * ld + col] = acc[0];
-    su[(4 + row) * ld + col] = acc[1];
+#pragma unroll
+    for (int f = 0; f < F; ++f) su[(4 * f + row) * ld + col] = acc[f];
   });
   __syncthreads();
   chain_cols(n, [&](int col) {
-    double acc[2] = {0.0, 0.0};
-    chain_mul<2>(su, ld, Pk, n, col, acc, ChainId{});
+    double acc[F] = {};
+    chain_mul<F>(su, ld, Pk, n, col, acc, ChainId{});
     if (col >= n) return;
-    if (I0 + row < n) out[(size_t)(I0 + row) * n + col] = acc[0];
-    if (I0 + 4 + row < n) out[(size_t)(I0 + 4 + row) * n + col] = acc[1];
+#pragma unroll
+    for (int f = 0; f < F; ++f)
+      if (I0 + 4 * f + row < n) out[(size_t)(I0 + 4 * f + row) * n + col] = acc[f];
   });
 }
 
@@ -1420,8 +1426,9 @@ int ortho_work(pw_waveset *ws, OrthoWork &w) {
   static std::once_flag lds_once;
   static hipError_t lds_err = hipSuccess;
   std::call_once(lds_once, [] {
-    const void *fns[] = {(const void *)k_panel_batch, (const void *)k_series_terms, (const void *)k_ns_chain,
-                         (const void *)k_build_chain, (const void *)k_ortho_small<1>, (const void *)k_ortho_small<2>};
+    const void *fns[] = {(const void *)k_panel_batch, (const void *)k_series_terms<2>, (const void *)k_series_terms<4>,
+                         (const void *)k_ns_chain, (const void *)k_build_chain, (const void *)k_ortho_small<1>,
+                         (const void *)k_ortho_small<2>};
     for (const void *f : fns) {
       hipFuncAttributes fa{};
       hipError_t e = hipFuncGetAttributes(&fa, f);
@@ -1471,8 +1478,17 @@ int panel_batch(pw_waveset *ws, const BatchArgs &a) {
 
 // LDS of two panels of `rows` rows
 inline size_t chain_lds(int n, int rows) { return (size_t)2 * rows * chain_ld(n) * sizeof(double); }
+// rows of a workgroup of the terms: 8 while that gives each CU one workgroup at
+// most, 16 beyond, which read the other operand half as often (same sums).  8
+// terms: 256 bands (256 workgroups of 8 rows) 24.8 us against 31.4, 272 bands
+// (272) 49.4 against 39.2, 400 97.6 against 73.0, 600 301 against 262; 16 terms: 96
+// bands 11.3 against 11.6, 128 17.3 against 16.9, 144 30.1 against 30.9, 192 40.8
+// against 38.4, 256 88.3 against 64.5, 416 379 against 295.
+inline int series_rows(int n, int nterm) { return (n + 7) / 8 * nterm > 256 ? 16 : 8; }
 void series_terms(pw_waveset *ws, const SeriesArgs &a, int nterm, OrthoState *st) {
-  k_series_terms<<<(a.n + 7) / 8 * nterm, chain_threads(a.n), chain_lds(a.n, 8), ws->stream>>>(a, nterm, st);
+  const int f = series_rows(a.n, nterm) / 4, grid = (a.n + 4 * f - 1) / (4 * f) * nterm;
+  auto *const terms = f == 4 ? k_series_terms<4> : k_series_terms<2>;
+  terms<<<grid, chain_threads(a.n), chain_lds(a.n, 4 * f), ws->stream>>>(a, nterm, st);
 }
 
 template <int MODE>
@@ -1513,10 +1529,11 @@ struct OrthoParams {
   int nns;    // Newton-Schulz steps
 };
 
-// A Newton-Schulz step as one chain of two products instead of two launches:
-// the chain costs 3.3 us per product and 2.5 in all for 144 bands, where the
-// launches take 5.0 each and a gap; its time grows with n^2 on a quarter of the
-// CUs, 18.7 us against 13.6 for 256 bands.
+// A Newton-Schulz step as one chain of two products instead of two launches: its
+// time grows with n^2 on a quarter of the CUs.  The kernels' times cross just
+// above 160 bands: the chain takes 8.2 us for 128, 8.6 for 144, 10.0 for 160,
+// 11.7 for 176, 12.2 for 192, 14.3 for 208 and 18.4 for 256, the two launches
+// 9.7, 10.0, 10.2, 11.1, 10.9, 12.0 and 12.9 and one more gap.
 constexpr int kNsChainMaxN = 160;
 // The series matrices one after the other, K - 1 products in one launch,
 // instead of doubled in J launches: 32 us against 41 for 144 bands, 71 against

@@ -59,3 +59,20 @@ def test_no_terms_where_the_loop_ends(nb):
         f()
     assert w.geti4("ORTHOITER") > 1 and w.geti4("ORTHOEIGEN") == 0
     assert w.geti4("ORTHOPASSES") == w.geti4("ORTHOITER") - 1
+
+
+@pytest.mark.parametrize("nb,spread", [(125, 6.0), (128, 6.0), (129, 6.0), (264, 1.1), (265, 1.1), (416, 1.1),
+                                       (609, 1.1)])
+def test_ortho_x_sixteen_rows(nb, spread):
+    """Terms of the series by panels of 16 rows, from more than one panel of 8
+    rows per CU on: whole panels, remainders of 1, 8, 9 and 13 rows, and the widest
+    set with terms (its two panels fill a CU's LDS)."""
+    import pwgpu
+    from oracle import waves as owv
+    print(f"case 16-row panels nb={nb}", flush=True)
+    occ, chichi, psipsi, chipsi = solve_case(nb, spread)
+    lam0 = 0.001 * np.random.default_rng(nb).normal(size=(nb, nb))
+    ref, it_ref = owv.ortho_x(occ, chichi, psipsi, chipsi, lam0.copy())
+    lam, it = pwgpu.ortho_x(occ, chichi, psipsi, chipsi, lam0)
+    assert it == it_ref
+    assert relerr(lam, ref) < 1e-10

@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(kBlock) k_pencil_any(PencilArgs a, Fft1D f, co
   for (int w = threadIdx.x; w < f.n * kTX; w += blockDim.x) b0[w] = io.load(w / kTX, q0 + w % kTX);
   __syncthreads();
   const T2 *r = lds_fft<T2>(b0, b1, f, kTX, kTX, 1, tw, SIGN, true);
-  for (int w = threadIdx.x; w < f.n * kTX; w += blockDim.x) io.store(w / kTX, q0 + w % kTX, r[w]);
+  for (int w = threadIdx.x; w < f.n * kTX; w += blockDim.x) io.store(io.out_row(w / kTX), q0 + w % kTX, r[w]);
 }
 
 // ---- in-place LDS transforms for the resident yz plane -----------------------

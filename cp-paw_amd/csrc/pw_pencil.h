@@ -53,10 +53,12 @@ template <typename T2> struct PencilIo {
     z.y = ok ? v.y : 0;
     return z;
   }
+  // row of element e in dst, negative: not written.  Read before the first
+  // store of a butterfly: a load behind a store waits for its own round trip
+  __device__ int out_row(int e) const { return forward ? e : map[e]; }
   // streaming stores: a pass writes each element once and more than L2 holds
-  __device__ void store(int e, int q, T2 v) const {
+  __device__ void store(int m, int q, T2 v) const {
     typedef decltype(v.x) V2 __attribute__((ext_vector_type(2)));
-    const int m = forward ? e : map[e];
     if (m < 0 || q >= npen) return;
     const unsigned i = (unsigned)m * ds + (unsigned)q;
     if (real && forward) {

@@ -31,3 +31,32 @@ def test_full_grid_lengths(n2, n3):
     for prec, tol in ((0, 1e-12), (1, 2e-5)):
         assert relerr(plane.fft_host("GTOR", fofg=fofg, prec=prec), pl.fft_gtor(fofg)) < tol
         assert relerr(plane.fft_host("RTOG", fofr=fofr, prec=prec), pl.fft_rtog(fofr)) < tol
+
+
+@pytest.mark.parametrize("n", [12, 14, 16, 18, 20, 22, 24, 28, 32, 36, 40, 44, 48, 56, 64, 72, 80, 88, 112, 128, 144])
+def test_full_grid_tiles(n):
+    """Lengths of one or two stages in wide tiles (a batch that fills the chip)
+    and in narrow ones (one band at a time): the same operations on each pencil,
+    so the same bits; the batch against the oracle as above.  n is the length
+    of the z pass, over 256 pencils, and of the y pass, over 64."""
+    import pwgpu
+    nb = 200 if n <= 40 else 100
+    for nr in ((16, 16, n), (64, n, 12)):
+        print(f"case full-grid tiles {nr}", flush=True)
+        rbas = np.diag([2.0 * math.pi * (k / 2 - 0.5) for k in nr])
+        plane = pwgpu.PlaneWave(rbas, 0.5, 0.5)
+        pl = opw.Plane(rbas, 0.5, 0.5)
+        assert plane.nr == nr
+        rng = np.random.default_rng(n)
+        fofg = rng.normal(size=(nb, pl.ngl)) + 1j * rng.normal(size=(nb, pl.ngl))
+        fofr = rng.normal(size=(nb, *nr[::-1])) + 1j * rng.normal(size=(nb, *nr[::-1]))
+        for prec, tol in ((0, 1e-12), (1, 2e-5)):
+            r = plane.fft_host("GTOR", fofg=fofg, prec=prec)
+            g = plane.fft_host("RTOG", fofr=fofr, prec=prec)
+            for b in (0, nb - 1):
+                one = slice(b, b + 1)
+                assert np.array_equal(r[one], plane.fft_host("GTOR", fofg=fofg[one], prec=prec)), (nr, prec)
+                assert np.array_equal(g[one], plane.fft_host("RTOG", fofr=fofr[one], prec=prec)), (nr, prec)
+                assert relerr(r[one], pl.fft_gtor(fofg[one])) < tol
+                assert relerr(g[one], pl.fft_rtog(fofr[one])) < tol
+        plane.close()

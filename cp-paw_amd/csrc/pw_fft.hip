@@ -117,21 +117,27 @@ template <typename T2> struct XTile;
 template <> struct XTile<double2> { static constexpr int n = 16; };
 template <> struct XTile<float2> { static constexpr int n = 32; };
 
-// Workgroup -> (stripe group, band) of the x passes, a 1D grid of nb ngroups
-// workgroups: consecutive workgroups go to the eight XCDs in turn.  In whole
-// octets of bands each XCD takes every stripe group of its bands (band = xcd +
-// 8 k), so the coefficients of a band, gathered and scattered in G order by
-// all its stripe groups, pass through one XCD's L2 instead of eight.  The
-// groups of the last nb mod 8 bands are dealt to all XCDs: with one band
-// (VOFRHO's transforms) they had all run on one XCD, 21 and 17 us for the
-// passes of the Si64 density sphere against 9 and 8.
-__device__ inline void x_block(int ngroups, int nb, int &group, int &band) {
-  const unsigned id = blockIdx.x, whole = (unsigned)nb & ~7u, n8 = whole * ngroups;
+// Workgroup -> (stripe group, band) of the x passes, a 1D grid: consecutive
+// workgroups go to the eight XCDs in turn.  In octets of bands each XCD takes
+// every stripe group of its bands (band = xcd + 8 k), so the coefficients of a
+// band, gathered and scattered in G order by all its stripe groups, pass through
+// one XCD's L2 instead of eight.  The groups of up to four bands beyond the whole
+// octets are dealt to all XCDs: with one band (VOFRHO's transforms) they had all
+// run on one XCD, 21 and 17 us for the passes of the Si64 density sphere against
+// 9 and 8; both passes of 52 bands of 64^3 in FP32 26.6 -> 22.4 us.  Five to seven
+// bands keep an XCD each: dealt to all, 62 bands took 31.3 us instead of 29.8, 30
+// bands 20.4 instead of 19.4; four are between (28 bands 18.4 us with an XCD each,
+// 19.5 dealt to all, 60 bands 29.7 and 30.8, 52 as above).  False where the octet
+// has no such band.
+__host__ __device__ inline unsigned x_octets(int nb) { return (unsigned)((nb & 7) > 4 ? nb + 7 : nb) & ~7u; }
+__device__ inline bool x_block(int ngroups, int nb, int &group, int &band) {
+  const unsigned id = blockIdx.x, oct = x_octets(nb), n8 = oct * ngroups;
   const unsigned j = id < n8 ? id / 8 : id - n8, q = j / (unsigned)ngroups;
-  band = (int)(id < n8 ? id % 8 + 8 * q : whole + q);
+  band = (int)(id < n8 ? id % 8 + 8 * q : oct + q);
   group = (int)(j - q * ngroups);
+  return band < nb;
 }
-inline dim3 x_grid(int ngroups, int nb) { return dim3((unsigned)(nb * ngroups)); }
+inline dim3 x_grid(int ngroups, int nb) { return dim3(std::max(x_octets(nb), (unsigned)nb) * ngroups); }
 // LDS pitch of the x passes' stripe tiles: odd, so that the tile's transposes
 // (neighbouring lanes on neighbouring stripes, one pitch apart) fall into
 // distinct banks
@@ -146,7 +152,7 @@ __global__ void __launch_bounds__(kBlock) k_xfwd(Geo g, Fft1D f, const T2 *tw, c
   constexpr int PX = XTile<T2>::n;
   if constexpr (NX > 0) g.nr1 = NX;
   int grp, band;
-  x_block((g.nstripe + PX - 1) / PX, nb, grp, band);
+  if (!x_block((g.nstripe + PX - 1) / PX, nb, grp, band)) return;
   extern __shared__ unsigned char smem_raw[];
   const int xp = x_pitch(g.nr1);
   T2 *b0 = reinterpret_cast<T2 *>(smem_raw);
@@ -186,7 +192,7 @@ __global__ void __launch_bounds__(kBlock) k_xinv(Geo g, Fft1D f, const T2 *tw, c
   constexpr int PX = XTile<T2>::n;
   if constexpr (NX > 0) g.nr1 = NX;
   int grp, band;
-  x_block((g.nstripe + PX - 1) / PX, nb, grp, band);
+  if (!x_block((g.nstripe + PX - 1) / PX, nb, grp, band)) return;
   extern __shared__ unsigned char smem_raw[];
   const int xp = x_pitch(g.nr1);
   T2 *b0 = reinterpret_cast<T2 *>(smem_raw);

@@ -60,3 +60,21 @@ def test_full_grid_tiles(n):
                 assert relerr(r[one], pl.fft_gtor(fofg[one])) < tol
                 assert relerr(g[one], pl.fft_rtog(fofr[one])) < tol
         plane.close()
+
+
+@pytest.mark.parametrize("nb", [1, 4, 5, 7, 8, 12, 13, 15, 16, 21])
+def test_x_pass_bands(nb):
+    """x passes with whole octets of bands and with one to seven beyond them
+    (a band per XCD, or its stripe groups on all of them)."""
+    import pwgpu
+    from pwgpu import model
+    print(f"case x passes of {nb} bands", flush=True)
+    s = model.tiny()
+    plane = pwgpu.PlaneWave(s.rbas, s.epw_psi, s.epw_rho)
+    pl = opw.Plane(s.rbas, s.epw_psi, s.epw_rho)
+    rng = np.random.default_rng(nb)
+    fofg = rng.normal(size=(nb, pl.ngl)) + 1j * rng.normal(size=(nb, pl.ngl))
+    fofr = rng.normal(size=(nb, pl.nr3, pl.nr2, pl.nr1)) + 1j * rng.normal(size=(nb, pl.nr3, pl.nr2, pl.nr1))
+    for prec, tol in ((0, 1e-12), (1, 2e-5)):
+        assert relerr(plane.fft_host("GTOR", fofg=fofg, prec=prec), pl.fft_gtor(fofg)) < tol
+        assert relerr(plane.fft_host("RTOG", fofr=fofr, prec=prec), pl.fft_rtog(fofr)) < tol

@@ -297,7 +297,7 @@ struct pw_waveset {
   // mixed form: factors of the projector functions for the positions
   // pfac_pos, P(atom,lmn,G) = (-i)^l F(isp,lmn,G) E(atom,G):
   // F = YLM*PRO [NSP*LMNXX][NGLP] doubles, then E = exp(-iG.R) [NAT][NGLP]
-  // double2, NGLP = NGL padded to 64 with zeros
+  // double2, NGLP = NGL padded to 64 with zeros, then E and F rounded to FP32
   void *d_pfac = nullptr;
   size_t pfac_bytes = 0;
   std::vector<double> pfac_pos;

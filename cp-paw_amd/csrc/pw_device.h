@@ -93,7 +93,7 @@ __device__ inline dbl4 mfma4(double a, double b, dbl4 c) {
 
 // sum of split partials: out[i] = scale * sum_s part[s][i] in a fixed order.
 // A block takes 32 outputs; its 8 lanes per output stride over the splits
-// with four accumulators each and are combined through LDS.
+// and are combined through LDS.
 constexpr int kRedC = 32, kRedS = 8;
 
 __device__ inline double rz(double) { return 0.0; }

@@ -377,9 +377,11 @@ __host__ __device__ constexpr int fft_lprod(const Fft1D &f, int st) {
   return L;
 }
 
-// threads of the yz passes: kYZ, twice as many where one FP64 plane fills a
-// CU's LDS (104 KiB for 80 x 80) and its workgroup is all that hides the latency
-// of the stages; 512 threads also take two rounds of butterflies per stage of 72
+// threads of the yz passes of a compile-time plane: kYZ, twice as many where one
+// FP64 plane fills a CU's LDS (104 KiB for 80 x 80) and its workgroup is all that
+// hides the latency of the stages; 72 x 72 and 80 x 80 of the planes instantiated
+// here (the run-time stages are written for kYZ and have not been measured with
+// more).  512 threads take two rounds of butterflies per stage of 72
 // x 72, 57 % full, 1024 one: 72 x 72 planes of 72 super bands 188 -> 178 us
 // (density 98 -> 94), 80 x 80 of 128 307 -> 279; 704 threads (one full round)
 // 183, 281 and 101.  Where two planes share a CU (64 x 64, one full round of

@@ -14,12 +14,13 @@
 // FP64 MFMA bound: 3.5 GFLOP per projector product at Si64 (512 projectors,
 // 144 bands, 23 847 G) is 48 us at the rate of a large FP64 product.  Measured
 // there against the complex products over the whole sphere: projections 287
-// -> 79 us, ADDPRO 328 -> 101, forces 272 -> 87, the three band overlaps of a
-// step 327 -> 82, ADDOPSI 101 -> 37.  The rest is the staging between the MFMAs:
-// the matrix units are busy 50 to 62 % of the time and vector instructions take
-// 13 to 20 %, which do not overlap.  With selects on every load, 64-bit products
-// in the addresses and (-i)^l by a switch the same kernels took 88, 107, 96, 89
-// and 39 us.
+// -> 77 us, ADDPRO 328 -> 99, forces 272 -> 85, the three band overlaps of a
+// step 327 -> 85, ADDOPSI 101 -> 36.  The rest is the staging between the MFMAs:
+// counted there, the matrix units are busy 63 % of the time in the projections,
+// 56 in the overlaps, 58 in the forces, 51 in ADDPRO and 43 in ADDOPSI, and vector
+// instructions take 11 to 20 %.  With selects on every load, 64-bit products in
+// the addresses and (-i)^l by a switch the same kernels took 88, 107, 96, 89 and
+// 39 us, with matrix units busy 42 to 58 % and vector instructions 14 to 24.
 #include <algorithm>
 
 #include "pw_device.h"
@@ -73,8 +74,7 @@ __global__ void k_half_e(ProjGeo q, int nh, int nhp, const int2 *__restrict__ hg
 // psi of one super band at (G, -G).  The loads are unconditional (clamped
 // indices): what is out of range meets a zero of the other operand or enters
 // elements that are not written.  On these kernels every vector instruction
-// counts: the FP64 matrix instructions keep the SIMD unit from issuing others,
-// and matrix and vector time added up to 72 % in all of them.
+// counts: what the staging lost of them the kernels lost in time (figures above).
 struct Pair {
   double2 p, m;
 };

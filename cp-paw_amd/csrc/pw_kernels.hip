@@ -200,7 +200,8 @@ __global__ void __launch_bounds__(64 * NW) k_colgemm(GA ga, GB gb, int nk, int n
 // ---------------------------------------------------------------------------
 // forces: F(atom) = 2 Omega sum_G G Re[i P conj(D)], D = psi conj(dE/dproj)
 // (WAVES_DEDPRO + WAVES_PROFORCE fused; the INVERTG symmetrisation of DEDPRO
-//  leaves this sum unchanged because P(-G) = conj(P(G))).
+//  leaves this sum unchanged where P(-G) = conj(P(G)); this kernel takes the
+//  PRO tables without that symmetry, and their forces are the plain sum).
 // D(ipro,G) = sum_b conj(ded[ipro][b]) psi[b][G] on MFMA (NW waves x 16 ipro
 // rows, NGB 16-G blocks); the epilogue contracts D with P and G and sums the
 // workgroup's G range: part[gtile][ipro][3].

@@ -158,7 +158,8 @@ int pw_waves_getr8(pw_waveset *ws, const char *id, double *val);
  * accepted), "ORTHOEIGEN" (solves so far through the eigenvectors of
  * sym(CHIPSI), taken when it is not positive definite), "ORTHOGRAPHMISSES"
  * (solves issued without a captured hipGraph: captures are made only while
- * one plan and one waveset exist in the process), "NLAMBDA" (multiplier history held: 0 none, 1 RLAM0, 2 RLAM0
+ * one plan and one waveset exist in the process; a small set's solve is one
+ * launch, needs none and is not counted), "NLAMBDA" (multiplier history held: 0 none, 1 RLAM0, 2 RLAM0
  * and RLAMM; counted as in WAVES_WRITELAMBDA, src/paw_waves2.f90:3948),
  * and the launch shapes of pw_waves_autotune: "SPLITWAVES" (waves of a
  * G-split row-product launch), "DENSBLOCKS" (workgroups of the density pass),
